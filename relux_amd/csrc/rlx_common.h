@@ -647,6 +647,20 @@ hipError_t launch_proj(hipStream_t s, int model, const PlanArg *plan, const Patc
                        const ProjDims &pd, const float *rcos, const float *rsin, void *q_out,
                        void *q_out2, int q_bf16, uint16_t *kpool, uint16_t *vpool, int32_t *table,
                        int P, int cus, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
+// The same over any number of rows in one launch (the MFMA GEMM of prefill
+// sizes); plans on the device only.  Taken past kProjRows rows, and past 32
+// when launch_proj's 16-feature work-groups are more than one round of the
+// CUs (us at K 4096, chunked kernel against GEMM: N 6144, 33 rows 23.8 / 22,
+// 64 rows 36.6 / 22; N 4096, 64 rows 21.0 / 20.8, 33 rows 14.3 / 21).
+inline bool proj_use_gemm(int rows, int model, const ProjDims &pd, int cus) {
+    return rows > kProjRows || (rows > 32 && proj_features(model, pd) > 16 * cus);
+}
+hipError_t launch_proj_gemm(hipStream_t s, int model, const Patch *patches, int n_patch,
+                            const AppendTok *toks, const int32_t *pos, int rows, const void *x,
+                            int x_bf16, int K, const uint16_t *wp, const ProjDims &pd,
+                            const float *rcos, const float *rsin, void *q_out, void *q_out2,
+                            int q_bf16, uint16_t *kpool, uint16_t *vpool, int32_t *table, int P,
+                            int cus, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 
 // Work-groups of the decode kernels one CU holds at once (occupancy).
 int mla_decode_wgs_per_cu(int nqt);

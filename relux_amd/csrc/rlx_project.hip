@@ -16,7 +16,8 @@
 // mla.go:384-389; the transformer block's residual add): out = x.W (+ the
 // residual), no RoPE, no append.
 //
-// Two kernels: at decode sizes (at most 32 rows) proj_skinny_kernel streams
+// Prefill sizes (proj_use_gemm) take rlx_project_gemm.hip.  Here two
+// kernels: at decode sizes (at most 32 rows) proj_skinny_kernel streams
 // the weights with every load in flight at once (below); otherwise
 // qkv_project_kernel: work-group = 16 output features x all rows (at most
 // 64); its 4 waves take contiguous ranges of the 32-wide k-steps
@@ -29,7 +30,7 @@
 // from HBM, so the second product costs no time.  The result lane holds 4
 // rows of one feature, so a RoPE pair partner (feature ^ 1) is one lane
 // away.
-#include "rlx_common.h"
+#include "rlx_project.h"
 
 namespace rlx {
 
@@ -71,20 +72,6 @@ __global__ void pack_proj_kernel(PackSrc src, int w_bf16, int K, int KP, int N, 
 constexpr int kProjWaves = 4;   // k split over the waves of a work-group
 constexpr int kProjChunk = 8;   // k-steps of W held in registers at once per wave
 
-// Output layouts (features in packed order, each part a multiple of 16):
-//   kProjGQA: q (H heads x D, RoPE)    -> q_out [rows][H][D]
-//             k (KVH x D, RoPE)        -> K pages (k-step-major)
-//             v (KVH x D)              -> dim-major V pages
-//   kProjMLA: q_c (H x D)              -> q_out  [rows][H][D]
-//             q_r (H x d_r, RoPE)      -> q_out2 [rows][H][d_r]
-//             c^KV (d_c)               -> latent rows [0, d_c)
-//             k^R (d_r, RoPE)          -> latent rows [d_c, d_c + d_r)
-//   kProjOut:  out (N = features)      -> q_out [rows][N] (+ q_out2, the
-//                                         residual, in the same dtype)
-constexpr int kProjGQA = 0;
-constexpr int kProjMLA = 1;
-constexpr int kProjOut = 2;
-
 // Output placement of one lane: feature n (lane col = n % 16) of the 4 rows
 // m*16 + grp*4 + i of lane group grp.  proj_place_plan and proj_place_rope
 // read what the plan and the RoPE tables hold for them (positions, append
@@ -100,28 +87,6 @@ struct ProjPlace {
     float c[4], s[4];      // RoPE (cos, sin) of each row
     int page[4], slot[4];  // append slot of each row (k / v / latent parts)
 };
-
-// Part of packed feature n: output part, feature within it, features per
-// RoPE head and rotated dims per head (0, 0: no RoPE).
-template <int MODEL>
-__device__ __forceinline__ void proj_part(const ProjDims &pd, int n, int &part, int &nn, int &hw, int &tw) {
-    part = 0;
-    nn = n;
-    hw = tw = 0;
-    if constexpr (MODEL == kProjGQA) {
-        const int NQ = pd.H * pd.DW, NK = pd.KVH * pd.DW;
-        part = n < NQ ? 0 : (n < NQ + NK ? 1 : 2);
-        nn = n - (part == 0 ? 0 : (part == 1 ? NQ : NQ + NK));
-        hw = part < 2 ? pd.DW : 0;  // (features past D: zero weights, no rotation)
-        tw = part < 2 ? pd.D : 0;
-    } else if constexpr (MODEL == kProjMLA) {
-        const int NQC = pd.H * pd.DW, NQR = pd.H * pd.DRP;
-        part = n < NQC ? 0 : (n < NQC + NQR ? 1 : (n < NQC + NQR + pd.DCP ? 2 : 3));
-        nn = n - (part == 0 ? 0 : (part == 1 ? NQC : (part == 2 ? NQC + NQR : NQC + NQR + pd.DCP)));
-        hw = (part == 1 || part == 3) ? pd.DRP : 0;
-        tw = hw ? pd.DR : 0;
-    }
-}
 
 // Plan reads of the placement (no load depends on another): part, RoPE
 // positions (pos < 0: no rotation), append slots.
@@ -309,16 +274,6 @@ __device__ __forceinline__ void proj_store(const ProjPlace &o, fl4 y, int m, int
             }
         }
     }
-}
-
-// Activations as MFMA A operands: bf16 pairs {hi, lo} of two f32 values
-// (lo = bf16(x - hi), zero where hi is not finite).
-__device__ __forceinline__ u32x2 proj_split2(float a, float b) {
-    const uint16_t ha = bf16_rne(a), hb = bf16_rne(b);
-    const float ra = bf16_f32(ha), rb = bf16_f32(hb);
-    const uint16_t la = (fabsf(ra) < INFINITY) ? bf16_rne(a - ra) : (uint16_t)0;
-    const uint16_t lb = (fabsf(rb) < INFINITY) ? bf16_rne(b - rb) : (uint16_t)0;
-    return u32x2{(uint32_t)ha | ((uint32_t)hb << 16), (uint32_t)la | ((uint32_t)lb << 16)};
 }
 
 template <bool ARG, bool XBF16, int MODEL>

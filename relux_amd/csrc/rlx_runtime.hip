@@ -186,6 +186,17 @@ int32_t stage(Cache *c, const void *data, size_t bytes, void **dev_out) {
     return RLX_OK;
 }
 
+// Whether the cache's stream is recording a graph (or may not be asked: the
+// null stream while another one records).
+bool capturing(Cache *c) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(c->stream, &st) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return st != hipStreamCaptureStatusNone;
+}
+
 // Append plans: patches then tokens (16-byte aligned), in the kernel
 // arguments when they fit, else staged.  Fills *plan or the device pointers.
 int32_t append_plan(Cache *c, const std::vector<Patch> &patches,
@@ -1132,13 +1143,22 @@ int32_t rlx_out_project(void *h, int32_t rows, const void *x, int32_t x_dtype, i
         x = pad[0];
         k_in = kp;
     }
+    ProjDims pd{};
+    pd.D = n_out;
+    pd.DW = (n_out + 15) / 16 * 16;
+    if (proj_use_gemm(rows, kProjModelOut, pd, c->cus)) {  // prefill sizes: one GEMM over all rows
+        hipEvent_t e0, e1;
+        if ((rc = timing_events(c, &e0, &e1, RLX_TIME_PROJECT))) return rc;
+        HIP_TRY(launch_proj_gemm(c->stream, kProjModelOut, nullptr, 0, nullptr, nullptr, rows, x,
+                                 x_dtype == RLX_BF16, k_in, (const uint16_t *)w_packed, pd, nullptr, nullptr,
+                                 out, (void *)residual, out_dtype == RLX_BF16, nullptr, nullptr, nullptr, 0,
+                                 c->cus, e0, e1));
+        return RLX_OK;
+    }
     for (int r0 = 0; r0 < rows; r0 += kProjRows) {
         const int n = std::min(kProjRows, rows - r0);
         hipEvent_t e0, e1;
         if ((rc = timing_events(c, &e0, &e1, RLX_TIME_PROJECT))) return rc;
-        ProjDims pd{};
-        pd.D = n_out;
-        pd.DW = (n_out + 15) / 16 * 16;
         HIP_TRY(launch_proj(c->stream, kProjModelOut, nullptr, nullptr, 0, nullptr, nullptr, 0, 0, n,
                             (const char *)x + (size_t)r0 * k_in * xb, x_dtype == RLX_BF16, k_in,
                             (const uint16_t *)w_packed, pd, nullptr, nullptr,
@@ -1221,6 +1241,26 @@ int32_t project_append(Cache *c, int model, int32_t layer, int32_t n_seqs, const
     if ((rc = plan_append(c, layer, n_seqs, seq_ids, n_tok, toks))) return rc;
     std::vector<Patch> patches = take_pending(c);
     const int xb = x_dtype == RLX_BF16 ? 2 : 4, qb = q_dtype == RLX_BF16 ? 2 : 4;
+    if (proj_use_gemm(total, model, pd, c->cus) && !capturing(c)) {
+        // Prefill sizes: one GEMM over all rows, its plan staged.  A stream
+        // under capture keeps the launches below, whose plans travel in the
+        // kernel arguments; so does a call whose plan cannot be staged.
+        Blob b;
+        const size_t o_p = b.add(patches), o_t = b.add(toks), o_pos = b.add(pos);
+        void *dev;
+        if (stage(c, b.bytes.data(), b.bytes.size(), &dev) == RLX_OK) {
+            const AppendTok *d_t = (const AppendTok *)((char *)dev + o_t);
+            HIP_TRY(launch_proj_pad_zero(c->stream, model, nullptr, d_t, 0, total, pd, ls.pool0, ls.pool1, c->P));
+            hipEvent_t e0, e1;
+            if ((rc = timing_events(c, &e0, &e1, RLX_TIME_PROJECT))) return rc;
+            HIP_TRY(launch_proj_gemm(c->stream, model, (const Patch *)((char *)dev + o_p), (int)patches.size(),
+                                     d_t, (const int32_t *)((char *)dev + o_pos), total, x,
+                                     x_dtype == RLX_BF16, d_model, (const uint16_t *)w_packed, pd, rope_cos,
+                                     rope_sin, q_out, model == kProjModelMLA ? q_out2 : nullptr,
+                                     q_dtype == RLX_BF16, ls.pool0, ls.pool1, c->d_table, c->P, c->cus, e0, e1));
+            return RLX_OK;
+        }
+    }
     for (int r0 = 0; r0 < total; r0 += kProjRows) {
         const int rows = std::min(kProjRows, total - r0);
         const std::vector<Patch> none;
