@@ -472,9 +472,10 @@ int32_t rlx_sample(void *cache, const float *logits, int32_t n_rows, int32_t voc
  * (the rng.Float32() draws) are device f32 [n_rows]; out_tokens device
  * int32 [n_rows].  Enqueued on the cache's stream: nothing is copied to or
  * from the host and the call does not wait -- except the first call that
- * needs a larger cache workspace (the split path's chunk lists, top-k in
- * (0, 256] past 8192 entries), which synchronises the stream and
- * allocates it once.  Same tokens as rlx_sample given the same windows
+ * needs a larger cache workspace (the split paths' chunk lists, top-k in
+ * (0, 256] past 8192 entries, or no top-k past 12288: at most 64 MiB),
+ * which synchronises the stream and allocates it once (without top-k a call
+ * that cannot -- its stream under capture, no memory -- runs unsplit).  Same tokens as rlx_sample given the same windows
  * and draws. */
 int32_t rlx_sample_async(void *cache, const float *logits, int32_t n_rows, int32_t vocab,
                          int64_t row_stride, const rlx_sampler_t *params, const int32_t *history,

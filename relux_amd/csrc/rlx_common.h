@@ -351,6 +351,28 @@ struct SampleArgs {
     int nch, pch, pcap;
     float *part_v;
     int32_t *part_i, *part_n;
+    // mass split (uch > 0, set by plan_sample_split; top-k off): row b's
+    // chunk c, q = b * uch + c, covers entries [c * upch, min(V, (c + 1) *
+    // upch)) and leaves its fastexp32 weights at mass_p[q * upch ..], the
+    // exact mass of each weight bucket at mass_h[q * kMassBuckets ..], the
+    // mass certain to be kept of each 256 entries at mass_s[q * useg ..], the
+    // entries still to be decided at mass_l[q * kMassList ..] and its record;
+    // urows rows at a time (the scratch's size)
+    int uch, upch, useg, urows;
+    float *mass_p, *mass_s;
+    uint32_t *mass_h;
+    uint2 *mass_l;
+    struct MassRec *mass_r;
+};
+constexpr int kMassBuckets = 1024;
+constexpr int kMassList = 1024;
+struct MassRec {
+    double total;  // mass of the chunk's weights in the buckets
+    double above;  // mass of the row's weights in heavier buckets than `bucket`
+    float max;     // largest scratch value
+    float rest;    // mass of the weights below the buckets
+    int n_list;    // entries to be decided
+    int bucket;    // top-p: the row's cutoff bucket (-1: below the buckets)
 };
 
 struct SpecArgs {

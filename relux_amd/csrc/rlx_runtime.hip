@@ -2722,6 +2722,22 @@ int32_t rlx_free_list(void *h, int32_t layer, int32_t *out, int32_t cap, int32_t
 
 // ---- token selection ------------------------------------------------------
 
+// Workspace of a Sample call, its split planned at byte `head` (behind what
+// the call keeps there itself).  The mass split is an optional one: a
+// workspace that cannot grow (a cap, or a stream under capture) leaves the
+// call on the whole-row path, which needs none.
+static int32_t sample_scratch(Cache *c, SampleArgs &a, int n_rows, size_t head) {
+    const size_t need = head + (size_t)plan_sample_split(a, n_rows, nullptr);
+    int32_t rc = RLX_OK;
+    if (a.uch > 0 && need > c->ws_cap && (capturing(c) || ensure_ws(c, need) != RLX_OK)) {
+        a.uch = 0;
+        return ensure_ws(c, head);
+    }
+    if ((rc = ensure_ws(c, need))) return rc;
+    plan_sample_split(a, n_rows, (char *)c->ws + head);
+    return RLX_OK;
+}
+
 int32_t rlx_greedy(void *h, const float *logits, int32_t n_rows, int32_t vocab, int64_t row_stride,
                    int32_t *out_tokens) {
     if (!h) return fail(RLX_ERR_INVALID, "null cache");
@@ -2796,10 +2812,10 @@ int32_t rlx_sample(void *h, const float *logits, int32_t n_rows, int32_t vocab, 
     SampleArgs a{};
     a.V = vocab;
     a.top_k = p->top_k;
+    a.top_p = p->top_p;
     const size_t o_split = ((size_t)n_rows * 4 + 255) & ~(size_t)255;
-    int32_t rc = ensure_ws(c, o_split + (size_t)plan_sample_split(a, n_rows, nullptr));
+    int32_t rc = sample_scratch(c, a, n_rows, o_split);
     if (rc) return rc;
-    plan_sample_split(a, n_rows, (char *)c->ws + o_split);
     if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
     char *d = (char *)dev;
     a.logits = logits;
@@ -2870,9 +2886,8 @@ int32_t rlx_sample_async(void *h, const float *logits, int32_t n_rows, int32_t v
     a.window = p->repeat_window;
     a.u = uniforms;
     a.out = out_tokens;
-    int32_t rc = ensure_ws(c, (size_t)plan_sample_split(a, n_rows, nullptr));
+    int32_t rc = sample_scratch(c, a, n_rows, 0);
     if (rc) return rc;
-    plan_sample_split(a, n_rows, (char *)c->ws);
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1, RLX_TIME_SELECT))) return rc;
     HIP_TRY(launch_sample(c->stream, a, n_rows, e0, e1));

@@ -3,9 +3,12 @@
 // work-groups.
 //
 // Launch shapes:
-//   * Greedy, and Sample without top-k, with top-k above kPartMaxK, or on a
-//     vocabulary of at most kPartChunk entries: one work-group per row
-//     (the whole-row path below).
+//   * Greedy, and Sample without top-k on a vocabulary of at most
+//     kMassMinVocab entries, with top-k above kPartMaxK, or with top-k on one
+//     of at most kPartChunk: one work-group per row (the whole-row path
+//     below).
+//   * Sample without top-k on a larger vocabulary: the mass split (its own
+//     comment below).
 //   * Sample with top-k on a larger vocabulary (the split path):
 //     sample_part_kernel, one work-group per (row, chunk of at most
 //     kPartChunk entries), holds its chunk in registers, applies the
@@ -52,10 +55,12 @@
 //     ballot per step;
 //   * the top-p cutoff is the key tau of the item where the descending
 //     cumulative probability first reaches p, i.e. the largest tau whose
-//     tail sum still reaches p: 31 bisection steps over probabilities kept
-//     in LDS; every item with key >= tau is kept (the reference keeps only
-//     as many items tied at tau as its sort order reaches: the one place
-//     the results can differ besides rounding);
+//     tail sum still reaches p, found by weight buckets on an LDS row (one
+//     scan of 1023 exact bucket masses, one of a bucket's 4096 weights) and
+//     by 31 bisection steps over the probabilities otherwise; every item
+//     with key >= tau is kept (the reference keeps only as many items tied
+//     at tau as its sort order reaches: the one place the results can differ
+//     besides rounding);
 //   * sums are per-thread sequential partials combined in a fixed order
 //     (64-lane trees, then the 8 wave results in order), so a call is
 //     deterministic; they round differently from a sequential sum by a few
@@ -121,7 +126,7 @@ struct SampLds {
         // id | count << 18 per distinct id, ascending
         uint32_t win[2 * kCandCap];
     };
-    float region[kRowCap];
+    alignas(16) float region[kRowCap];
 };
 static_assert(2 * kCandCap == kSampMaxSeen, "the window list fills the candidate arrays");
 static_assert(kSampMaxVocab <= (1 << 18) && kSampMaxSeen < (1 << 13), "id | count << 18 fits 31 bits");
@@ -607,6 +612,103 @@ __device__ __forceinline__ void topk_select(Src &c, int top_k, SampLds &s) {
     }
 }
 
+// ---- top-p by weight buckets ---------------------------------------------------
+// fastexp32 of x - m <= 0 is the float whose bits are the integer part of an
+// f32 near 1e9, so down to 2^-32 of the largest weight (bits 1065 to 797
+// million) they are multiples of 64: a bucket is 2^18 bit values (32 buckets
+// an octave, 1023 of them; 4096 possible weights each), its mass the integer
+// sum of the 24-bit significands / 64 -- exact, so no order of summation
+// shows.  The cutoff is the largest weight whose exact tail mass times 1/S1
+// reaches top_p: one scan of the buckets' masses, then one of the counts of
+// the 4096 weights of the bucket it falls in, where a bisection over the
+// float keys takes 31 passes over the set (one work-group, 16 rows, T 0.8,
+// top-p 0.95: V 1000 18.7 -> 10.9 us, 4000 37.9 -> 16.7, 8192 33.4 -> 18.8).
+constexpr int kMassTop = 0x3F79D1C0 >> 18;  // bucket of the largest weight: fastexp32(0)
+__device__ __forceinline__ int mass_bucket(uint32_t bits) { return kMassTop - (int)(bits >> 18); }
+__device__ __forceinline__ uint32_t mass_sig(uint32_t bits) { return ((bits & 0x7FFFFFu) | 0x800000u) >> 6; }
+// Weight of one unit of mass_sig in a bucket: 2^(exponent - 150 + 6).
+__device__ __forceinline__ double mass_unit(int bucket) {
+    return __longlong_as_double((int64_t)(1023 - 144 + ((kMassTop - bucket) >> 5)) << 52);
+}
+
+// Exclusive prefix over the block in thread order, in f64.
+__device__ __forceinline__ double blk_dscan_excl(double v, double *tmp, double *total) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    double inc = v;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const double up = __shfl_up(inc, o);
+        if (lane >= o) inc += up;
+    }
+    __syncthreads();
+    if (lane == 63) tmp[w] = inc;
+    __syncthreads();
+    double base = 0.0, tot = 0.0;
+    for (int i = 0; i < kSW; i++) {
+        if (i < w) base += tmp[i];
+        tot += tmp[i];
+    }
+    *total = tot;
+    return base + (inc - v);
+}
+
+// The bucket in which the tail mass times i1 reaches top_p, from the masses
+// d0, d1 of buckets 2 tid and 2 tid + 1 (kMassBuckets: below them all), and
+// *above, the mass of the heavier ones.  tmp: kSW + 1 doubles of LDS.
+__device__ __forceinline__ int mass_find_bucket(double d0, double d1, double i1, float top_p, double *tmp,
+                                                int *best, double *above) {
+    const int tid = threadIdx.x;
+    if (tid == 0) *best = kMassBuckets;
+    double total;
+    const double ex = blk_dscan_excl(d0 + d1, tmp, &total);
+    if ((ex + d0) * i1 >= (double)top_p)
+        atomicMin(best, 2 * tid);
+    else if ((ex + (d0 + d1)) * i1 >= (double)top_p)
+        atomicMin(best, 2 * tid + 1);
+    __syncthreads();
+    const int bk = *best;
+    if (tid == (bk >> 1)) tmp[kSW] = (bk & 1) ? ex + d0 : ex;
+    __syncthreads();
+    *above = tmp[kSW];
+    return bk;
+}
+// The bits of the lightest weight kept, from the counts cnt[4096] of bucket
+// bk's weights; *mass: the tail mass there.
+__device__ __forceinline__ uint32_t mass_find_tau(const uint32_t *cnt, int bk, double above, double i1,
+                                                  float top_p, double *tmp, int *best, double *mass) {
+    const int tid = threadIdx.x;
+    const uint32_t base = (uint32_t)(kMassTop - bk) << 18;
+    const double unit = mass_unit(bk), p = (double)top_p;
+    // weights from the heaviest, 8 a thread
+    uint32_t n[8];
+#pragma unroll
+    for (int k = 0; k < 8; k++) n[k] = cnt[4095 - (8 * tid + k)];
+    double mine = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) mine += (double)n[k] * (double)mass_sig(base + 64u * (4095 - (8 * tid + k)));
+    if (tid == 0) *best = 4096;
+    double bt;
+    double cum = blk_dscan_excl(mine, tmp, &bt);
+    int at = 4096;
+    double m = 0.0;
+#pragma unroll
+    for (int k = 0; k < 8; k++) {
+        cum += (double)n[k] * (double)mass_sig(base + 64u * (4095 - (8 * tid + k)));
+        if (at == 4096 && n[k] != 0u && (above + cum * unit) * i1 >= p) {
+            at = 8 * tid + k;
+            m = above + cum * unit;
+        }
+    }
+    if (at < 4096) atomicMin(best, at);
+    __syncthreads();
+    const int first = *best;
+    if (first < 4096 ? at == first : tid == 0) tmp[kSW] = first < 4096 ? m : above + bt * unit;
+    __syncthreads();
+    *mass = tmp[kSW];
+    // (4096: the two prefixes round apart, the whole bucket is kept)
+    return first < 4096 ? base + 64u * (uint32_t)(4095 - first) : base;
+}
+
 // Softmax, top-p, min-p and the draw (sampler.go:117-206) over a working
 // set in mode M.
 template <int M>
@@ -626,7 +728,50 @@ __device__ __forceinline__ int sample_finish(Src &c, float top_p, float min_p, f
     const float S1 = blk_sum(sm, s);
     c.n1 = S1 > 0.f;
     c.i1 = c.n1 ? __fdiv_rn(1.f, S1) : 1.f;
-    if constexpr (M != 2) {  // values -> stage-1 probabilities, in place
+    // Top-p on an LDS row by weight buckets; a cutoff below them, and the
+    // other modes, search below.
+    uint32_t tau = 0;
+    bool found = false;
+    if constexpr (M == 0) {
+        if (top_p > 0.f && top_p < 1.f && c.n1) {
+            unsigned long long *hist = (unsigned long long *)s.cv;
+            uint32_t *cnt = (uint32_t *)s.cv;
+            double *tmp = (double *)s.key;
+            for (int i = tid; i < kMassBuckets; i += kST) hist[i] = 0ull;
+            __syncthreads();
+#pragma unroll 8
+            for (int i = tid; i < c.n; i += kST) {
+                const float x = s.region[i];
+                const float p = (x == -INFINITY) ? 0.f : fastexp32_dev(__fsub_rn(x, c.m));
+                s.region[i] = p;
+                const int bk = mass_bucket(__float_as_uint(p));
+                if ((uint32_t)bk < (uint32_t)(kMassBuckets - 1))
+                    atomicAdd(&hist[bk], (unsigned long long)mass_sig(__float_as_uint(p)));
+            }
+            __syncthreads();
+            double above, mass;
+            const int bk = mass_find_bucket((double)hist[2 * tid] * mass_unit(2 * tid),
+                                            (double)hist[2 * tid + 1] * mass_unit(2 * tid + 1), (double)c.i1,
+                                            top_p, tmp, &s.best, &above);
+            found = bk < kMassBuckets;
+            if (found) {
+                for (int i = tid; i < 4096; i += kST) cnt[i] = 0u;
+                __syncthreads();
+#pragma unroll 8
+                for (int i = tid; i < c.n; i += kST) {
+                    const uint32_t w = __float_as_uint(s.region[i]);
+                    if (mass_bucket(w) == bk) atomicAdd(&cnt[(w >> 6) & 4095u], 1u);
+                }
+                __syncthreads();
+                const uint32_t t = mass_find_tau(cnt, bk, above, (double)c.i1, top_p, tmp, &s.best, &mass);
+                tau = fkey(__fmul_rn(__uint_as_float(t), c.i1));
+            }
+#pragma unroll 8
+            for (int i = tid; i < c.n; i += kST) s.region[i] = __fmul_rn(s.region[i], c.i1);
+            __syncthreads();
+        }
+    }
+    if (M == 1 || (M == 0 && !(top_p > 0.f && top_p < 1.f && c.n1))) {  // values -> stage-1 probabilities, in place
         float *lw = M == 0 ? s.region : s.cv;
 #pragma unroll 8
         for (int i = tid; i < c.n; i += kST) {
@@ -671,6 +816,8 @@ __device__ __forceinline__ int sample_finish(Src &c, float top_p, float min_p, f
             __syncthreads();
             res = (uint32_t)s.sel_i[0];
             __syncthreads();
+        } else if (found) {
+            res = tau;
         } else {
             auto tail = [&](uint32_t t) {
                 float a = 0.f;
@@ -1451,6 +1598,369 @@ __global__ __launch_bounds__(kST) void sample_part_kernel(const SampleArgs a) {
     }
 }
 
+// ---- Sample without top-k over vocabulary chunks ------------------------------
+// The whole-row path walks the vocabulary 31 times for the top-p cutoff, one
+// work-group a row.  Split, work-groups of one (row, chunk):
+//   * sample_max_kernel: penalties, temperature, the scratch values stored,
+//     the chunk's largest;
+//   * sample_mass_kernel: with the row's largest m, each entry's fastexp32
+//     weight and the mass of the weights by bucket;
+//   * sample_cut_kernel (top-p): the bucket the cutoff falls in, from the
+//     row's buckets; the entries in it are listed, the mass of the heavier
+//     ones summed per 256 entries (without top-p sample_mass_kernel sums);
+// then mass_finish in sample_kernel, a work-group per row: the exact cutoff
+// among the listed entries, min-p, the draw over the 256-entry sums and the
+// walk of the one it falls in.
+//
+// A chunk's bucket mass fits 32 bits (8192 entries of 18-bit units).  Lighter
+// weights, and NaN and overflow (weight 0), are summed in f32 in a fixed
+// order.  A cutoff below the buckets (top_p within 1e-4 of 1) or more than
+// kMassList entries of a chunk to be decided (nearly constant rows) take the
+// whole-row path.
+//
+// Bound: launches and round trips (3 or 4 launches; 4 B per entry read from
+// HBM, 8 written and 12 read again in L2).  16 rows of 50257, T 0.8, top-p
+// 0.95: 845 us (whole row, 31 passes over memory by one work-group a row) ->
+// 29.2 us (max 5, mass 6, cut 9, finish 9); temperature alone 82 -> 18 us.
+struct alignas(16) MassLds {
+    float red[2][kSW];
+    double dtmp[kSW + 1];
+    int best, n;
+    union {
+        uint32_t hist[kMassBuckets];
+        uint32_t pcw[kPartChunk / 2];  // penalty slots of the chunk
+    };
+};
+
+template <int R>
+__device__ __forceinline__ void mass_max(const SampleArgs &a, int lo, int n, MassLds &s) {
+    const int b = blockIdx.x;
+    const int64_t q = (int64_t)b * a.uch + blockIdx.y;
+    float x[4 * R];
+    reg_load<R>(a.logits + (int64_t)b * a.stride + lo, n, x);
+    if (a.hist || a.seen_off) {
+        WinIds w;
+        win_load(a, b, w);
+        reg_penalties<R>(a, w, lo, n, x, s.pcw);
+    }
+    float t = a.temperature;
+    if (t <= 0.f) t = 1e-5f;
+    float mx = -INFINITY;
+    float *o = a.mass_p + q * a.upch;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const int e = reg_idx(j, 0);
+        if (t != 1.f) {
+#pragma unroll
+            for (int k = 0; k < 4; k++) x[4 * j + k] = __fdiv_rn(x[4 * j + k], t);
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            if (e + k >= n) x[4 * j + k] = -INFINITY;  // (past the row)
+            mx = fmaxf(mx, x[4 * j + k]);
+        }
+        if (e < a.upch) *(float4 *)(o + e) = make_float4(x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]);
+    }
+    mx = blk_max(mx, s);
+    if (threadIdx.x == 0) a.mass_r[q].max = mx;
+}
+__global__ __launch_bounds__(kST) void sample_max_kernel(const SampleArgs a) {
+    __shared__ MassLds s;
+    const int lo = blockIdx.y * a.upch, n = min(a.V - lo, a.upch);
+    if (a.upch <= 8 * kST)
+        mass_max<2>(a, lo, n, s);
+    else
+        mass_max<4>(a, lo, n, s);
+}
+
+// min-p keeps weights of at least min_p times the heaviest (fastexp32(0)),
+// both scaled by 1/S1 and 1/S2 with rounding: certain above hi, impossible
+// below lo (the four roundings are within 2^-22), decided exactly between.
+struct MassMinp {
+    uint32_t lo, hi;
+};
+__device__ __forceinline__ MassMinp mass_minp(float min_p) {
+    if (!(min_p > 0.f)) return MassMinp{0u, 0u};
+    const float m = fastexp32_dev(0.f) * min_p;
+    return MassMinp{__float_as_uint(m * (1.f - 0x1p-20f)), __float_as_uint(m * (1.f + 0x1p-20f))};
+}
+
+// A chunk's weights in registers: the mass certain to be kept of each wave's
+// 256 entries, and the entries to be decided (bucket bk, the top-p cutoff's,
+// -1 without top-p; or between the min-p bounds).
+template <int R>
+__device__ __forceinline__ void mass_collect(const SampleArgs &a, const uint32_t (&w)[4 * R], int bk, MassLds &s) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t q = (int64_t)blockIdx.x * a.uch + blockIdx.y;
+    const MassMinp mp = mass_minp(a.min_p);
+    if (tid == 0) s.n = 0;
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        float sum = 0.f;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const uint32_t v = w[4 * j + k];
+            const int d = mass_bucket(v) - bk;  // (bk -1: never 0, heavier ones only by min-p)
+            const bool heavy = bk < 0 || d < 0, at = bk >= 0 && d == 0;
+            if ((at && v >= mp.lo) || (heavy && v >= mp.lo && v <= mp.hi && v != 0u)) {
+                const int i = atomicAdd(&s.n, 1);
+                if (i < kMassList)
+                    a.mass_l[q * kMassList + i] = make_uint2(v, (uint32_t)(reg_idx(j, k)));
+            } else if (at) {
+                // below the min-p bounds: only the cutoff's search needs it
+                const int i = atomicAdd(&s.n, 1);
+                if (i < kMassList) a.mass_l[q * kMassList + i] = make_uint2(v, 0xFFFFFFFFu);
+            } else if (heavy && v > mp.hi) {
+                sum += __uint_as_float(v);
+            }
+        }
+        sum = wave_sum_dpp(sum);
+        if (lane == 0 && j * kSW + wave < a.useg) a.mass_s[q * a.useg + j * kSW + wave] = sum;
+    }
+    __syncthreads();
+    if (tid == 0) a.mass_r[q].n_list = s.n;
+}
+
+__device__ __forceinline__ bool mass_topp(const SampleArgs &a) { return a.top_p > 0.f && a.top_p < 1.f; }
+
+template <int R>
+__device__ __forceinline__ void mass_weights(const SampleArgs &a, MassLds &s) {
+    const int tid = threadIdx.x, b = blockIdx.x;
+    const int64_t q = (int64_t)b * a.uch + blockIdx.y;
+    float *p = a.mass_p + q * a.upch;
+    float x[4 * R];
+    reg_load<R>(p, a.upch, x);
+    const bool topp = mass_topp(a);
+    for (int i = tid; i < kMassBuckets; i += kST) s.hist[i] = 0u;
+    // the row's largest scratch value from its chunks' (every wave by itself)
+    float m = -INFINITY;
+    for (int c = tid & 63; c < a.uch; c += 64) m = fmaxf(m, a.mass_r[(int64_t)b * a.uch + c].max);
+    m = wave_max_dpp(m);
+    __syncthreads();
+    float rest = 0.f;
+    double own = 0.0;
+    uint32_t bits[4 * R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        const int e = reg_idx(j, 0);
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float v = x[4 * j + k];
+            const float w = v == -INFINITY ? 0.f : fastexp32_dev(__fsub_rn(v, m));
+            bits[4 * j + k] = __float_as_uint(w);
+            const int bk = mass_bucket(bits[4 * j + k]);
+            if ((uint32_t)bk < (uint32_t)(kMassBuckets - 1)) {
+                own += (double)w;
+                if (topp) atomicAdd(&s.hist[bk], mass_sig(bits[4 * j + k]));
+            } else {
+                rest += w;
+            }
+        }
+        if (e < a.upch)
+            *(u32x4 *)((uint32_t *)p + e) = u32x4{bits[4 * j], bits[4 * j + 1], bits[4 * j + 2], bits[4 * j + 3]};
+    }
+    double total;
+    (void)blk_dscan_excl(own, s.dtmp, &total);
+    rest = blk_sum(rest, s);  // (its barriers complete the histogram)
+    if (tid == 0) {
+        a.mass_r[q].total = total;
+        a.mass_r[q].rest = rest;
+    }
+    if (topp) {
+        for (int i = tid; i < kMassBuckets / 2; i += kST)
+            ((uint2 *)(a.mass_h + q * kMassBuckets))[i] = ((const uint2 *)s.hist)[i];
+    } else {
+        mass_collect<R>(a, bits, -1, s);
+    }
+}
+__global__ __launch_bounds__(kST) void sample_mass_kernel(const SampleArgs a) {
+    __shared__ MassLds s;
+    if (a.upch <= 8 * kST)
+        mass_weights<2>(a, s);
+    else
+        mass_weights<4>(a, s);
+}
+
+// S1 of a row from its chunks' records (at most 64: one a lane), and the
+// longest of their lists.
+__device__ __forceinline__ float mass_s1(const SampleArgs &a, int b, int &most) {
+    const int lane = threadIdx.x & 63;
+    double t = 0.0;
+    most = 0;
+    if (lane < a.uch) {
+        const MassRec m = a.mass_r[(int64_t)b * a.uch + lane];
+        t = m.total + (double)m.rest;
+        most = m.n_list;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        t += __shfl_xor(t, o);
+        most = max(most, __shfl_xor(most, o));
+    }
+    return (float)t;
+}
+
+template <int R>
+__device__ __forceinline__ void mass_cut(const SampleArgs &a, MassLds &s) {
+    const int tid = threadIdx.x, b = blockIdx.x;
+    const int64_t q0 = (int64_t)b * a.uch, q = q0 + blockIdx.y;
+    float x[4 * R];
+    reg_load<R>(a.mass_p + q * a.upch, a.upch, x);
+    // Buckets 2 tid, 2 tid + 1 of the row, then the prefix from the heaviest.
+    uint64_t h0 = 0, h1 = 0;
+#pragma unroll 8
+    for (int c = 0; c < a.uch; c++) {
+        const uint2 v = ((const uint2 *)(a.mass_h + (q0 + c) * kMassBuckets))[tid];
+        h0 += v.x;
+        h1 += v.y;
+    }
+    int most;
+    const float S1 = mass_s1(a, b, most);
+    const double i1 = S1 > 0.f ? (double)__fdiv_rn(1.f, S1) : 0.0;
+    double above;
+    const int bk = mass_find_bucket((double)h0 * mass_unit(2 * tid), (double)h1 * mass_unit(2 * tid + 1), i1,
+                                    a.top_p, s.dtmp, &s.best, &above);
+    if (tid == 0) {
+        a.mass_r[q].bucket = bk < kMassBuckets ? bk : -1;
+        a.mass_r[q].above = above;
+    }
+    if (bk >= kMassBuckets) return;
+    uint32_t w[4 * R];
+#pragma unroll
+    for (int i = 0; i < 4 * R; i++) w[i] = reg_idx(i / 4, i % 4) < a.upch ? __float_as_uint(x[i]) : 0u;
+    mass_collect<R>(a, w, bk, s);
+}
+__global__ __launch_bounds__(kST) void sample_cut_kernel(const SampleArgs a) {
+    __shared__ MassLds s;
+    if (a.upch <= 8 * kST)
+        mass_cut<2>(a, s);
+    else
+        mass_cut<4>(a, s);
+}
+
+constexpr int kMassSegs = 1024;  // 256-entry sums of the longest row
+static_assert(kSampMaxVocab / kPartChunk * (kPartChunk / 256) <= kMassSegs && kMassSegs <= 2 * kST,
+              "two sums a thread");
+constexpr double kMassFix = 0x1p50;  // weights as integers: exact down to the lightest bucket
+
+// The row's token (sampler.go:117-206), or -1 where the whole-row path has
+// to serve it.
+__device__ __forceinline__ int mass_finish(const SampleArgs &a, int b, float min_p, float r, SampLds &s) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int64_t q0 = (int64_t)b * a.uch;
+    uint32_t *cnt = (uint32_t *)s.region;                          // weights of the cutoff bucket
+    unsigned long long *add = (unsigned long long *)(s.region + 4096);  // listed mass per 256 entries
+    double *tmp = (double *)(s.region + 4096 + 2 * kMassSegs);
+    const bool topp = mass_topp(a);
+    const MassRec r0 = a.mass_r[q0];
+    const int nseg = a.uch * a.useg;
+    float s0 = 2 * tid < nseg ? a.mass_s[q0 * a.useg + 2 * tid] : 0.f;
+    float s1 = 2 * tid + 1 < nseg ? a.mass_s[q0 * a.useg + 2 * tid + 1] : 0.f;
+    // Wave w takes the lists of chunks w, w + 8, ..; its first 64 entries stay
+    // in registers for the second walk.
+    const int n0 = wave < a.uch ? min(a.mass_r[q0 + wave].n_list, kMassList) : 0;
+    const uint2 first = a.mass_l[(q0 + min(wave, a.uch - 1)) * kMassList + lane];
+    for (int i = tid; i < 4096; i += kST) cnt[i] = 0u;
+    for (int i = tid; i < kMassSegs; i += kST) add[i] = 0ull;
+    int most;
+    const float S1 = mass_s1(a, b, most);
+    if (!(S1 > 0.f) || (topp && r0.bucket < 0) || ((topp || min_p > 0.f) && most > kMassList)) return -1;
+    const float i1 = __fdiv_rn(1.f, S1);
+    auto listed = [&](auto f) {
+        if (lane < n0) f(first, wave);
+        for (int c = wave; c < a.uch; c += kSW) {
+            const int n = c == wave ? n0 : a.mass_r[q0 + c].n_list;
+            for (int i = lane + (c == wave ? 64 : 0); i < n; i += 64) f(a.mass_l[(q0 + c) * kMassList + i], c);
+        }
+    };
+    __syncthreads();
+    uint32_t tau = 0;  // bits of the lightest weight kept
+    float i2 = 1.f;
+    if (topp) {
+        listed([&](uint2 v, int) {
+            if (mass_bucket(v.x) == r0.bucket) atomicAdd(&cnt[(v.x >> 6) & 4095u], 1u);
+        });
+        __syncthreads();
+        double mass;
+        tau = mass_find_tau(cnt, r0.bucket, r0.above, (double)i1, a.top_p, tmp, &s.best, &mass);
+        const float S2 = (float)(mass * (double)i1);
+        if (S2 > 0.f) i2 = __fdiv_rn(1.f, S2);
+    }
+    // Weight after softmax and top-p (both scalings rounded), and the min-p
+    // floor (the heaviest entry has weight fastexp32(0)).
+    auto kept = [&](uint32_t bits) {
+        return bits >= tau ? __fmul_rn(__fmul_rn(__uint_as_float(bits), i1), i2) : 0.f;
+    };
+    const float thr = min_p > 0.f ? __fmul_rn(kept(__float_as_uint(fastexp32_dev(0.f))), min_p) : 0.f;
+    if (topp || min_p > 0.f) {
+        listed([&](uint2 v, int c) {
+            if (v.y == 0xFFFFFFFFu || v.x < tau || kept(v.x) < thr) return;
+            atomicAdd(&add[c * a.useg + (int)(v.y >> 8)],
+                      (unsigned long long)((double)__uint_as_float(v.x) * kMassFix));
+        });
+        __syncthreads();
+    }
+    const double m0 = (double)s0 + (double)add[2 * tid] * (1.0 / kMassFix);
+    const double m1 = (double)s1 + (double)add[2 * tid + 1] * (1.0 / kMassFix);
+    double total;
+    const double ex = blk_dscan_excl(m0 + m1, tmp, &total);
+    float i3 = 1.f;
+    if (min_p > 0.f) {
+        const float S3 = (float)(total * (double)i1 * (double)i2);
+        if (S3 > 0.f) i3 = __fdiv_rn(1.f, S3);
+    }
+    // Categorical draw: the first 256 entries whose end passes r, then their walk.
+    const double scale = (double)i1 * (double)i2 * (double)i3, rd = (double)r;
+    if (tid == 0) s.best = INT_MAX;
+    __syncthreads();
+    if (rd < (ex + m0) * scale)
+        atomicMin(&s.best, 2 * tid);
+    else if (rd < (ex + (m0 + m1)) * scale)
+        atomicMin(&s.best, 2 * tid + 1);
+    __syncthreads();
+    const int g = s.best;
+    if (g == INT_MAX) return a.V - 1;
+    if (tid == g >> 1) tmp[kSW] = ((g & 1) ? ex + m0 : ex) * scale;
+    __syncthreads();
+    if (wave == 0) {
+        const int c = g / a.useg, at = (g - c * a.useg) * 256 + 4 * lane, e0 = c * a.upch + at;
+        float w[4] = {0.f, 0.f, 0.f, 0.f};
+        if (at < a.upch) {
+            const u32x4 v = *(const u32x4 *)((const uint32_t *)a.mass_p + (q0 + c) * a.upch + at);
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const float y = kept(v[k]);
+                w[k] = min_p > 0.f ? (y < thr ? 0.f : __fmul_rn(y, i3)) : y;
+            }
+        }
+        double inc = ((double)w[0] + w[1]) + ((double)w[2] + w[3]), own = inc;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const double up = __shfl_up(inc, o);
+            if (lane >= o) inc += up;
+        }
+        double cum = tmp[kSW] + (inc - own);
+        int hit = INT_MAX, last = -1;
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            cum += (double)w[k];
+            if (w[k] > 0.f) last = e0 + k;
+            if (hit == INT_MAX && rd < cum) hit = e0 + k;
+        }
+        // the first hit; should rounding leave none, the last entry with weight
+        const uint64_t any = __ballot(hit != INT_MAX), some = __ballot(last >= 0);
+        int t = a.V - 1;
+        if (any)
+            t = __shfl(hit, __builtin_ctzll(any));
+        else if (some)
+            t = __shfl(last, 63 - __builtin_clzll(some));
+        if (lane == 0) s.sel_i[0] = t;
+    }
+    __syncthreads();
+    return min(s.sel_i[0], a.V - 1);
+}
+
 // Sample, one work-group per row: phase two of the split path when the
 // chunk lists are there, else the whole row.
 __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs a) {
@@ -1469,6 +1979,14 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs a) {
             if (threadIdx.x == 0) a.out[b] = t;
             return;
         }
+    }
+    if (a.uch > 0) {
+        const int t = mass_finish(a, b, a.min_p, a.u[b], s);
+        if (t >= 0) {
+            if (threadIdx.x == 0) a.out[b] = t;
+            return;
+        }
+        __syncthreads();
     }
     const float *row = a.logits + (int64_t)b * a.stride;
     if (a.hist) {
@@ -1768,16 +2286,38 @@ __global__ __launch_bounds__(kST) void spec_final_kernel(const SpecArgs a) {
     }
 }
 
-hipError_t launch_sample(hipStream_t st, const SampleArgs &a, int n_rows, hipEvent_t e0,
+hipError_t launch_sample(hipStream_t st, const SampleArgs &args, int n_rows, hipEvent_t e0,
                          hipEvent_t e1) {
     if (e0) (void)hipEventRecord(e0, st);
-    if (a.nch > 0) {
-        sample_part_kernel<<<dim3(n_rows, a.nch), dim3(kST), 0, st>>>(a);
-        const hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
+    hipError_t e = hipSuccess;
+    SampleArgs a = args;
+    const int step = a.uch > 0 ? a.urows : n_rows;
+    for (int r0 = 0; r0 < n_rows && e == hipSuccess; r0 += step) {
+        const int n = min(step, n_rows - r0);
+        if (a.uch > 0) {
+            sample_max_kernel<<<dim3(n, a.uch), dim3(kST), 0, st>>>(a);
+            if ((e = hipGetLastError()) != hipSuccess) break;
+            sample_mass_kernel<<<dim3(n, a.uch), dim3(kST), 0, st>>>(a);
+            if ((e = hipGetLastError()) != hipSuccess) break;
+            if (a.top_p > 0.f && a.top_p < 1.f) {
+                sample_cut_kernel<<<dim3(n, a.uch), dim3(kST), 0, st>>>(a);
+                if ((e = hipGetLastError()) != hipSuccess) break;
+            }
+        } else if (a.nch > 0) {
+            sample_part_kernel<<<dim3(n, a.nch), dim3(kST), 0, st>>>(a);
+            if ((e = hipGetLastError()) != hipSuccess) break;
+        }
+        sample_kernel<<<dim3(n), dim3(kST), 0, st>>>(a);
+        e = hipGetLastError();
+        a.logits += (int64_t)n * a.stride;
+        a.u += n;
+        a.out += n;
+        if (a.seen_off) a.seen_off += n;
+        if (a.hist) {
+            a.hist += (int64_t)n * a.hist_stride;
+            a.hist_len += n;
+        }
     }
-    sample_kernel<<<dim3(n_rows), dim3(kST), 0, st>>>(a);
-    const hipError_t e = hipGetLastError();
     if (e1) (void)hipEventRecord(e1, st);
     return e;
 }
@@ -1833,6 +2373,29 @@ void topk_split(int V, int top_k, int &nch, int &pch, int &pcap) {
     pcap = cap;
 }
 
+// Mass split (top-k off): chunks of up to kPartChunk entries, as many rows
+// at a time as 64 MiB of scratch hold.  Taken past 12288 entries, where the
+// whole row in one work-group's LDS starts to cost more than three or four
+// launches (16 rows, us, whole row / split: top-p at V 8200 18 / 27, 16000
+// 33 / 27, 32000 43 / 27; temperature alone 10 / 16, 22 / 16, 25 / 16).
+constexpr int kMassMinVocab = 12288;
+constexpr int64_t kMassScratch = 64 << 20;
+void mass_split(SampleArgs &a, int n_rows) {
+    a.uch = a.upch = a.useg = a.urows = 0;
+    a.mass_p = a.mass_s = nullptr;
+    a.mass_h = nullptr;
+    a.mass_l = nullptr;
+    a.mass_r = nullptr;
+    const bool topk = a.top_k > 0 && a.top_k < a.V;
+    if (topk || a.V <= kMassMinVocab || a.V > kSampMaxVocab) return;
+    const int n = (a.V + kPartChunk - 1) / kPartChunk;
+    a.upch = ((a.V + n - 1) / n + 3) & ~3;
+    a.uch = (a.V + a.upch - 1) / a.upch;
+    a.useg = (a.upch + 255) / 256;
+    const int64_t row = (int64_t)a.uch * (a.upch * 4 + kMassBuckets * 4 + kMassList * 8 + a.useg * 4 + 32);
+    a.urows = (int)max((int64_t)1, min((int64_t)n_rows, kMassScratch / row));
+}
+
 int64_t carve(int64_t &off, int64_t bytes) {
     const int64_t at = off;
     off += (bytes + 255) & ~(int64_t)255;
@@ -1844,8 +2407,25 @@ int64_t plan_sample_split(SampleArgs &a, int n_rows, char *base) {
     topk_split(a.V, a.top_k, a.nch, a.pch, a.pcap);
     a.part_v = nullptr;
     a.part_i = a.part_n = nullptr;
-    if (a.nch == 0) return 0;
+    mass_split(a, n_rows);
     int64_t off = 0;
+    if (a.uch > 0) {
+        const int64_t chunks = (int64_t)a.urows * a.uch;
+        const int64_t o_p = carve(off, chunks * a.upch * 4);
+        const int64_t o_h = carve(off, chunks * kMassBuckets * 4);
+        const int64_t o_l = carve(off, chunks * kMassList * 8);
+        const int64_t o_s = carve(off, chunks * a.useg * 4);
+        const int64_t o_r = carve(off, chunks * (int64_t)sizeof(MassRec));
+        if (base) {
+            a.mass_p = (float *)(base + o_p);
+            a.mass_h = (uint32_t *)(base + o_h);
+            a.mass_l = (uint2 *)(base + o_l);
+            a.mass_s = (float *)(base + o_s);
+            a.mass_r = (MassRec *)(base + o_r);
+        }
+        return off;
+    }
+    if (a.nch == 0) return 0;
     const int64_t slots = (int64_t)n_rows * a.nch * a.pcap;
     const int64_t o_n = carve(off, (int64_t)n_rows * a.nch * 16);
     const int64_t o_v = carve(off, slots * 4);
