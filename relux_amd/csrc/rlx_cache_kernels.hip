@@ -78,73 +78,143 @@ hipError_t launch_page_copy(hipStream_t s, const uint64_t *src, const uint64_t *
     return hipGetLastError();
 }
 
-// GQA append.  Thread = (token, kv head, 8-dim chunk of the stored head
-// dim hd).  K goes to its page (k_page_off layout) with one 16-byte store; V
-// goes to a dim-major page (8 strided 2-byte stores).  The caller's rows
-// hold hdi <= hd dims (a multiple of 8); the stored dims past hdi are
-// written as zeros.  The first n_patch threads also apply the table
-// patches; the scatter itself takes its destinations from the plan, not the
-// table.
-template <bool ARG>
+// GQA append of runs (up to 8 tokens in one 8-slot group of a page).  K goes
+// to its page (k_page_off layout) with a 16-byte store per token and 8-dim
+// chunk of the stored head dim hd, V to a dim-major page.  The caller's rows
+// hold hdi <= hd dims (a multiple of 8); the stored dims past hdi are written
+// as zeros.  The first n_patch threads also apply the table patches; the
+// scatter itself takes its destinations from the plan, not the table.
+//
+// kAppTok: thread = (run, token t < per, kv head, chunk), 8 strided 2-byte V
+// stores, for verify steps.  kAppFlat: the same with one token per run and
+// rows in call order (a decode step), whose addresses wait for no record.
+// kAppRun: thread = (run, kv head, chunk), all loads of its tokens before the
+// stores; a full run's 8 x 8 block of V is turned in registers and stored as 8
+// 16-byte pieces of a dim each (a shorter run, at a prompt's ends, as above).
+//
+// Bound: the launch at decode sizes, then memory (2 B read and written per
+// element) and, with 2-byte stores, the store rate.  5 600 tokens x 8 kv heads
+// x 128 dims: 27.3 us a token per thread, 14.2 by whole runs.
+constexpr int kAppFlat = 0, kAppTok = 1, kAppRun = 2;
+template <bool ARG, int MODE>
 __global__ void kv_append_kernel(typename PlanSel<ARG>::T plan, uint16_t *__restrict__ kpool,
                                  uint16_t *__restrict__ vpool, int32_t *__restrict__ table,
                                  const Patch *__restrict__ patches, int n_patch,
-                                 const AppendTok *__restrict__ toks, int tok_off, int n_tok,
+                                 const AppendRun *__restrict__ runs, int run_off, int n_runs, int per,
                                  const void *__restrict__ k_src, const void *__restrict__ v_src,
-                                 int src_bf16, int layout, int kvh, int hd, int hdi, int P) {
+                                 int src_bf16, int tok_row, int kvh, int hd, int hdi, int P) {
     int64_t gid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (gid < n_patch) {
         const Patch pt = plan_patch<ARG>(patches, (int)gid);
         table[pt.idx] = pt.val;
     }
-    const int chunks = hd >> 3;
-    const int64_t per_tok = (int64_t)kvh * chunks;
-    if (gid >= (int64_t)n_tok * per_tok) return;
-    const int t = (int)(gid / per_tok);
-    const int rem = (int)(gid - (int64_t)t * per_tok);
+    const int chunks = hd >> 3, per_tok = kvh * chunks;
+    const int64_t total = (int64_t)n_runs * per * per_tok;
+    if (gid >= total) return;
+    // (run, token); 32-bit division where it fits
+    const int u = total <= 0xFFFFFFFFll ? (int)((uint32_t)gid / (uint32_t)per_tok) : (int)(gid / per_tok);
+    const int rem = (int)(gid - (int64_t)u * per_tok);
     const int h = rem / chunks;
     const int d0 = (rem - h * chunks) * 8;
-    const AppendTok tk = plan_tok<ARG>(toks, tok_off, t);
-    const int j = t - tk.seq_row0;  // row within its sequence
-    int64_t src_off;
-    if (layout == kLayoutSHD)
-        src_off = ((int64_t)t * kvh + h) * hdi + d0;
-    else
-        src_off = (int64_t)tk.seq_row0 * kvh * hdi + ((int64_t)h * tk.seq_n + j) * hdi + d0;
-    uint16_t kv[8] = {0, 0, 0, 0, 0, 0, 0, 0}, vv[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (d0 < hdi) {
-        load8_bf16(k_src, src_off, src_bf16, kv);
-        load8_bf16(v_src, src_off, src_bf16, vv);
+    const int i = MODE == kAppTok ? u / per : u;
+    const AppendRun run = plan_run<ARG>(runs, run_off, i);
+    const int n = (int)(run.head_n >> 29) + 1;
+    const int64_t src = (MODE == kAppFlat ? (int64_t)u * kvh + h
+                                          : (int64_t)run.row + (int64_t)h * (run.head_n & 0x1FFFFFFFu)) * hdi + d0;
+    const int64_t step = (int64_t)tok_row * hdi;  // elements from one token to the next
+    auto load = [&](const void *p, int t) {
+        uint16_t e[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (d0 < hdi) load8_bf16(p, src + t * step, src_bf16, e);
+        u32x4 r;
+#pragma unroll
+        for (int j = 0; j < 4; j++) r[j] = (uint32_t)e[2 * j] | ((uint32_t)e[2 * j + 1] << 16);
+        return r;
+    };
+    uint16_t *kd = kpool + ((int64_t)run.page * kvh + h) * P * hd;
+    uint16_t *vd = vpool + (((int64_t)run.page * kvh + h) * hd + d0) * P + run.slot;
+    auto put = [&](int t, const u32x4 &k, const u32x4 &v) {
+        *(u32x4 *)(kd + k_page_off(run.slot + t, d0, hd)) = k;
+#pragma unroll
+        for (int d = 0; d < 8; d++) vd[(int64_t)d * P + t] = (uint16_t)(v[d >> 1] >> (16 * (d & 1)));
+    };
+    if constexpr (MODE != kAppRun) {
+        const int t = MODE == kAppTok ? u - i * per : 0;
+        if (t >= n) return;
+        const u32x4 k = load(k_src, t), v = load(v_src, t);
+        put(t, k, v);
+    } else {
+        u32x4 kv[8], vv[8];
+        if (n == 8) {  // (slot is a multiple of 8)
+#pragma unroll
+            for (int t = 0; t < 8; t++) {
+                kv[t] = load(k_src, t);
+                vv[t] = load(v_src, t);
+            }
+#pragma unroll
+            for (int t = 0; t < 8; t++) *(u32x4 *)(kd + k_page_off(run.slot + t, d0, hd)) = kv[t];
+#pragma unroll
+            for (int d = 0; d < 8; d++) {
+                u32x4 w;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const uint32_t lo = vv[2 * j][d >> 1] >> (16 * (d & 1));
+                    const uint32_t hi = vv[2 * j + 1][d >> 1] >> (16 * (d & 1));
+                    w[j] = (lo & 0xFFFFu) | (hi << 16);
+                }
+                *(u32x4 *)(vd + (int64_t)d * P) = w;
+            }
+            return;
+        }
+#pragma unroll
+        for (int t = 0; t < 7; t++)
+            if (t < n) {
+                kv[t] = load(k_src, t);
+                vv[t] = load(v_src, t);
+            }
+#pragma unroll
+        for (int t = 0; t < 7; t++)
+            if (t < n) put(t, kv[t], vv[t]);
     }
-    uint16_t *kd = kpool + ((int64_t)tk.page * kvh + h) * P * hd + k_page_off(tk.slot, d0, hd);
-    u32x4 pk;
-#pragma unroll
-    for (int i = 0; i < 4; i++) pk[i] = (uint32_t)kv[2 * i] | ((uint32_t)kv[2 * i + 1] << 16);
-    *(u32x4 *)kd = pk;
-    uint16_t *vd = vpool + (((int64_t)tk.page * kvh + h) * hd + d0) * P + tk.slot;
-#pragma unroll
-    for (int i = 0; i < 8; i++) vd[(int64_t)i * P] = vv[i];
 }
 
-hipError_t launch_kv_append(hipStream_t s, const PlanArg *plan, int tok_off, uint16_t *kpool,
+hipError_t launch_kv_append(hipStream_t s, const PlanArg *plan, int run_off, uint16_t *kpool,
                             uint16_t *vpool, int32_t *table, const Patch *patches, int n_patch,
-                            const AppendTok *toks, int n_tok, const void *k_src, const void *v_src,
-                            int src_bf16, int layout, int kvh, int hd, int hdi, int P) {
-    int64_t work = (int64_t)n_tok * kvh * (hd / 8);
+                            const AppendRun *runs, int n_runs, int most, const void *k_src,
+                            const void *v_src, int src_bf16, int layout, int kvh, int hd, int hdi, int P) {
+    const int64_t per_tok = (int64_t)kvh * (hd / 8);
+    // Whole runs from 4096 waves of single tokens (2048 tokens of 8 kv heads
+    // x 128 dims): fewer leave a few waves with 8 tokens' round trips each
+    // (256 tokens 8 us against 4; 5 600 tokens 14 against 27).
+    const int mode = (int64_t)n_runs * most * per_tok >= 4096 * 64 ? kAppRun
+                     : most == 1 && layout == kLayoutSHD           ? kAppFlat
+                                                                   : kAppTok;
+    const int per = mode == kAppTok ? most : 1;
+    int64_t work = (int64_t)n_runs * per * per_tok;
     if (work < n_patch) work = n_patch;
     if (work <= 0) return hipSuccess;
+    const int tok_row = layout == kLayoutSHD ? kvh : 1;
     // One-wave work-groups: a decode step's append (a few thousand threads,
     // each one load and a few stores) then spreads over as many CUs as it has
     // waves instead of sitting on a handful.
     const unsigned grid = (unsigned)((work + 63) / 64);
-    if (plan)
-        kv_append_kernel<true><<<grid, 64, 0, s>>>(*plan, kpool, vpool, table, patches, n_patch,
-                                                   toks, tok_off, n_tok, k_src, v_src, src_bf16,
-                                                   layout, kvh, hd, hdi, P);
-    else
-        kv_append_kernel<false><<<grid, 64, 0, s>>>(NoPlan{0}, kpool, vpool, table, patches,
-                                                    n_patch, toks, tok_off, n_tok, k_src, v_src,
-                                                    src_bf16, layout, kvh, hd, hdi, P);
+#define RLX_KV_APPEND(ARGV, MODEV, PLANV)                                                                    \
+    kv_append_kernel<ARGV, MODEV><<<grid, 64, 0, s>>>(PLANV, kpool, vpool, table, patches, n_patch, runs,    \
+                                                      run_off, n_runs, per, k_src, v_src, src_bf16, tok_row, \
+                                                      kvh, hd, hdi, P)
+#define RLX_KV_APPEND_MODE(ARGV, PLANV)          \
+    if (mode == kAppRun)                         \
+        RLX_KV_APPEND(ARGV, kAppRun, PLANV);     \
+    else if (mode == kAppFlat)                   \
+        RLX_KV_APPEND(ARGV, kAppFlat, PLANV);    \
+    else                                         \
+        RLX_KV_APPEND(ARGV, kAppTok, PLANV);
+    if (plan) {
+        RLX_KV_APPEND_MODE(true, *plan)
+    } else {
+        RLX_KV_APPEND_MODE(false, NoPlan{0})
+    }
+#undef RLX_KV_APPEND_MODE
+#undef RLX_KV_APPEND
     return hipGetLastError();
 }
 

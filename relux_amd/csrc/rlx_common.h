@@ -101,6 +101,16 @@ struct AppendTok {
     int32_t seq_n;
 };
 
+// Up to 8 consecutive tokens of a sequence in one 8-slot group of a page (GQA
+// append): their page, first slot and count, and where their rows sit in the
+// caller's source buffer, in rows of one kv head.
+struct AppendRun {
+    int32_t page;
+    int32_t slot;      // of the first token
+    uint32_t row;      // row of the first token's kv head 0
+    uint32_t head_n;   // rows from one kv head to the next (< 2^29) | (count - 1) << 29
+};
+
 // One sequence of an attention / gather call.
 struct AttRow {
     int32_t tab;     // flat index of the sequence's first live table entry
@@ -178,6 +188,16 @@ __device__ __forceinline__ AppendTok plan_tok(const AppendTok *toks, int tok_off
         return AppendTok{p[0], p[1], p[2], p[3]};
     } else {
         return toks[i];
+    }
+}
+template <bool ARG>
+__device__ __forceinline__ AppendRun plan_run(const AppendRun *runs, int off, int i) {
+    if constexpr (ARG) {
+        const __attribute__((address_space(4))) int32_t *p =
+            (const __attribute__((address_space(4))) int32_t *)(kernarg_plan() + off + i * sizeof(AppendRun));
+        return AppendRun{p[0], p[1], (uint32_t)p[2], (uint32_t)p[3]};
+    } else {
+        return runs[i];
     }
 }
 // ---- append bodies shared by the append kernels and fused launches -------
@@ -421,12 +441,12 @@ hipError_t launch_fill_i32(hipStream_t s, int32_t *dst, int32_t val, int64_t n);
 // pointer arrays are device-readable.
 hipError_t launch_page_copy(hipStream_t s, const uint64_t *src, const uint64_t *dst, int n, int64_t bytes);
 
-// plan: patches and tokens in the kernel arguments (tokens at byte tok_off);
-// nullptr: patches / toks are device arrays.
-hipError_t launch_kv_append(hipStream_t s, const PlanArg *plan, int tok_off, uint16_t *kpool,
+// plan: patches and runs (launch_mla_append: tokens) in the kernel arguments
+// (at byte run_off / tok_off); nullptr: device arrays.  most: the longest run.
+hipError_t launch_kv_append(hipStream_t s, const PlanArg *plan, int run_off, uint16_t *kpool,
                             uint16_t *vpool, int32_t *table,
-                            const Patch *patches, int n_patch, const AppendTok *toks, int n_tok,
-                            const void *k_src, const void *v_src, int src_bf16, int layout,
+                            const Patch *patches, int n_patch, const AppendRun *runs, int n_runs,
+                            int most, const void *k_src, const void *v_src, int src_bf16, int layout,
                             int kvh, int hd, int hdi, int P);
 hipError_t launch_mla_append(hipStream_t s, const PlanArg *plan, int tok_off, uint16_t *pool,
                              int32_t *table, const Patch *patches,

@@ -197,30 +197,31 @@ bool capturing(Cache *c) {
     return st != hipStreamCaptureStatusNone;
 }
 
-// Append plans: patches then tokens (16-byte aligned), in the kernel
+// Append plans: patches then tokens (or runs; 16-byte aligned), in the kernel
 // arguments when they fit, else staged.  Fills *plan or the device pointers.
-int32_t append_plan(Cache *c, const std::vector<Patch> &patches,
-                    const std::vector<AppendTok> &toks, PlanArg *plan_arg, const PlanArg **plan,
-                    int *tok_off, const Patch **d_patches, const AppendTok **d_toks) {
+template <class T>
+int32_t append_plan(Cache *c, const std::vector<Patch> &patches, const std::vector<T> &toks,
+                    PlanArg *plan_arg, const PlanArg **plan, int *tok_off, const Patch **d_patches,
+                    const T **d_toks) {
     const size_t off = (patches.size() * sizeof(Patch) + 15) & ~(size_t)15;
     *plan = nullptr;
     *d_patches = nullptr;
     *d_toks = nullptr;
     *tok_off = (int)off;
-    if (off + toks.size() * sizeof(AppendTok) <= sizeof(PlanArg)) {
+    if (off + toks.size() * sizeof(T) <= sizeof(PlanArg)) {
         if (!patches.empty()) memcpy(plan_arg->b, patches.data(), patches.size() * sizeof(Patch));
-        if (!toks.empty()) memcpy(plan_arg->b + off, toks.data(), toks.size() * sizeof(AppendTok));
+        if (!toks.empty()) memcpy(plan_arg->b + off, toks.data(), toks.size() * sizeof(T));
         *plan = plan_arg;
         return RLX_OK;
     }
-    std::vector<char> bytes(off + toks.size() * sizeof(AppendTok));
+    std::vector<char> bytes(off + toks.size() * sizeof(T));
     if (!patches.empty()) memcpy(bytes.data(), patches.data(), patches.size() * sizeof(Patch));
-    if (!toks.empty()) memcpy(bytes.data() + off, toks.data(), toks.size() * sizeof(AppendTok));
+    if (!toks.empty()) memcpy(bytes.data() + off, toks.data(), toks.size() * sizeof(T));
     void *dev;
     int32_t rc = stage(c, bytes.data(), bytes.size(), &dev);
     if (rc) return rc;
     *d_patches = (const Patch *)dev;
-    *d_toks = (const AppendTok *)((char *)dev + off);
+    *d_toks = (const T *)((char *)dev + off);
     return RLX_OK;
 }
 
@@ -487,6 +488,26 @@ int32_t plan_append(Cache *c, int layer, int n_seqs, const int32_t *seq_ids, con
         row0 += n_tok[i];
     }
     return RLX_OK;
+}
+
+// The tokens of a GQA append as runs of consecutive tokens within an 8-slot
+// group of a page: a prompt's plan is 1/8 the size of its token list, and a
+// verify step's fits the kernel arguments.  most: the longest.
+std::vector<AppendRun> append_runs(const Cache *c, const std::vector<AppendTok> &toks, int layout, int &most) {
+    std::vector<AppendRun> runs;
+    most = 1;
+    runs.reserve(toks.size());
+    for (size_t t = 0; t < toks.size();) {
+        const AppendTok &k = toks[t];
+        const size_t end = std::min((size_t)k.seq_row0 + k.seq_n, t + 8 - k.slot % 8);
+        const uint32_t row0 = (uint32_t)k.seq_row0;
+        const uint32_t row = layout == RLX_LAYOUT_SHD ? (uint32_t)t * c->kvh : row0 * c->kvh + (uint32_t)t - row0;
+        const uint32_t head = layout == RLX_LAYOUT_SHD ? 1u : (uint32_t)k.seq_n;
+        most = std::max(most, (int)(end - t));
+        runs.push_back(AppendRun{k.page, k.slot, row, head | (uint32_t)(end - t - 1) << 29});
+        t = end;
+    }
+    return runs;
 }
 
 // Context splits of the MLA decode, per row: nsplit_r = ceil(len_r /
@@ -1050,16 +1071,18 @@ static int32_t kv_append_impl(Cache *c, int32_t layer, int32_t n_seqs, const int
         v_src = pad[1];
     }
     std::vector<Patch> patches = take_pending(c);
+    int most;
+    const std::vector<AppendRun> runs = append_runs(c, toks, src_layout, most);
     PlanArg plan_arg;
     const PlanArg *plan;
-    int tok_off;
+    int run_off;
     const Patch *d_patches;
-    const AppendTok *d_toks;
-    if ((rc = append_plan(c, patches, toks, &plan_arg, &plan, &tok_off, &d_patches, &d_toks)))
+    const AppendRun *d_runs;
+    if ((rc = append_plan(c, patches, runs, &plan_arg, &plan, &run_off, &d_patches, &d_runs)))
         return rc;
     LayerState &ls = c->L[layer];
-    HIP_TRY(launch_kv_append(c->stream, plan, tok_off, ls.pool0, ls.pool1, c->d_table, d_patches,
-                             (int)patches.size(), d_toks, (int)toks.size(), k_src, v_src,
+    HIP_TRY(launch_kv_append(c->stream, plan, run_off, ls.pool0, ls.pool1, c->d_table, d_patches,
+                             (int)patches.size(), d_runs, (int)runs.size(), most, k_src, v_src,
                              src_dtype == RLX_BF16, src_layout, c->kvh, c->hd, c->hdi, c->P));
     return RLX_OK;
 }
