@@ -608,7 +608,16 @@ struct PrefillArgs {
     const uint16_t *kr;     // dense: rope keys [Tp][64] per sequence, sequence s at row part
     const int32_t *table;
     const AttRow *rows;     // dense: part = token offset of the sequence, nsplit = Tp
-    const int4 *work;       // (row, head group, query tile, unused)
+    const int4 *work;       // (row, head group, query tile, part slot or -1: the whole tile)
+    // Tiles cut along the keys (n_merge > 0): part slot p attends key blocks
+    // [ranges[p].x, ranges[p].y) and leaves its unnormalised sums at part_o
+    // [p][256][dims of the launch] and its rows' (max, sum) at part_ml
+    // [p][256]; merge lists the cut tiles as (row, head group, query tile |
+    // parts << 20, first slot).
+    const int2 *ranges;
+    float *part_o, *part_ml;
+    const int4 *merge;
+    int n_merge;
     const void *q;          // paged: [rows][H][qd]; dense: q_nope [rows][H][qd]
     const void *q2;         // dense: q_rope [rows][H][qd2]
     void *out;
@@ -625,6 +634,8 @@ struct PrefillArgs {
     int dv0;     // first V dim of this launch (head dims of 256 run as two 128-dim launches)
 };
 
+// Scratch of one part slot: 256 rows of (at most) 128 value dims, and (max, sum).
+constexpr size_t kPrefillPartO = (size_t)kPrefillRows * 128 * 4, kPrefillPartMl = (size_t)kPrefillRows * 8;
 hipError_t launch_prefill(hipStream_t s, int src, int hd, const PrefillArgs &a, int n_work,
                           hipEvent_t ev0, hipEvent_t ev1);
 // W_UK / W_UV [d_c][H*D] transposed to wt [H*DP][512] (once per call): head

@@ -81,10 +81,10 @@ __device__ __forceinline__ int pf_swz(int r) { return (r >> 1) & 7; }
 template <int DQK, int DV, int SRC>
 struct PfShape {
     static constexpr int KS = DQK / 16;                              // score k-steps
-    static constexpr int NKR = DQK / 64;                             // K regions
+    static constexpr int NKR = (DQK + 63) / 64;                      // K regions (the last may be half used)
     static constexpr int DP = SRC == kSrcDense ? DQK - 64 : DQK;     // dense: K_c row pitch
-    static constexpr int ST = NKR * 512 + DV * 8;                    // chunks per stage
-    static constexpr int LV = DV / 64;                               // V^T loads per wave
+    static constexpr int LV = (DV + 63) / 64;                        // V^T loads per wave
+    static constexpr int ST = NKR * 512 + LV * 512;                  // chunks per stage
     static constexpr int LPW = NKR + LV;                             // ring loads per wave
     static constexpr int S = ST * 16 * 4 <= 131072 ? 4 : ST * 16 * 3 <= 163840 ? 3 : 2;  // blocks in flight + 1
     // Staggered waves (waves 4-7 run their P.V of block j - 1 in iteration
@@ -95,7 +95,7 @@ struct PfShape {
     static constexpr bool STAG = SRC == kSrcDense && ST * 16 * (S + 1) <= 163840;
     static constexpr int SR = S + (STAG ? 1 : 0);                    // ring stages
     static constexpr int MD = DV / 32;                               // output dim tiles
-    static_assert(DQK % 64 == 0 && DV % 64 == 0, "whole 64-dim regions");
+    static_assert(DQK % 32 == 0 && DV % 32 == 0 && (SRC == kSrcPaged || DQK % 64 == 0), "whole 32-dim tiles");
     static_assert(SRC == kSrcPaged || DV == 128, "dense: 128 value dims per launch");
 };
 
@@ -124,9 +124,17 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
         kend = min(R.len, pf_limit(a.mask_mode, R.len, R.nq, jmax) + 1);
         if (a.mask_mode == kMaskRef && R.nq != R.len) kend = R.len;
     }
-    const int nblk = (kend + kKeyBlock - 1) / kKeyBlock;
+    // Key blocks [jb, je): all of the tile's, or its part's.
+    int jb = 0, je = (kend + kKeyBlock - 1) / kKeyBlock;
+    if (wk.w >= 0) {
+        const int2 r = a.ranges[wk.w];
+        jb = r.x;
+        je = r.y;
+    }
 
     // ---- per-lane ring load offsets (fixed for every block) ----------------
+    // (A half used region's chunks past the row, and V^T rows past DV, repeat
+    // the last ones: loaded, never multiplied.)
     // K regions: this wave's rows kr = 8 wave + lane / 8 (16-key group
     // wave / 2), logical chunk klc (dims 64 q + 8 klc of region q).
     const int kr = 8 * wave + (lane >> 3);
@@ -135,7 +143,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
 #pragma unroll
     for (int q = 0; q < NKR; q++) {
         if (SRC == kSrcPaged)
-            ko[q] = (uint32_t)k_page_off(kr & 15, 64 * q + klc * 8, DQK) * 2;
+            ko[q] = (uint32_t)k_page_off(kr & 15, min(64 * q + klc * 8, DQK - 8), DQK) * 2;
         else if (q < NKR - 1)
             ko[q] = (uint32_t)(kr * DP + 64 * q + klc * 8) * 2;
         else
@@ -147,8 +155,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
 #pragma unroll
     for (int i = 0; i < LV; i++) {
         const int p = (8 * i + wave) * 64 + lane;
-        vd[i] = p >> 3;
-        vlc[i] = (p & 7) ^ pf_swz(vd[i]);
+        vlc[i] = (p & 7) ^ pf_swz(p >> 3);
+        vd[i] = min(p >> 3, DV - 1);
         ov[i] = (SRC == kSrcDense) ? (uint32_t)((int64_t)(a.dv0 + vd[i]) * R.nsplit + vlc[i] * 8) * 2 : 0u;
     }
     auto pdiv = [&](int t) { return POW2 ? t >> a.pshift : t / a.P; };
@@ -162,6 +170,11 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
     // Blocks are issued in order, one per call: running K_c / V^T / rope-key
     // pointers and stage offset of the next block to issue.
     const uint16_t *kc_next = kc_seq, *vt_next = vt_seq, *kr_next = kr_seq;
+    if (SRC == kSrcDense) {
+        kc_next += (int64_t)jb * kKeyBlock * DP;
+        vt_next += (int64_t)jb * kKeyBlock;
+        kr_next += (int64_t)jb * kKeyBlock * kMlaDr;
+    }
     uint32_t st_next = 0;
     constexpr uint32_t kStageBytes = SH::ST * 16;
 
@@ -233,7 +246,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
             for (int q = 0; q < NKR; q++) {
                 const uint16_t *gp;
                 if (SRC == kSrcPaged)
-                    gp = a.kpool + ((int64_t)pgt * a.KVH + hg) * a.P * DQK + k_page_off(pmod(t), 64 * q + klc * 8, DQK);
+                    gp = a.kpool + ((int64_t)pgt * a.KVH + hg) * a.P * DQK +
+                         k_page_off(pmod(t), min(64 * q + klc * 8, DQK - 8), DQK);
                 else if (q < NKR - 1)
                     gp = kc_seq + (int64_t)t * DP + 64 * q + klc * 8;
                 else
@@ -260,9 +274,9 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
     // Wait until this wave's loads of block j landed: S - 2 blocks were
     // issued after it in the steady state, fewer at the end.
     auto wait_block = [&](int j) {
-        if (j + S - 2 < nblk) {
+        if (j + S - 2 < je) {
             RLX_WAIT_VM((S - 2) * LPW);
-        } else if (S >= 4 && j + 1 < nblk) {
+        } else if (S >= 4 && j + 1 < je) {
             RLX_WAIT_VM(LPW);
         } else {
             RLX_WAIT_VM(0);
@@ -270,7 +284,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
     };
     static_assert(S <= 4, "wait_block covers at most two blocks ahead");
 
-    for (int j = 0; j < S - 1 && j < nblk; j++) issue_block(j);
+    for (int j = jb; j < jb + S - 1 && j < je; j++) issue_block(j);
 
     // ---- query operand (B of S^T) and key limit of the lane's row ----------
     const int qrow_t = wave * 32 + l32;
@@ -337,6 +351,10 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
 #pragma unroll
     for (int off = 32; off >= 1; off >>= 1) kmin = min(kmin, __shfl_xor(kmin, off));
     kmin = __builtin_amdgcn_readfirstlane(kmin);
+    // A wave with no query row (a verify's few rows, the end of a prompt)
+    // only loads its share of the ring and passes the barriers.  (The widest
+    // shapes have no registers left for that loop: they multiply zeros.)
+    const bool idle = DQK < 256 && kmin == 0x7fffffff;
 #pragma unroll
     for (int ks = 0; ks < KS; ks++) asm volatile("" ::"v"(qb[ks]));
 
@@ -395,6 +413,17 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
         __builtin_amdgcn_sched_barrier(0);
     };
 
+    // V^T entries of the sequence's last block past its live length.
+    auto zero_tail = [&](int k0, int st_read) {
+        uint16_t *Vw = ring + st_read + NKR * 4096;
+        const int live = R.len - k0;
+        for (int e = tid; e < DV * kKeyBlock; e += 64 * kWaves) {
+            const int d = e / kKeyBlock, kk = e - d * kKeyBlock;
+            if (kk >= live) Vw[d * kKeyBlock + (((kk >> 3) ^ pf_swz(d)) << 3) + (kk & 7)] = 0;
+        }
+        ring_barrier();
+    };
+
     // Staggered schedule: waves w and w + 4 share a SIMD.  Waves 0-3 run
     // block j's scores, softmax and P.V in iteration j; waves 4-7 first run
     // the P.V of block j - 1 (its weights kept in registers), then block j's
@@ -408,22 +437,14 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
     auto run = [&](auto lagc) {
     constexpr bool lag = decltype(lagc)::value;
     int st_prev = 0;
-    for (int j = 0, st_read = 0; j < nblk;
+    for (int j = jb, st_read = 0; j < je;
          j++, st_prev = st_read, st_read = (st_read + SH::ST * 8 == SR * SH::ST * 8) ? 0 : st_read + SH::ST * 8) {
         wait_block(j);
         ring_barrier();
-        if (SRC == kSrcPaged && j + S - 1 < nblk) issue_block(j + S - 1);
+        if (SRC == kSrcPaged && j + S - 1 < je) issue_block(j + S - 1);
         const int k0 = j * kKeyBlock;
         const uint16_t *st = ring + st_read;
-        if (k0 + kKeyBlock > R.len) {
-            uint16_t *Vw = ring + st_read + NKR * 4096;
-            const int live = R.len - k0;
-            for (int e = tid; e < DV * kKeyBlock; e += 64 * kWaves) {
-                const int d = e / kKeyBlock, kk = e - d * kKeyBlock;
-                if (kk >= live) Vw[d * kKeyBlock + (((kk >> 3) ^ pf_swz(d)) << 3) + (kk & 7)] = 0;
-            }
-            ring_barrier();
-        }
+        if (k0 + kKeyBlock > R.len) zero_tail(k0, st_read);
         // Weights of key tile 0 are computed with the current running max
         // while tile 1's score products execute, and those of tile 1 while
         // tile 0's P.V products execute.  A tile is redone after a rescale to
@@ -444,7 +465,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
         // The lagging waves' P.V of the previous block (its stage stays
         // resident through this iteration).
         if constexpr (lag)
-            if (j > 0) pv_plain(ring + st_prev);
+            if (j > jb) pv_plain(ring + st_prev);
         fl16 sc[2];
         float lt[2] = {0.f, 0.f};
         // With FOLD, sc holds s - m_use (m_use = the running max, 0 before a
@@ -546,7 +567,7 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
         // load stalled by memory back-pressure does not hold up this block's
         // score reads (config 4: -0.5 %).  (The paged source issues right
         // after the barrier: its block loads wait on page-table reads.)
-        if (SRC == kSrcDense && j + S - 1 < nblk) issue_block(j + S - 1);
+        if (SRC == kSrcDense && j + S - 1 < je) issue_block(j + S - 1);
         if (need_mask) mask(1);
         fixup(0);
         if constexpr (lag) {
@@ -585,12 +606,21 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
     }
 
     if constexpr (lag)
-        if (nblk > 0) pv_plain(ring + st_prev);  // the last block's P.V
+        if (je > jb) pv_plain(ring + st_prev);  // the last block's P.V
     };
-    if (STAG && wave >= kWaves / 2)
+    if (idle) {
+        for (int j = jb, st_read = 0; j < je;
+             j++, st_read = (st_read + SH::ST * 8 == SR * SH::ST * 8) ? 0 : st_read + SH::ST * 8) {
+            wait_block(j);
+            ring_barrier();
+            if (j + S - 1 < je) issue_block(j + S - 1);
+            if ((j + 1) * kKeyBlock > R.len) zero_tail(j * kKeyBlock, st_read);
+        }
+    } else if (STAG && wave >= kWaves / 2) {
         run(std::true_type{});
-    else
+    } else {
         run(std::false_type{});
+    }
 
     // ---- normalise and write ----------------------------------------------
     {
@@ -598,6 +628,17 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
         l_part = __uint_as_float(sw[0]) + __uint_as_float(sw[1]);
     }
     if (!rvalid) return;
+    if (wk.w >= 0) {  // a part: unnormalised, merged by prefill_merge_kernel
+        const int64_t pr = (int64_t)wk.w * kTileRows + qrow_t;
+        if (hh == 0) *(float2 *)(a.part_ml + pr * 2) = make_float2(m_run, l_part);
+#pragma unroll
+        for (int md = 0; md < MD; md++)
+#pragma unroll
+            for (int g4 = 0; g4 < 4; g4++)
+                *(fl4 *)(a.part_o + pr * DV + md * 32 + 8 * g4 + 4 * hh) =
+                    fl4{acc[md][4 * g4], acc[md][4 * g4 + 1], acc[md][4 * g4 + 2], acc[md][4 * g4 + 3]};
+        return;
+    }
     const float inv = (l_part > 0.f) ? 1.f / l_part : 0.f;
     const int64_t obase = ((a.layout == kLayoutSHD || SRC == kSrcDense)
                                ? ((int64_t)(R.qrow + qj) * a.HQ + a.h0 + qh) * a.od
@@ -620,28 +661,75 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
         }
 }
 
+// The parts of a cut tile merged with log-sum-exp weights: DV / 4 lanes a
+// row, a float4 of every part each.
+template <int DV, int SRC>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(const PrefillArgs a) {
+    constexpr int LPR = DV / 4, RPB = 256 / LPR;
+    const int4 t = a.merge[blockIdx.x];
+    const AttRow R = a.rows[t.x];
+    const int G = (SRC == kSrcPaged) ? a.H / a.KVH : 1, toks = kTileRows / G;
+    if (threadIdx.x >= RPB * LPR) return;
+    const int row = blockIdx.y * RPB + threadIdx.x / LPR, d = threadIdx.x % LPR * 4;
+    const int qj = (t.z & 0xFFFFF) * toks + row / G, qh = t.y * G + row % G, np = t.z >> 20;
+    if (qj >= R.nq || row >= toks * G || a.dv0 + d >= a.od) return;
+    const float *ml = a.part_ml + ((int64_t)t.w * kTileRows + row) * 2;
+    const float *po = a.part_o + ((int64_t)t.w * kTileRows + row) * DV + d;
+    float M = -INFINITY;
+    for (int p = 0; p < np; p++) M = fmaxf(M, ml[(int64_t)p * kTileRows * 2]);
+    fl4 o = fl4{0.f, 0.f, 0.f, 0.f};
+    float L = 0.f;
+#pragma unroll 4
+    for (int p = 0; p < np; p++) {
+        const float2 v = *(const float2 *)(ml + (int64_t)p * kTileRows * 2);
+        // (a part whose keys are all masked for this row: m -inf, sums 0)
+        const float w = (v.x == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(v.x - M);
+        L += w * v.y;
+        o += *(const fl4 *)(po + (int64_t)p * kTileRows * DV) * w;
+    }
+    o *= (L > 0.f) ? 1.f / L : 0.f;
+    const int64_t off = ((a.layout == kLayoutSHD || SRC == kSrcDense)
+                             ? ((int64_t)(R.qrow + qj) * a.HQ + a.h0 + qh) * a.od
+                             : ((int64_t)R.qrow * a.HQ + (int64_t)(a.h0 + qh) * R.nq + qj) * a.od) + a.dv0 + d;
+    if (a.out_bf16) {
+        u32x2 w;
+        w[0] = (uint32_t)bf16_rne(o[0]) | ((uint32_t)bf16_rne(o[1]) << 16);
+        w[1] = (uint32_t)bf16_rne(o[2]) | ((uint32_t)bf16_rne(o[3]) << 16);
+        *(u32x2 *)((uint16_t *)a.out + off) = w;
+    } else {
+        *(fl4 *)((float *)a.out + off) = o;
+    }
+}
+
+template <int DQK, int DV, int SRC>
+hipError_t launch_prefill_shape(hipStream_t s, const PrefillArgs &a, int n_work, hipEvent_t e0, hipEvent_t e1) {
+    constexpr int kRpb = 256 / (DV / 4);  // rows per merge work-group
+    const dim3 g(n_work), b(64 * kWaves);
+    hipError_t e = a.pshift >= 0
+                       ? launch_timed(prefill_kernel<DQK, DV, SRC, true>, g, b, s, e0, e1, a, a.table)
+                       : launch_timed(prefill_kernel<DQK, DV, SRC, false>, g, b, s, e0, e1, a, a.table);
+    if (e != hipSuccess || a.n_merge <= 0) return e;
+    prefill_merge_kernel<DV, SRC><<<dim3(a.n_merge, (kTileRows + kRpb - 1) / kRpb), 256, 0, s>>>(a);
+    return hipGetLastError();
+}
+
 hipError_t launch_prefill(hipStream_t s, int src, int hd, const PrefillArgs &a, int n_work,
                           hipEvent_t ev0, hipEvent_t ev1) {
     if (n_work <= 0) return hipSuccess;
-    const dim3 g(n_work), b(64 * kWaves);
-    const bool p2 = a.pshift >= 0;
-#define RLX_PF(DQK, DV, SRC, A, E0, E1)                                                              \
-    (p2 ? launch_timed(prefill_kernel<DQK, DV, SRC, true>, g, b, s, E0, E1, A, A.table)            \
-        : launch_timed(prefill_kernel<DQK, DV, SRC, false>, g, b, s, E0, E1, A, A.table))
-    if (src == kSrcPaged && hd == 128) return RLX_PF(128, 128, kSrcPaged, a, ev0, ev1);
-    if (src == kSrcPaged && hd == 64) return RLX_PF(64, 64, kSrcPaged, a, ev0, ev1);
-    if (src == kSrcDense && hd == 128) return RLX_PF(192, 128, kSrcDense, a, ev0, ev1);
+    if (src == kSrcPaged && hd == 128) return launch_prefill_shape<128, 128, kSrcPaged>(s, a, n_work, ev0, ev1);
+    if (src == kSrcPaged && hd == 96) return launch_prefill_shape<96, 96, kSrcPaged>(s, a, n_work, ev0, ev1);
+    if (src == kSrcPaged && hd == 64) return launch_prefill_shape<64, 64, kSrcPaged>(s, a, n_work, ev0, ev1);
+    if (src == kSrcDense && hd == 128) return launch_prefill_shape<192, 128, kSrcDense>(s, a, n_work, ev0, ev1);
     if (hd == 256) {  // two launches, one per 128 value dims (the scores are computed in each)
         PrefillArgs a0 = a, a1 = a;
         a0.dv0 = 0;
         a1.dv0 = 128;
-        hipError_t e = src == kSrcPaged ? RLX_PF(256, 128, kSrcPaged, a0, ev0, nullptr)
-                                        : RLX_PF(320, 128, kSrcDense, a0, ev0, nullptr);
+        hipError_t e = src == kSrcPaged ? launch_prefill_shape<256, 128, kSrcPaged>(s, a0, n_work, ev0, nullptr)
+                                        : launch_prefill_shape<320, 128, kSrcDense>(s, a0, n_work, ev0, nullptr);
         if (e != hipSuccess) return e;
-        return src == kSrcPaged ? RLX_PF(256, 128, kSrcPaged, a1, nullptr, ev1)
-                                : RLX_PF(320, 128, kSrcDense, a1, nullptr, ev1);
+        return src == kSrcPaged ? launch_prefill_shape<256, 128, kSrcPaged>(s, a1, n_work, nullptr, ev1)
+                                : launch_prefill_shape<320, 128, kSrcDense>(s, a1, n_work, nullptr, ev1);
     }
-#undef RLX_PF
     return hipErrorInvalidValue;
 }
 

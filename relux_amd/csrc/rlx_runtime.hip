@@ -17,6 +17,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <fcntl.h>
 #include <sys/mman.h>
 #include <unistd.h>
@@ -585,6 +586,102 @@ int tile_keys(const AttRow &r, int mask_mode, int toks, int qt) {
     return r.len;
 }
 
+// Cuts of a prefill call's tiles along the keys.  A work-group (one per CU)
+// walks its tile's keys in blocks of 64, so a call with fewer tiles than CUs,
+// or a few long ones, leaves most of the chip waiting: B 1, 8 kv heads, 16 new
+// tokens on 8192 ran 8 work-groups of 128 blocks.  Tiles of more than `target`
+// blocks are cut into equal parts, merged by their (max, sum) afterwards;
+// the target is the one of a few whose estimate is least: the longest
+// work-group or the CUs' share of the work, kPfStart blocks of start-up per
+// work-group, the merge's launch and its traffic counted in (a block takes
+// about 2 us), if it saves a tenth.  Calls that fill the chip stay whole.
+// Measured (32 heads over 8, D 128, T 8192, us whole / cut): 16 new tokens 231 /
+// 39, 128 235 / 56, 512 251 / 112; T 0: 1024 60 / 55.
+constexpr double kPfStart = 2.5, kPfMerge = 1.5, kPfMergePart = 0.035;
+constexpr int kPfMaxParts = 480;  // 64 MB of partial sums
+struct PrefillSplit {
+    std::vector<int2> ranges;  // part slot -> key blocks
+    std::vector<int4> merge;   // PrefillArgs::merge
+};
+// groups: the tiles by (sequence, head group), `w` -1; blocks(tile): its key
+// blocks.  Cut groups are regrouped by part, so that parts of the same keys
+// stay together and single groups spread over the XCDs.
+// fill: the share of a tile's 256 rows that hold queries (what the merge moves).
+template <class F>
+PrefillSplit split_prefill(std::vector<std::vector<int4>> &groups, std::vector<double> &cost, int cus,
+                           double fill, F blocks) {
+    PrefillSplit sp;
+    int64_t total = 0, tiles = 0;
+    int most = 0;
+    for (auto &g : groups)
+        for (auto &t : g) {
+            const int b = blocks(t);
+            total += b;
+            tiles++;
+            most = std::max(most, b);
+        }
+    if (tiles == 0 || tiles >= 2 * (int64_t)cus) return sp;
+    auto estimate = [&](int64_t n, double longest) {
+        const double share = ((double)total + (double)n * kPfStart) / cus;
+        const double last = n > cus ? 0.5 * ((double)total / n + kPfStart) : 0.0;
+        return std::max(longest + kPfStart, share + last);
+    };
+    int target = 0;
+    double best = 0.9 * estimate(tiles, most);
+    const int base = (int)std::max<int64_t>(4, (total + cus - 1) / cus);
+    for (int k = 4; k <= 10; k += 1) {
+        const int t = base * k / 4;
+        if (t >= most) break;
+        int64_t n = 0, cut = 0;
+        double longest = 0.0;
+        for (auto &g : groups)
+            for (auto &w : g) {
+                const int b = blocks(w), m = (b + t - 1) / t;
+                n += std::max(m, 1);
+                if (m > 1) cut += m;
+                longest = std::max(longest, m > 1 ? std::ceil((double)b / m) : (double)b);
+            }
+        if (cut > kPfMaxParts) continue;
+        const double e = estimate(n, longest) + kPfMerge + kPfMergePart * fill * (double)cut;
+        if (e < best) {
+            best = e;
+            target = t;
+        }
+    }
+    if (target == 0) return sp;
+    std::vector<std::vector<int4>> out;
+    std::vector<double> oc;
+    for (auto &g : groups) {
+        std::vector<std::vector<int4>> part;  // by part number
+        std::vector<double> pc;
+        for (auto &w : g) {
+            const int b = blocks(w), m = std::max(1, (b + target - 1) / target);
+            if ((int)part.size() < m) {
+                part.resize(m);
+                pc.resize(m, 0.0);
+            }
+            if (m > 1) sp.merge.push_back(int4{w.x, w.y, w.z | m << 20, (int)sp.ranges.size()});
+            for (int k = 0; k < m; k++) {
+                const int lo = (int)((int64_t)b * k / m), hi = (int)((int64_t)b * (k + 1) / m);
+                int4 item = w;
+                if (m > 1) {
+                    item.w = (int)sp.ranges.size();
+                    sp.ranges.push_back(int2{lo, hi});
+                }
+                part[k].push_back(item);
+                pc[k] += hi - lo;
+            }
+        }
+        for (size_t k = 0; k < part.size(); k++) {
+            out.push_back(std::move(part[k]));
+            oc.push_back(pc[k]);
+        }
+    }
+    groups = std::move(out);
+    cost = std::move(oc);
+    return sp;
+}
+
 // One AttRow per sequence, or -- with qtile > 0 (GQA decode kernel only) --
 // one per tile of at most qtile queries, each with its own context splits.
 // Cuts of the GQA decode ranges, in units of 64 padded positions: cut i is
@@ -709,6 +806,26 @@ int gqa_decode_split(const Cache *c, AttRow *rows, int n_rows, int *pre, int *cu
     }
     *total64_out = total64;
     return n_ranges;
+}
+
+// split_prefill for a call whose own scratch is `head` bytes of the workspace,
+// the partial sums behind it.  A workspace that cannot grow to them (a cap, or
+// a stream under capture) keeps the tiles whole.
+PrefillSplit prefill_parts(Cache *c, std::vector<std::vector<int4>> &groups, std::vector<double> &cost,
+                           const std::vector<AttRow> &rows, int mask_mode, int toks, size_t head) {
+    auto g = groups;
+    auto k = cost;
+    int nq = 0;
+    for (const AttRow &r : rows) nq = std::max(nq, r.nq);
+    const double fill = std::min(1.0, (double)nq / toks);
+    PrefillSplit sp = split_prefill(g, k, c->cus, fill, [&](const int4 &w) {
+        return (tile_keys(rows[w.x], mask_mode, toks, w.z) + 63) / 64;
+    });
+    const size_t need = head + sp.ranges.size() * (kPrefillPartO + kPrefillPartMl);
+    if (sp.ranges.empty() || (need > c->ws_cap && (capturing(c) || ensure_ws(c, need) != RLX_OK))) return {};
+    groups = std::move(g);
+    cost = std::move(k);
+    return sp;
 }
 
 // One AttRow per sequence of an attention call, with nsplit[i] context
@@ -1513,9 +1630,12 @@ int32_t check_gqa_attend(Cache *c, int32_t layer, int32_t n_seqs, const int32_t 
 // Whether GQA calls with more query rows per kv head than the decode kernel
 // holds run as FA2 chunked prefill: stored head dims 64, 128 and 256 (any
 // caller head_dim they hold), any G = heads per kv head up to 256 (a tile
-// holds floor(256 / G) tokens); other shapes tile their queries through
-// the decode kernel.
+// holds floor(256 / G) tokens); head dim 96 with groups the decode kernel
+// takes too (1000 new tokens of 2 sequences on 2000, 32 heads over 8 of 80
+// dims: 468 us as query tiles, 116 in FA2).  Other shapes tile their queries
+// through the decode kernel.
 bool gqa_use_fa2(const Cache *c, int G) {
+    if (c->hd == 96) return G <= gqa_rows_cap(c);
     return (c->hd == 64 || c->hd == 128 || c->hd == 256) && G <= kPrefillRows;
 }
 
@@ -1567,8 +1687,10 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
     const int max_qr = G * max_nq;
     // Query rows past cap (the decode kernel's per kv head) take FA2 or query
     // tiles (gqa_use_fa2).
-    const bool fa2 = gqa_use_fa2(c, G);
+    // (Head dim 96 under capture: query tiles, whose plan travels in the kernel
+    // arguments where it fits.)
     const int cap = gqa_rows_cap(c);
+    const bool fa2 = gqa_use_fa2(c, G) && !(c->hd == 96 && max_qr > cap && capturing(c));
     if (max_qr > cap && !fa2 && G > cap)
         return fail(RLX_ERR_UNSUPPORTED, "heads per kv head = %d with head_dim %d (at most %d)", G,
                     c->hdi, cap);
@@ -1588,15 +1710,16 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
                 groups.emplace_back();
                 cost.push_back(0.0);
                 for (int qt = tiles - 1; qt >= 0; qt--) {
-                    groups.back().push_back(int4{i, kvh, qt, 0});
+                    groups.back().push_back(int4{i, kvh, qt, -1});
                     cost.back() += tile_keys(rows[i], mask_mode, toks, qt);
                 }
             }
         }
+        const PrefillSplit sp = prefill_parts(c, groups, cost, rows, mask_mode, toks, 0);
         const std::vector<int4> work = xcd_order(groups, cost);
         if ((rc = flush_patches(c))) return rc;
         Blob b;
-        size_t o_r = b.add(rows), o_w = b.add(work);
+        size_t o_r = b.add(rows), o_w = b.add(work), o_g = b.add(sp.ranges), o_m = b.add(sp.merge);
         void *dev;
         if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
         if (scale <= 0.f) scale = (float)(1.0 / std::sqrt((double)c->hdu));
@@ -1606,6 +1729,11 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
         a.table = c->d_table;
         a.rows = (const AttRow *)((char *)dev + o_r);
         a.work = (const int4 *)((char *)dev + o_w);
+        a.ranges = (const int2 *)((char *)dev + o_g);
+        a.merge = (const int4 *)((char *)dev + o_m);
+        a.n_merge = (int)sp.merge.size();
+        a.part_o = (float *)c->ws;
+        a.part_ml = (float *)((char *)c->ws + sp.ranges.size() * kPrefillPartO);
         a.q = q;
         a.out = out;
         a.q_bf16 = q_dtype == RLX_BF16;
@@ -1891,7 +2019,8 @@ int32_t rlx_gqa_attend_noalloc(void *h, int32_t layer, int32_t n_seqs, const int
     for (int i = 0; i < n_seqs; i++) max_nq = std::max(max_nq, n_q ? n_q[i] : 1);
     const int max_qr = G * max_nq;
     // Decode and verify calls only: the FA2 path's work lists are staged.
-    const bool fa2 = gqa_use_fa2(c, G);
+    // (Head dim 96: query tiles, as every head dim without FA2.)
+    const bool fa2 = gqa_use_fa2(c, G) && c->hd != 96;
     const int cap = gqa_rows_cap(c);
     if (max_qr > cap && (fa2 || G > cap))
         return fail(RLX_ERR_UNSUPPORTED,
@@ -1943,19 +2072,40 @@ int32_t rlx_gqa_attend_noalloc(void *h, int32_t layer, int32_t n_seqs, const int
 }
 
 // Whether an MLA call runs as FA2 chunked prefill (latents expanded per
-// call) rather than the absorbed decode kernel: past kMlaGroupRowsMax query
-// rows (heads x queries) per sequence.  Up to that the absorbed kernel runs
-// head groups of 32 rows, each re-reading the sequence's latent rows (1152 B
-// per token and group) -- far less than an expansion writes and reads back
-// (4 bytes x 128 dims x heads per token) at decode and verify sizes.
-// RLX_MLA_FA2_ROWS overrides the bound (tests run both paths on one shape;
-// read per call).
+// call) rather than the absorbed decode kernel, which takes groups of 32 query
+// rows (heads x queries), each re-reading the sequence's latent rows (1152 B
+// per token and group): never up to kMlaGroupRowsMax rows per sequence, where
+// an expansion (4 bytes x 128 dims x heads per token written and read back)
+// costs far more, and past them by an estimate of both, of n = the call's
+// rows, their pairs with keys, and heads x keys expanded (us, fitted at 16,
+// 32 and 128 heads, head_dim 128, 1 and 4 sequences; absorbed / FA2: 16 heads
+// on 8192 keys, 65 new tokens 87 / 133, 128 138 / 140, 256 277 / 152; 128
+// heads on 8192, 9 92 / 589, 32 268 / 587, 64 642 / 593; 4 x 1024 keys, 16
+// heads, 96 137 / 107).  Other head dims, whose merge is slower, keep the
+// bound alone.  RLX_MLA_FA2_ROWS overrides it (tests run both paths on one
+// shape; read per call).
+// len(i): the live tokens of sequence i the call attends.
 constexpr int kMlaGroupRowsMax = 1024;
-static bool mla_use_fa2(const Cache *c, int max_qr, int head_dim) {
-    (void)c;
+static bool mla_use_fa2(int n_seqs, const int32_t *n_q, int num_heads, int head_dim,
+                        const std::function<int64_t(int)> &len) {
+    int max_nq = 0;
+    double rows = 0.0, pairs = 0.0, keys = 0.0;
+    for (int i = 0; i < n_seqs; i++) {
+        const int nq = n_q ? n_q[i] : 1;
+        max_nq = std::max(max_nq, nq);
+        rows += (double)num_heads * nq;
+        pairs += (double)num_heads * nq * len(i);
+        keys += len(i);
+    }
+    if (head_dim > 256) return false;
+    const int64_t max_qr = (int64_t)num_heads * max_nq;
     const char *e = getenv("RLX_MLA_FA2_ROWS");
-    const int lim = (e && atoi(e) > 0) ? atoi(e) : kMlaGroupRowsMax;
-    return max_qr > lim && head_dim <= 256;
+    if (e && atoi(e) > 0) return max_qr > atoi(e);
+    if (max_qr <= kMlaGroupRowsMax) return false;
+    if (head_dim != 128) return true;
+    const double absorbed = 22.0 + 0.012 * rows + 6.5e-6 * pairs;
+    const double expanded = 62.0 + 5.2e-4 * num_heads * keys + 6e-7 * pairs;
+    return !(absorbed < 0.85 * expanded);
 }
 
 // Padded head dim of the expanded K_c / V^T rows of an MLA prefill.
@@ -1977,12 +2127,10 @@ static int mla_prefill_heads(int64_t tok_off, int num_heads, int dp) {
 static int32_t mla_prefill_check(Cache *c, int layer, int n_seqs, const int32_t *seq_ids,
                                  const int32_t *n_q, const int32_t *add_tok, int num_heads,
                                  int head_dim) {
-    int max_nq = 0;
-    for (int i = 0; i < n_seqs; i++) max_nq = std::max(max_nq, n_q ? n_q[i] : 1);
-    if (!mla_use_fa2(c, num_heads * max_nq, head_dim)) return RLX_OK;
+    auto len = [&](int i) { return (int64_t)c->L[layer].seqs[seq_ids[i]].len + (add_tok ? add_tok[i] : 0); };
+    if (!mla_use_fa2(n_seqs, n_q, num_heads, head_dim, len)) return RLX_OK;
     int64_t tok_off = 0;
-    for (int i = 0; i < n_seqs; i++)
-        tok_off += ((int64_t)c->L[layer].seqs[seq_ids[i]].len + (add_tok ? add_tok[i] : 0) + 127) / 128 * 128;
+    for (int i = 0; i < n_seqs; i++) tok_off += (len(i) + 127) / 128 * 128;
     const int dp = mla_prefill_dp(head_dim);
     if (tok_off > 0 && mla_prefill_heads(tok_off, num_heads, dp) < 1)
         return fail(RLX_ERR_UNSUPPORTED,
@@ -2021,7 +2169,7 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
     int max_nq = 0;
     for (int i = 0; i < n_seqs; i++) max_nq = std::max(max_nq, n_q ? n_q[i] : 1);
     const int max_qr = num_heads * max_nq;
-    if (mla_use_fa2(c, max_qr, head_dim)) {
+    if (mla_use_fa2(n_seqs, n_q, num_heads, head_dim, [&](int i) { return (int64_t)ls.seqs[seq_ids[i]].len; })) {
         if (app)
             HIP_TRY(launch_mla_append(c->stream, app->plan, app->tok_off, app->pool, app->table,
                                       app->patches, app->n_patch, app->toks, app->n_tok, app->c_src,
@@ -2047,7 +2195,7 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
                 pgroups.emplace_back();
                 pcost.push_back(0.0);
                 for (int qt = tiles - 1; qt >= 0; qt--) {
-                    pgroups.back().push_back(int4{i, h, qt, 0});
+                    pgroups.back().push_back(int4{i, h, qt, -1});
                     pcost.back() += tile_keys(rows[i], mask_mode, kPrefillRows, qt);
                 }
             }
@@ -2060,6 +2208,13 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
         const int hg = mla_prefill_heads(tok_off, num_heads, dp);
         if (hg < 1) return fail(RLX_ERR_UNSUPPORTED, "MLA prefill call too large");
         const int n_groups = (num_heads + hg - 1) / hg;
+        const size_t w_bytes = (size_t)num_heads * dp * kMlaDc * 2;
+        const size_t e_bytes = (size_t)tok_off * hg * dp * 2;
+        const size_t r_bytes = (size_t)tok_off * kMlaDr * 2;  // rope keys of the call
+        const size_t x_bytes = (2 * w_bytes + 2 * e_bytes + r_bytes + 255) & ~(size_t)255;
+        // (parts chosen over all heads: a head's attention is the same
+        // computation however the heads are grouped)
+        PrefillSplit sp = prefill_parts(c, pgroups, pcost, rows, mask_mode, kPrefillRows, x_bytes);
         // work items of the group of heads [0, hg) (the xcd order), reused by
         // every group with its heads counted from the group's first
         std::vector<std::vector<int4>> pg_grp;
@@ -2070,13 +2225,18 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
                 pc_grp.push_back(pcost[k]);
             }
         const std::vector<int4> pwork = xcd_order(pg_grp, pc_grp);
+        auto heads_below = [](const std::vector<int4> &v, int n) {
+            std::vector<int4> o;
+            for (const int4 &w : v)
+                if (w.y < n) o.push_back(w);
+            return o;
+        };
+        sp.merge = heads_below(sp.merge, hg);
         if ((rc = flush_patches(c))) return rc;
-        const size_t w_bytes = (size_t)num_heads * dp * kMlaDc * 2;
-        const size_t e_bytes = (size_t)tok_off * hg * dp * 2;
-        const size_t r_bytes = (size_t)tok_off * kMlaDr * 2;  // rope keys of the call
-        if ((rc = ensure_ws(c, 2 * w_bytes + 2 * e_bytes + r_bytes))) return rc;
+        if ((rc = ensure_ws(c, x_bytes))) return rc;
         Blob b;
-        size_t o_r = b.add(rows), o_d = b.add(dwork), o_p = b.add(pwork);
+        size_t o_r = b.add(rows), o_d = b.add(dwork), o_p = b.add(pwork), o_g = b.add(sp.ranges),
+               o_m = b.add(sp.merge);
         void *dev;
         if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
         char *ws = (char *)c->ws;
@@ -2104,6 +2264,11 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
             a.table = c->d_table;
             a.rows = drows;
             a.work = (const int4 *)((char *)dev + o_p);
+            a.ranges = (const int2 *)((char *)dev + o_g);
+            a.merge = (const int4 *)((char *)dev + o_m);
+            a.n_merge = (int)sp.merge.size();
+            a.part_o = (float *)(ws + x_bytes);
+            a.part_ml = (float *)(ws + x_bytes + sp.ranges.size() * kPrefillPartO);
             a.q = q_nope;
             a.q2 = q_rope;
             a.out = out;
@@ -2126,13 +2291,15 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
             // work items of heads >= nh (a last, smaller group) are dropped
             int n_work = (int)pwork.size();
             if (nh < hg) {
-                std::vector<int4> part_w;
-                for (const int4 &w : pwork)
-                    if (w.y < nh) part_w.push_back(w);
+                const std::vector<int4> w = heads_below(pwork, nh), m = heads_below(sp.merge, nh);
+                Blob lb;
+                const size_t l_w = lb.add(w), l_m = lb.add(m);
                 void *dw;
-                if ((rc = stage(c, part_w.data(), part_w.size() * sizeof(int4), &dw))) return rc;
-                a.work = (const int4 *)dw;
-                n_work = (int)part_w.size();
+                if ((rc = stage(c, lb.bytes.data(), lb.bytes.size(), &dw))) return rc;
+                a.work = (const int4 *)((char *)dw + l_w);
+                a.merge = (const int4 *)((char *)dw + l_m);
+                a.n_merge = (int)m.size();
+                n_work = (int)w.size();
             }
             HIP_TRY(launch_prefill(c->stream, kSrcDense, dp, a, n_work, g == 0 ? e0 : nullptr,
                                    g == n_groups - 1 ? e1 : nullptr));
