@@ -638,13 +638,13 @@ struct PrefillArgs {
 constexpr size_t kPrefillPartO = (size_t)kPrefillRows * 128 * 4, kPrefillPartMl = (size_t)kPrefillRows * 8;
 hipError_t launch_prefill(hipStream_t s, int src, int hd, const PrefillArgs &a, int n_work,
                           hipEvent_t ev0, hipEvent_t ev1);
-// W_UK / W_UV [d_c][H*D] transposed to wt [H*DP][512] (once per call): head
-// dims padded with zero rows to DP (128 or 256), channels with zero columns
-// to 512.
+// W_UK / W_UV [d_c][H*D] packed as W^T fragments of H*DP features x 512
+// channels (once per call): head dims padded with zeros to DP (128 or 256),
+// channels to 512.
 hipError_t launch_mla_wt(hipStream_t s, const uint16_t *w_uk, const uint16_t *w_uv, int H, int D,
                          int dc, int DP, uint16_t *wt_k, uint16_t *wt_v);
-// K_c [H][Tp][DP] / V^T [H][DP][Tp] of H heads from their transposed weights
-// (wt_k, wt_v: the heads' rows of the transposed matrices).
+// K_c [H][Tp][DP] / V^T [H][DP][Tp] of H heads from their packed weights
+// (wt_k, wt_v: the heads' fragments).
 hipError_t launch_mla_rope_gather(hipStream_t s, const uint16_t *pool, const int32_t *table,
                                   const AttRow *rows, const int2 *work, int n_work, int P,
                                   uint16_t *kr);

@@ -2079,9 +2079,9 @@ int32_t rlx_gqa_attend_noalloc(void *h, int32_t layer, int32_t n_seqs, const int
 // costs far more, and past them by an estimate of both, of n = the call's
 // rows, their pairs with keys, and heads x keys expanded (us, fitted at 16,
 // 32 and 128 heads, head_dim 128, 1 and 4 sequences; absorbed / FA2: 16 heads
-// on 8192 keys, 65 new tokens 87 / 133, 128 138 / 140, 256 277 / 152; 128
-// heads on 8192, 9 92 / 589, 32 268 / 587, 64 642 / 593; 4 x 1024 keys, 16
-// heads, 96 137 / 107).  Other head dims, whose merge is slower, keep the
+// on 8192 keys, 65 new tokens 87 / 116, 128 138 / 124, 256 277 / 136; 128
+// heads on 8192, 9 92 / 442, 32 268 / 436, 64 642 / 447; 4 x 1024 keys, 16
+// heads, 96 137 / 86).  Other head dims, whose merge is slower, keep the
 // bound alone.  RLX_MLA_FA2_ROWS overrides it (tests run both paths on one
 // shape; read per call).
 // len(i): the live tokens of sequence i the call attends.
@@ -2103,8 +2103,8 @@ static bool mla_use_fa2(int n_seqs, const int32_t *n_q, int num_heads, int head_
     if (e && atoi(e) > 0) return max_qr > atoi(e);
     if (max_qr <= kMlaGroupRowsMax) return false;
     if (head_dim != 128) return true;
-    const double absorbed = 22.0 + 0.012 * rows + 6.5e-6 * pairs;
-    const double expanded = 62.0 + 5.2e-4 * num_heads * keys + 6e-7 * pairs;
+    const double absorbed = 22.0 + 0.010 * rows + 5.5e-6 * pairs;
+    const double expanded = 53.0 + 3.7e-4 * num_heads * keys + 6e-7 * pairs;
     return !(absorbed < 0.85 * expanded);
 }
 
