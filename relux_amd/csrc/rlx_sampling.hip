@@ -1962,12 +1962,15 @@ __device__ __forceinline__ int mass_finish(const SampleArgs &a, int b, float min
 }
 
 // Sample, one work-group per row: phase two of the split path when the
-// chunk lists are there, else the whole row.
+// chunk lists are there, else the whole row.  MASS: the last phase of the
+// mass split, the whole row where that cannot serve it (a kernel of its own,
+// so that neither carries the other's code).
+template <bool MASS>
 __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs a) {
     __shared__ SampLds s;
     const int b = blockIdx.x;
     Src c;
-    if (a.nch > 0) {
+    if (!MASS && a.nch > 0) {
         const int64_t q = (int64_t)b * a.nch;
         uint32_t lb, ub;
         float t = a.temperature;
@@ -1980,7 +1983,7 @@ __global__ __launch_bounds__(kST) void sample_kernel(const SampleArgs a) {
             return;
         }
     }
-    if (a.uch > 0) {
+    if constexpr (MASS) {
         const int t = mass_finish(a, b, a.min_p, a.u[b], s);
         if (t >= 0) {
             if (threadIdx.x == 0) a.out[b] = t;
@@ -2307,7 +2310,10 @@ hipError_t launch_sample(hipStream_t st, const SampleArgs &args, int n_rows, hip
             sample_part_kernel<<<dim3(n, a.nch), dim3(kST), 0, st>>>(a);
             if ((e = hipGetLastError()) != hipSuccess) break;
         }
-        sample_kernel<<<dim3(n), dim3(kST), 0, st>>>(a);
+        if (a.uch > 0)
+            sample_kernel<true><<<dim3(n), dim3(kST), 0, st>>>(a);
+        else
+            sample_kernel<false><<<dim3(n), dim3(kST), 0, st>>>(a);
         e = hipGetLastError();
         a.logits += (int64_t)n * a.stride;
         a.u += n;
