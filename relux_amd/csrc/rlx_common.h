@@ -483,13 +483,15 @@ hipError_t launch_mla_gather(hipStream_t s, const uint16_t *pool, const int32_t 
                              uint16_t *kr_out, int dc, int dr, int P);
 
 // plan: the rows in the kernel arguments (nullptr: rows and work on the device).
+// single: every row lies in one range (nsplit 1) and out is not q's memory: with
+// a plan the decode kernel writes the outputs itself and no merge is launched.
 hipError_t launch_gqa_decode(hipStream_t s, const PlanArg *plan, const uint16_t *kpool,
                              const uint16_t *vpool, const int32_t *table, const AttRow *rows,
                              int n_rows, const int4 *ranges, int n_ranges, const void *q, int q_bf16,
                              int layout, int H, int KVH, int hd, int hdi, int P, int total64,
                              int snap64, int ranges_off, float qscale,
                              int mask_mode, int nqt, float *part_o, float *part_ml, void *out,
-                             int out_bf16, int max_qr, hipEvent_t ev0, hipEvent_t ev1);
+                             int out_bf16, int max_qr, bool single, hipEvent_t ev0, hipEvent_t ev1);
 
 // Sources of the prefill kernel: the paged GQA cache, or (MLA) per-sequence
 // decompressed K_c / V^T plus rope keys from the paged latent rows.

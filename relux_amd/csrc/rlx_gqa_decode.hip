@@ -37,19 +37,49 @@ __device__ __forceinline__ int key_limit(int mask_mode, int len, int nq, int qi)
     return len - 1;
 }
 
+// 4 consecutive output elements at element o (DQ is a multiple of 8: all in or
+// all out of a head row); one store when the caller's buffer is aligned for it.
+__device__ __forceinline__ void gqa_store4(void *out, int64_t o, const float (&v)[4], int out_bf16) {
+    const bool vec = (((uintptr_t)out) & (out_bf16 ? 7 : 15)) == 0;
+    if (out_bf16) {
+        uint16_t *dst = (uint16_t *)out + o;
+        if (vec) {
+            const uint32_t lo = bf16_rne(v[0]) | ((uint32_t)bf16_rne(v[1]) << 16);
+            const uint32_t hi = bf16_rne(v[2]) | ((uint32_t)bf16_rne(v[3]) << 16);
+            *(uint2 *)dst = make_uint2(lo, hi);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) dst[i] = bf16_rne(v[i]);
+        }
+    } else {
+        float *dst = (float *)out + o;
+        if (vec) {
+            *(float4 *)dst = make_float4(v[0], v[1], v[2], v[3]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) dst[i] = v[i];
+        }
+    }
+}
+
 // head_dim 256 takes one 16-row query tile with the whole register file
 // (its two block register sets alone are 128 VGPRs).
 template <int D, int NQT>
 constexpr int gqa_min_waves() { return D >= 256 ? 1 : (NQT == 1 ? 3 : 1); }
 
-template <int D, int NQT, bool ARG>
+// DIRECT: every row of the call lies in one range, so wave 0's merge of the
+// four waves is the row's result and goes straight to the output: no partial,
+// no merge launch (a call with 200 tokens 16.1 us with it, 13.9 without; 32 rows of
+// 760 29.4 and 25.7). A template, since both ends in one kernel cost
+// head_dim 64 a wave per SIMD and spill at 128.
+template <int D, int NQT, bool ARG, bool DIRECT>
 __global__ __launch_bounds__(256, (gqa_min_waves<D, NQT>())) void gqa_decode_kernel(
     typename PlanSel<ARG>::T plan, const uint16_t *__restrict__ kpool,
     const uint16_t *__restrict__ vpool, const int32_t *__restrict__ table,
     const AttRow *__restrict__ rows, const int4 *__restrict__ ranges, int n_rows,
     const void *__restrict__ q, int q_bf16, int layout, int H, int KVH, int DQ, int P, int total64,
     int snap64, int ranges_off, float qscale, int mask_mode, float *__restrict__ part_o,
-    float *__restrict__ part_ml) {
+    float *__restrict__ part_ml, void *__restrict__ out, int out_bf16) {
     // head_dim 16 holds only 4 dims per lane: its score step is one MFMA
     // 16x16x16 (4 bf16 per lane); wider heads use 16x16x32 k-steps.
     constexpr bool K16 = (D == 16);
@@ -433,18 +463,35 @@ __global__ __launch_bounds__(256, (gqa_min_waves<D, NQT>())) void gqa_decode_ker
                     f[w] = (sm[w][qr] == -INFINITY) ? 0.f : __builtin_amdgcn_exp2f(sm[w][qr] - M);
                     L += f[w] * sl[w][qr];
                 }
-                float *po = part_o + (((int64_t)pidx * KVH + kvh) * QRP + qr) * D;
+                if constexpr (DIRECT) {
+                    if (qr >= G * R.qn) continue;
+                    const int ql = qr / G, qi = R.q0 + ql, h = kvh * G + (qr - ql * G);
+                    const int64_t ob = (layout == kLayoutSHD)
+                                           ? ((int64_t)(R.qrow + qi) * H + h) * DQ
+                                           : ((int64_t)R.qrow * H + (int64_t)h * R.nq + qi) * DQ;
+                    const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++) {
-                    fl4 o = acc[nt][mt] * f[0];
+                    for (int mt = 0; mt < MT; mt++) {
+                        fl4 o = acc[nt][mt] * f[0];
 #pragma unroll
-                    for (int w = 1; w < 4; w++) o += so[w - 1][nt][mt][lane] * f[w];
-                    *(fl4 *)(po + mt * 16 + grp * 4) = o;
-                }
-                if (grp == 0) {
-                    float *pm = part_ml + (((int64_t)pidx * KVH + kvh) * QRP + qr) * 2;
-                    pm[0] = M;
-                    pm[1] = L;
+                        for (int w = 1; w < 4; w++) o += so[w - 1][nt][mt][lane] * f[w];
+                        const float v[4] = {o[0] * inv, o[1] * inv, o[2] * inv, o[3] * inv};
+                        if (mt * 16 + grp * 4 < DQ) gqa_store4(out, ob + mt * 16 + grp * 4, v, out_bf16);
+                    }
+                } else {
+                    float *po = part_o + (((int64_t)pidx * KVH + kvh) * QRP + qr) * D;
+#pragma unroll
+                    for (int mt = 0; mt < MT; mt++) {
+                        fl4 o = acc[nt][mt] * f[0];
+#pragma unroll
+                        for (int w = 1; w < 4; w++) o += so[w - 1][nt][mt][lane] * f[w];
+                        *(fl4 *)(po + mt * 16 + grp * 4) = o;
+                    }
+                    if (grp == 0) {
+                        float *pm = part_ml + (((int64_t)pidx * KVH + kvh) * QRP + qr) * 2;
+                        pm[0] = M;
+                        pm[1] = L;
+                    }
                 }
             }
         }
@@ -530,28 +577,7 @@ __global__ __launch_bounds__(256) void gqa_combine_kernel(
     const int qi = R.q0 + ql;
     const int64_t o = (layout == kLayoutSHD) ? ((int64_t)(R.qrow + qi) * H + h) * DQ + d0
                                              : ((int64_t)R.qrow * H + (int64_t)h * R.nq + qi) * DQ + d0;
-    // DQ is a multiple of 8: the 4 dims are all in or all out; one store
-    // when the caller's buffer is aligned for it
-    const bool vec = (((uintptr_t)out) & (out_bf16 ? 7 : 15)) == 0;
-    if (out_bf16) {
-        uint16_t *dst = (uint16_t *)out + o;
-        if (vec) {
-            const uint32_t lo = bf16_rne(v[0]) | ((uint32_t)bf16_rne(v[1]) << 16);
-            const uint32_t hi = bf16_rne(v[2]) | ((uint32_t)bf16_rne(v[3]) << 16);
-            *(uint2 *)dst = make_uint2(lo, hi);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; i++) dst[i] = bf16_rne(v[i]);
-        }
-    } else {
-        float *dst = (float *)out + o;
-        if (vec) {
-            *(float4 *)dst = make_float4(v[0], v[1], v[2], v[3]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; i++) dst[i] = v[i];
-        }
-    }
+    gqa_store4(out, o, v, out_bf16);
 }
 
 template <int D, int NQT, bool ARG>
@@ -562,12 +588,15 @@ static hipError_t launch_gqa_t(hipStream_t s, typename PlanSel<ARG>::T plan,
                                int layout, int H, int KVH, int DQ, int P, int total64, int snap64,
                                int ranges_off, float qscale,
                                int mask_mode, float *part_o, float *part_ml, void *out,
-                               int out_bf16, int max_qr, hipEvent_t ev0, hipEvent_t ev1) {
-    hipError_t e = launch_timed(gqa_decode_kernel<D, NQT, ARG>, dim3(n_ranges * KVH), dim3(256), s,
-                                ev0, ev1, plan, kpool, vpool, table, rows, ranges, n_rows, q, q_bf16,
-                                layout, H, KVH, DQ, P, total64, snap64, ranges_off, qscale,
-                                mask_mode, part_o, part_ml);
-    if (e != hipSuccess) return e;
+                               int out_bf16, int max_qr, bool single, hipEvent_t ev0, hipEvent_t ev1) {
+    auto kernel = gqa_decode_kernel<D, NQT, ARG, false>;
+    if constexpr (ARG)
+        if (single) kernel = gqa_decode_kernel<D, NQT, ARG, true>;
+    hipError_t e = launch_timed(kernel, dim3(n_ranges * KVH), dim3(256), s, ev0, ev1, plan, kpool,
+                                vpool, table, rows, ranges, n_rows, q, q_bf16, layout, H, KVH, DQ, P,
+                                total64, snap64, ranges_off, qscale, mask_mode, part_o, part_ml, out,
+                                out_bf16);
+    if (e != hipSuccess || (ARG && single)) return e;
     constexpr int TQ = 256 / (D / 4);  // query rows per combine work-group
     gqa_combine_kernel<ARG><<<dim3(n_rows, KVH, (max_qr + TQ - 1) / TQ), 256, 0, s>>>(
         plan, rows, part_o, part_ml, out, out_bf16, layout, H, KVH, D, DQ, 16 * NQT);
@@ -580,7 +609,7 @@ hipError_t launch_gqa_decode(hipStream_t s, const PlanArg *plan, const uint16_t 
                              int layout, int H, int KVH, int hd, int hdi, int P, int total64,
                              int snap64, int ranges_off, float qscale,
                              int mask_mode, int nqt, float *part_o, float *part_ml, void *out,
-                             int out_bf16, int max_qr, hipEvent_t ev0, hipEvent_t ev1) {
+                             int out_bf16, int max_qr, bool single, hipEvent_t ev0, hipEvent_t ev1) {
     if (n_ranges <= 0) return hipSuccess;
 #define RLX_GQA_CASE(DD, NN)                                                                    \
     if (hd == DD && nqt == NN)                                                                  \
@@ -588,12 +617,12 @@ hipError_t launch_gqa_decode(hipStream_t s, const PlanArg *plan, const uint16_t 
                                                  ranges, n_ranges, q, q_bf16, layout, H, KVH,   \
                                                  hdi, P, total64, snap64, ranges_off,           \
                                                  qscale, mask_mode, part_o, part_ml, out,       \
-                                                 out_bf16, max_qr, ev0, ev1)                    \
+                                                 out_bf16, max_qr, single, ev0, ev1)            \
                     : launch_gqa_t<DD, NN, false>(s, NoPlan{0}, kpool, vpool, table, rows,      \
                                                   n_rows, ranges, n_ranges, q, q_bf16, layout,  \
                                                   H, KVH, hdi, P, total64, snap64, -1, qscale,  \
                                                   mask_mode, part_o, part_ml, out, out_bf16,    \
-                                                  max_qr, ev0, ev1);
+                                                  max_qr, single, ev0, ev1);
     RLX_GQA_CASE(128, 1)
     RLX_GQA_CASE(128, 2)
     RLX_GQA_CASE(64, 1)

@@ -763,8 +763,40 @@ int gqa_wg_per_cu() {
     }();
     return v;
 }
-int gqa_decode_split(const Cache *c, AttRow *rows, int n_rows, int *pre, int *cuts, int4 *ranges,
-                     int *total64_out) {
+// Cuts at row boundaries only, for calls whose work-groups stay short that way:
+// with no row divided the decode kernel writes the outputs itself and the merge
+// launch falls away.  The ranges hold consecutive rows, at most as much as the
+// longest row or an even share.  The line is the tokens a work-group may hold:
+// 768 at head_dim 128, and by the row bytes elsewhere.  At batch 1, 32/8 heads of
+// 128, one range against cuts and a merge: 600 tokens 13.6 against 16.6 us, 800
+// 14.7 against 16.6, 1000 18.2 against 16.8; heads of 64: 1000 tokens 13.7 against
+// 16.8, 1600 17.1 against 17.9, 2000 20.4 against 20.4.  With two query tiles (17 to
+// 32 query rows a kv head) two thirds of it: 8 x 760 tokens, 32 query rows,
+// took 23.9 whole against 23.0, 8 x 510 22.0 against 24.7.  The ranges have to fit the
+// kernel arguments (the kernel's own search knows even cuts only).  Returns their
+// number, or 0.
+int gqa_whole_rows(const Cache *c, int nqt, const int *pre, int n_rows, int full, int *cuts) {
+    const int line = (nqt == 1 ? 1536 : 1024) / std::max(c->hd, 64);  // 64-token units
+    if ((size_t)n_rows * sizeof(AttRow) + (size_t)full * sizeof(int4) > kPlanArgBytes) return 0;
+    int most = (pre[n_rows] + full - 1) / full;
+    for (int i = 0; i < n_rows; i++) most = std::max(most, pre[i + 1] - pre[i]);
+    for (; most <= line; most++) {
+        int n = 0;
+        cuts[0] = 0;
+        for (int i = 0; i < n_rows && n < full; i++)
+            if (pre[i + 1] - cuts[n] > most) {
+                n++;
+                if (n < full) cuts[n] = pre[i];
+            }
+        if (n >= full) continue;
+        cuts[n + 1] = pre[n_rows];
+        return n + 1;
+    }
+    return 0;
+}
+
+int gqa_decode_split(const Cache *c, int nqt, AttRow *rows, int n_rows, int *pre, int *cuts,
+                     int4 *ranges, int *total64_out) {
     pre[0] = 0;
     for (int i = 0; i < n_rows; i++) pre[i + 1] = pre[i] + (rows[i].len + 63) / 64;
     const int total64 = pre[n_rows];
@@ -790,8 +822,12 @@ int gqa_decode_split(const Cache *c, AttRow *rows, int n_rows, int *pre, int *cu
     // kept.)
     if (q3 >= 16 && (int64_t)total64 * 64 >= (int64_t)q3 * kGqaLongRange) want = q3;
     if (ranges_override > 0) want = std::min(ranges_override, full);
-    const int n_ranges = std::max(1, std::min(want, total64));
-    gqa_range_cuts(pre, n_rows, n_ranges, kGqaSnap64, cuts);
+    int n_ranges = std::max(1, std::min(want, total64));
+    const int whole = ranges_override > 0 ? 0 : gqa_whole_rows(c, nqt, pre, n_rows, full, cuts);
+    if (whole > 0)
+        n_ranges = whole;
+    else
+        gqa_range_cuts(pre, n_rows, n_ranges, kGqaSnap64, cuts);
     for (int k = 0; k < n_rows; k++) rows[k].part = -1;
     int r = 0;
     for (int i = 0; i < n_ranges; i++) {
@@ -826,6 +862,22 @@ PrefillSplit prefill_parts(Cache *c, std::vector<std::vector<int4>> &groups, std
     groups = std::move(g);
     cost = std::move(k);
     return sp;
+}
+
+// Whether the decode kernel may write a call's outputs itself: every row lies in
+// one range, and out does not overlap q, which other work-groups may still read
+// (the merge runs after all of them).
+bool gqa_single(const AttRow *rows, int n, const void *q, int q_dtype, const void *out,
+                int out_dtype, int row_elems) {
+    size_t tokens = 0;
+    for (int i = 0; i < n; i++) {
+        if (rows[i].nsplit != 1) return false;
+        tokens = std::max(tokens, (size_t)rows[i].qrow + rows[i].nq);
+    }
+    const char *qb = (const char *)q, *ob = (const char *)out;
+    const size_t qn = tokens * row_elems * (q_dtype == RLX_BF16 ? 2 : 4);
+    const size_t on = tokens * row_elems * (out_dtype == RLX_BF16 ? 2 : 4);
+    return ob >= qb + qn || qb >= ob + on;
 }
 
 // One AttRow per sequence of an attention call, with nsplit[i] context
@@ -1766,7 +1818,7 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
     std::vector<int> pre(n_rows + 1), cuts(c->cus + 2);
     std::vector<int4> ranges(c->cus + 1);
     int total64 = 0;
-    const int n_ranges = gqa_decode_split(c, rows.data(), n_rows, pre.data(), cuts.data(),
+    const int n_ranges = gqa_decode_split(c, nqt, rows.data(), n_rows, pre.data(), cuts.data(),
                                           ranges.data(), &total64);
     ranges.resize(n_ranges);
     const int parts = n_rows + n_ranges;
@@ -1808,7 +1860,9 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
                               d_ranges, n_ranges, q, q_dtype == RLX_BF16, qo_layout, num_heads,
                               c->kvh, c->hd, c->hdi, c->P, total64, kGqaSnap64, ranges_off, qscale,
                               mask_mode, nqt, (float *)c->ws, (float *)((char *)c->ws + po_bytes),
-                              out, out_dtype == RLX_BF16, std::min(max_qr, cap), e0, e1));
+                              out, out_dtype == RLX_BF16, std::min(max_qr, cap),
+                              gqa_single(rows.data(), n_rows, q, q_dtype, out, out_dtype, num_heads * c->hdi),
+                              e0, e1));
     return RLX_OK;
 }
 }  // namespace
@@ -1943,7 +1997,7 @@ static int32_t gqa_ref_image_impl(Cache *c, int32_t layer, int32_t n_seqs, const
     std::vector<int> pre(n_rows + 1), cuts(c->cus + 2);
     std::vector<int4> ranges(c->cus + 1);
     int total64 = 0;
-    const int n_ranges = gqa_decode_split(c, rows.data(), n_rows, pre.data(), cuts.data(), ranges.data(),
+    const int n_ranges = gqa_decode_split(c, nqt, rows.data(), n_rows, pre.data(), cuts.data(), ranges.data(),
                                           &total64);
     ranges.resize(n_ranges);
     const int parts = n_rows + n_ranges;
@@ -1974,7 +2028,7 @@ static int32_t gqa_ref_image_impl(Cache *c, int32_t layer, int32_t n_seqs, const
                               (const int4 *)((char *)dev + o_w), n_ranges, q, q_dtype == RLX_BF16, qo_layout,
                               num_heads, c->kvh, c->hd, c->hdi, c->P, total64, kGqaSnap64, -1, qscale,
                               mask_mode, nqt, po, pm, out, out_dtype == RLX_BF16, std::min(max_qr, cap),
-                              nullptr, nullptr));
+                              false, nullptr, nullptr));
     return RLX_OK;
 }
 
@@ -2043,7 +2097,7 @@ int32_t rlx_gqa_attend_noalloc(void *h, int32_t layer, int32_t n_seqs, const int
     int pre[kRowCap + 1], cuts[kRangeCap + 1];
     int4 ranges[kRangeCap];
     int total64 = 0;
-    const int n_ranges = gqa_decode_split(c, rows, n_rows, pre, cuts, ranges, &total64);
+    const int n_ranges = gqa_decode_split(c, nqt, rows, n_rows, pre, cuts, ranges, &total64);
     const int QRP = 16 * nqt;
     const size_t parts = (size_t)n_rows + n_ranges;
     const size_t po_bytes = parts * c->kvh * QRP * c->hd * sizeof(float);
@@ -2067,7 +2121,9 @@ int32_t rlx_gqa_attend_noalloc(void *h, int32_t layer, int32_t n_seqs, const int
                               num_heads, c->kvh, c->hd, c->hdi, c->P, total64, kGqaSnap64, ranges_off,
                               scale * 1.4426950408889634f, mask_mode, nqt, (float *)scr,
                               (float *)((char *)scr + po_bytes), out, out_dtype == RLX_BF16,
-                              std::min(max_qr, cap), nullptr, nullptr));
+                              std::min(max_qr, cap),
+                              gqa_single(rows, n_rows, q, q_dtype, out, out_dtype, num_heads * c->hdi),
+                              nullptr, nullptr));
     return RLX_OK;
 }
 
