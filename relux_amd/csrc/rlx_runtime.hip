@@ -298,6 +298,16 @@ int32_t ensure_ws(Cache *c, size_t bytes) {
     return RLX_OK;
 }
 
+// A workspace of `bytes` that a call can do without: false where it cannot
+// grow (a cap, no memory, a stream under capture), and the failed allocation
+// is not left behind for the next launch's error check.
+bool optional_ws(Cache *c, size_t bytes) {
+    if (bytes > c->ws_cap && capturing(c)) return false;
+    if (ensure_ws(c, bytes) == RLX_OK) return true;  // (counts it as a request too)
+    (void)hipGetLastError();
+    return false;
+}
+
 // Caller rows of a head dim that is not a multiple of 8 cross the boundary
 // through the handle's adapter buffer: inputs are copied to rows of the next
 // multiple of 8 (zero filled: zero dims add nothing to a dot product and
@@ -858,7 +868,7 @@ PrefillSplit prefill_parts(Cache *c, std::vector<std::vector<int4>> &groups, std
         return (tile_keys(rows[w.x], mask_mode, toks, w.z) + 63) / 64;
     });
     const size_t need = head + sp.ranges.size() * (kPrefillPartO + kPrefillPartMl);
-    if (sp.ranges.empty() || (need > c->ws_cap && (capturing(c) || ensure_ws(c, need) != RLX_OK))) return {};
+    if (sp.ranges.empty() || !optional_ws(c, need)) return {};
     groups = std::move(g);
     cost = std::move(k);
     return sp;
@@ -1452,6 +1462,7 @@ int32_t project_append(Cache *c, int model, int32_t layer, int32_t n_seqs, const
                                      q_dtype == RLX_BF16, ls.pool0, ls.pool1, c->d_table, c->P, c->cus, e0, e1));
             return RLX_OK;
         }
+        (void)hipGetLastError();  // (not for the next launch's error check)
     }
     for (int r0 = 0; r0 < total; r0 += kProjRows) {
         const int rows = std::min(kProjRows, total - r0);
@@ -2975,7 +2986,7 @@ int32_t rlx_free_list(void *h, int32_t layer, int32_t *out, int32_t cap, int32_t
 static int32_t sample_scratch(Cache *c, SampleArgs &a, int n_rows, size_t head) {
     const size_t need = head + (size_t)plan_sample_split(a, n_rows, nullptr);
     int32_t rc = RLX_OK;
-    if (a.uch > 0 && need > c->ws_cap && (capturing(c) || ensure_ws(c, need) != RLX_OK)) {
+    if (a.uch > 0 && !optional_ws(c, need)) {
         a.uch = 0;
         return ensure_ws(c, head);
     }
