@@ -305,6 +305,28 @@ __device__ __forceinline__ int2 plan_work(const int2 *work, int n_rows, int b) {
     }
 }
 
+// The same of an MLA call with head groups.  Work-group b runs on XCD b mod 8,
+// and the groups of a sequence (consecutive rows of equal splits) read the same
+// latent rows: splits 8 at a time, the groups of those 8 one after the other, so
+// that split s of every group runs on one XCD at about the same time.  The
+// staged list (mla_attend_impl) holds this order; from the arguments it is
+// computed: the row whose partials b falls among names the sequence.
+template <bool ARG>
+__device__ __forceinline__ int2 plan_work_grouped(const int2 *work, int n_rows, int b, int H, int QRP) {
+    const int2 w = plan_work<ARG>(work, n_rows, b);
+    if constexpr (ARG) {
+        const __attribute__((address_space(4))) int32_t *p =
+            (const __attribute__((address_space(4))) int32_t *)kernarg_plan() + w.x * 8;
+        const uint32_t ns = (uint32_t)p[4], g = (uint32_t)p[6] / (uint32_t)QRP;  // nsplit, group of row w.x
+        const uint32_t groups = ((uint32_t)H * (uint32_t)p[2] + (uint32_t)QRP - 1) / (uint32_t)QRP;
+        const uint32_t i = g * ns + (uint32_t)w.y;  // place among the sequence's work-groups
+        const uint32_t s0 = i / (8 * groups) * 8, m = min(8u, ns - s0), rem = i - s0 * groups;
+        return int2{w.x - (int)g + (int)(rem / m), (int)(s0 + rem % m)};
+    } else {
+        return w;
+    }
+}
+
 
 // Upper bound on context splits of one sequence (the runtime sizes splits so
 // that it holds).

@@ -221,7 +221,8 @@ __global__ __launch_bounds__(64 * MlaShape<NQT>::NW, MlaShape<NQT>::WGS) void ml
     const int wave = tid >> 6;
     const int col = lane & 15;
     const int grp = lane >> 4;
-    const int2 wk = plan_work<ARG>(work, n_rows, blockIdx.x);
+    const int2 wk = KEEP ? plan_work_grouped<ARG>(work, n_rows, blockIdx.x, H, 16 * NQT)
+                         : plan_work<ARG>(work, n_rows, blockIdx.x);
     const AttRow R = plan_row<ARG>(rows, wk.x);
     // This work item's query rows: rows [q0, q0 + qn) of the sequence's
     // H x nq (query-major: row qi H + h), one head group of a call with more

@@ -2428,14 +2428,17 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
     // equal splits).  Work-group b runs on XCD b mod 8, so split s of every
     // group is placed at the same position mod 8 of consecutive runs of 8
     // work-groups: the groups of a split run on one XCD at about the same
-    // time and all but the first find its tiles in that XCD's L2.  (The
-    // plan then travels staged: the kernel-argument form derives the work
-    // list in row order.)
+    // time and all but the first find its tiles in that XCD's L2.  A plan of
+    // at most 64 rows travels in the kernel arguments and each work-group
+    // computes its place in this order (plan_work_grouped); a larger one is
+    // staged with the list (8 sequences around 8k, 128 heads, a pass: staged
+    // 81.4 us, in the arguments 77.5).
+    const bool staged = rows.size() * sizeof(AttRow) > sizeof(PlanArg);
     const bool grouped = rows.size() > (size_t)n_seqs;
-    if (!grouped) {
+    if (staged && !grouped) {
         for (size_t r = 0; r < rows.size(); r++)
             for (int sp = 0; sp < nsplit[r]; sp++) work.push_back(int2{(int)r, sp});
-    } else {
+    } else if (staged) {
         for (size_t r0 = 0; r0 < rows.size();) {
             size_t r1 = r0;
             while (r1 < rows.size() && rows[r1].qrow == rows[r0].qrow) r1++;  // one sequence's groups
@@ -2457,7 +2460,7 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
     const PlanArg *plan = nullptr;
     const AttRow *d_rows = nullptr;
     const int2 *d_work = nullptr;
-    if (!grouped && rows.size() * sizeof(AttRow) <= sizeof(PlanArg)) {
+    if (!staged) {
         memcpy(plan_arg.b, rows.data(), rows.size() * sizeof(AttRow));
         plan = &plan_arg;
     } else {
@@ -2474,7 +2477,7 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1))) return bail(rc);
     HIP_TRY(launch_mla_decode(c->stream, plan, ls.pool0, c->d_table, d_rows, (int)rows.size(), d_work,
-                              (int)work.size(), q_nope,
+                              parts, q_nope,
                               q_rope, q_dtype == RLX_BF16, (const uint16_t *)w_uk,
                               (const uint16_t *)w_uv, num_heads, head_dim, c->dc, c->dr, total_q,
                               row_nq, c->P, qscale, kmask, nqt, (uint16_t *)ws,
