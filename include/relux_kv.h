@@ -151,7 +151,10 @@ int32_t rlx_cache_set_stream(void *cache, void *stream);
  * latents, staged plans) from a per-handle workspace, and calls whose
  * plans do not fit the kernel arguments stage them through 8 upload slots
  * (pinned host + device); a call that needs more than either holds grows it
- * on the spot (stream sync, hipFree, hipMalloc inside that call).  This
+ * on the spot (stream sync, hipMalloc, hipFree inside that call).  A
+ * workspace that a captured call put into a graph is kept until the handle
+ * is destroyed, however it grows; a captured call that can do without
+ * scratch (chunked prefill, sampling without top-k) takes none.  This
  * grows the workspace to at least workspace_bytes, every staging slot to
  * at least staging_bytes and the adapter buffer (rows of a head_dim, d_model
  * or k_in that the kernels take padded) to at least adapter_bytes now, so
@@ -161,11 +164,11 @@ int32_t rlx_cache_set_stream(void *cache, void *stream);
 int32_t rlx_cache_reserve(void *cache, uint64_t workspace_bytes, uint64_t staging_bytes,
                           uint64_t adapter_bytes);
 /* out[0] workspace capacity, out[1] the largest workspace any call on the
- * handle has asked for, out[2] the smallest staging slot's capacity, out[3]
- * the largest plan any call has staged, out[4] adapter capacity, out[5] the
- * largest adapter request (bytes).  A trial run of the largest calls
- * followed by rlx_cache_reserve(out[1], out[3], out[5]) on a fresh handle
- * keeps every later call of those sizes from allocating. */
+ * handle has asked for (granted or not), out[2] the smallest staging slot's
+ * capacity, out[3] the largest plan any call has staged, out[4] adapter
+ * capacity, out[5] the largest adapter request (bytes).  A trial run of the
+ * largest calls followed by rlx_cache_reserve(out[1], out[3], out[5]) on a
+ * fresh handle keeps every later call of those sizes from allocating. */
 int32_t rlx_cache_memory(void *cache, uint64_t *out);
 
 /* ---- append (scatter into pages) -------------------------------------- */
@@ -477,9 +480,10 @@ int32_t rlx_sample(void *cache, const float *logits, int32_t n_rows, int32_t voc
  * from the host and the call does not wait -- except the first call that
  * needs a larger cache workspace (the split paths' chunk lists, top-k in
  * (0, 256] past 8192 entries, or no top-k past 12288: at most 64 MiB),
- * which synchronises the stream and allocates it once (without top-k a call
- * that cannot -- its stream under capture, no memory -- runs unsplit).  Same tokens as rlx_sample given the same windows
- * and draws. */
+ * which synchronises the stream and allocates it once.  Without top-k a
+ * call runs its rows unsplit where there is no memory for it, and always on
+ * a stream under capture, so that its graph holds no scratch.  Same tokens
+ * as rlx_sample given the same windows and draws. */
 int32_t rlx_sample_async(void *cache, const float *logits, int32_t n_rows, int32_t vocab,
                          int64_t row_stride, const rlx_sampler_t *params, const int32_t *history,
                          int64_t hist_stride, const int32_t *hist_len, const float *uniforms,

@@ -28,6 +28,7 @@
 
 #include "../../include/relux_kv.h"
 #include "rlx_common.h"
+#include "rlx_scratch.h"
 
 using namespace rlx;
 
@@ -128,12 +129,8 @@ struct Cache {
     std::map<int64_t, int32_t> pending;  // flat table index -> value
     Slot slots[kSlots];
     int next_slot = 0;
-    void *ws = nullptr;
-    size_t ws_cap = 0;
-    size_t ws_peak = 0;     // largest workspace a call asked for
-    void *ad = nullptr;     // adapter rows of head dims that are not multiples of 8
-    size_t ad_cap = 0;
-    size_t ad_peak = 0;     // largest adapter request
+    Scratch ws;             // workspace
+    Scratch ad;             // adapter rows of head dims that are not multiples of 8
     size_t stage_peak = 0;  // largest plan a call staged
     SpillTier spill;
     // Attention-kernel timing: event pairs, reused across reports.
@@ -153,6 +150,30 @@ struct Cache {
         return L[layer].table[(int64_t)seq * max_pages + k];
     }
 };
+
+// The allocator of a handle's growable buffers (rlx_scratch.h).  A refused
+// allocation is not left behind for the next launch's error check.
+struct HipMem {
+    hipStream_t stream;
+    void *get(size_t n) {
+        void *p = nullptr;
+        return checked(hipMalloc(&p, n)) ? p : nullptr;
+    }
+    void put(void *p) { (void)hipFree(p); }
+    bool sync() { return checked(hipStreamSynchronize(stream)); }
+
+private:
+    static bool checked(hipError_t e) {
+        if (e != hipSuccess) (void)hipGetLastError();
+        return e == hipSuccess;
+    }
+};
+
+int32_t grown(Grow g, const char *what, size_t bytes) {
+    if (g == Grow::kOk) return RLX_OK;
+    return fail(RLX_ERR_HIP, g == Grow::kSync ? "%s of %zu bytes: its stream cannot be waited for"
+                                              : "%s of %zu bytes: out of memory", what, bytes);
+}
 
 // Copy `bytes` of host data into the next staging slot and enqueue its
 // upload; returns the device address the kernels should read.
@@ -277,35 +298,44 @@ int32_t flush_patches_inline(Cache *c) {
     return RLX_OK;
 }
 
+// RLX_WS_MAX_KB caps the workspace (tests force the failure path of a call
+// with it; unset or 0: no cap).
+bool ws_capped(const Cache *c, size_t bytes, long long *kb) {
+    const char *lim = bytes > c->ws.cap ? getenv("RLX_WS_MAX_KB") : nullptr;
+    *kb = lim ? atoll(lim) : 0;
+    return *kb > 0 && bytes > (size_t)*kb << 10;
+}
+
+// A buffer that a call's launches are about to use: one that goes into a graph
+// is kept until the handle closes.
+void mark_held(Cache *c, Scratch &s, size_t bytes) {
+    if (bytes && !s.held && capturing(c)) s.held = true;
+}
+
 int32_t ensure_ws(Cache *c, size_t bytes) {
-    c->ws_peak = std::max(c->ws_peak, bytes);
-    if (bytes <= c->ws_cap) return RLX_OK;
-    // RLX_WS_MAX_KB caps the workspace (tests force the failure path of a
-    // call with it; unset or 0: no cap).
-    if (const char *lim = getenv("RLX_WS_MAX_KB")) {
-        const long long kb = atoll(lim);
-        if (kb > 0 && bytes > (size_t)kb << 10)
-            return fail(RLX_ERR_HIP, "workspace of %zu bytes exceeds RLX_WS_MAX_KB=%lld", bytes, kb);
+    long long kb;
+    if (ws_capped(c, bytes, &kb)) {
+        c->ws.peak = std::max(c->ws.peak, bytes);
+        return fail(RLX_ERR_HIP, "workspace of %zu bytes exceeds RLX_WS_MAX_KB=%lld", bytes, kb);
     }
-    size_t cap = std::max(bytes, c->ws_cap * 2);
-    cap = (cap + 65535) & ~(size_t)65535;
-    HIP_TRY(hipStreamSynchronize(c->stream));
-    if (c->ws) HIP_TRY(hipFree(c->ws));
-    c->ws = nullptr;
-    c->ws_cap = 0;
-    HIP_TRY(hipMalloc(&c->ws, cap));
-    c->ws_cap = cap;
-    return RLX_OK;
+    HipMem m{c->stream};
+    const int32_t rc = grown(c->ws.need(m, bytes), "workspace", bytes);
+    if (rc == RLX_OK) mark_held(c, c->ws, bytes);
+    return rc;
 }
 
 // A workspace of `bytes` that a call can do without: false where it cannot
-// grow (a cap, no memory, a stream under capture), and the failed allocation
-// is not left behind for the next launch's error check.
+// grow (a cap, no memory), and on a stream under capture, where
+// a graph would keep the scratch of a call that needs none.
 bool optional_ws(Cache *c, size_t bytes) {
-    if (bytes > c->ws_cap && capturing(c)) return false;
-    if (ensure_ws(c, bytes) == RLX_OK) return true;  // (counts it as a request too)
-    (void)hipGetLastError();
-    return false;
+    long long kb;
+    const bool capped = ws_capped(c, bytes, &kb);
+    if (capped || capturing(c)) {
+        c->ws.peak = std::max(c->ws.peak, bytes);
+        return false;
+    }
+    HipMem m{c->stream};
+    return c->ws.want(m, bytes);
 }
 
 // Caller rows of a head dim that is not a multiple of 8 cross the boundary
@@ -321,17 +351,11 @@ int32_t adapter_regions(Cache *c, const size_t *bytes, int n, char **out) {
         off[i] = total;
         total += (bytes[i] + 255) & ~(size_t)255;
     }
-    c->ad_peak = std::max(c->ad_peak, total);
-    if (total > c->ad_cap) {
-        const size_t cap = (std::max(total, c->ad_cap * 2) + 65535) & ~(size_t)65535;
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        if (c->ad) HIP_TRY(hipFree(c->ad));
-        c->ad = nullptr;
-        c->ad_cap = 0;
-        HIP_TRY(hipMalloc(&c->ad, cap));
-        c->ad_cap = cap;
-    }
-    for (int i = 0; i < n; i++) out[i] = (char *)c->ad + off[i];
+    HipMem m{c->stream};
+    const int32_t rc = grown(c->ad.need(m, total), "adapter buffer", total);
+    if (rc) return rc;
+    mark_held(c, c->ad, total);
+    for (int i = 0; i < n; i++) out[i] = (char *)c->ad.ptr + off[i];
     return RLX_OK;
 }
 
@@ -415,8 +439,9 @@ void destroy_cache(Cache *c) {
         if (ls.pool1) (void)hipFree(ls.pool1);
     }
     if (c->d_table) (void)hipFree(c->d_table);
-    if (c->ws) (void)hipFree(c->ws);
-    if (c->ad) (void)hipFree(c->ad);
+    HipMem mem{c->stream};
+    c->ws.release(mem);
+    c->ad.release(mem);
     for (auto &p : c->tev) {
         (void)hipEventDestroy(p.first);
         (void)hipEventDestroy(p.second);
@@ -854,9 +879,9 @@ int gqa_decode_split(const Cache *c, int nqt, AttRow *rows, int n_rows, int *pre
     return n_ranges;
 }
 
-// split_prefill for a call whose own scratch is `head` bytes of the workspace,
-// the partial sums behind it.  A workspace that cannot grow to them (a cap, or
-// a stream under capture) keeps the tiles whole.
+// split_prefill for a call whose own scratch is `head` bytes of the workspace
+// (there already), the partial sums behind it.  Without room for them
+// (optional_ws) the tiles stay whole.
 PrefillSplit prefill_parts(Cache *c, std::vector<std::vector<int4>> &groups, std::vector<double> &cost,
                            const std::vector<AttRow> &rows, int mask_mode, int toks, size_t head) {
     auto g = groups;
@@ -1148,24 +1173,10 @@ int32_t rlx_cache_set_stream(void *h, void *stream) {
 int32_t rlx_cache_reserve(void *h, uint64_t ws_bytes, uint64_t stage_bytes, uint64_t ad_bytes) {
     if (!h) return fail(RLX_ERR_INVALID, "null cache");
     Cache *c = as_cache(h);
-    if (ws_bytes > c->ws_cap) {
-        const size_t cap = ((size_t)ws_bytes + 65535) & ~(size_t)65535;
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        if (c->ws) HIP_TRY(hipFree(c->ws));
-        c->ws = nullptr;
-        c->ws_cap = 0;
-        HIP_TRY(hipMalloc(&c->ws, cap));
-        c->ws_cap = cap;
-    }
-    if (ad_bytes > c->ad_cap) {
-        const size_t cap = ((size_t)ad_bytes + 65535) & ~(size_t)65535;
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        if (c->ad) HIP_TRY(hipFree(c->ad));
-        c->ad = nullptr;
-        c->ad_cap = 0;
-        HIP_TRY(hipMalloc(&c->ad, cap));
-        c->ad_cap = cap;
-    }
+    HipMem m{c->stream};
+    int32_t rc;
+    if ((rc = grown(c->ws.reserve(m, ws_bytes), "workspace", ws_bytes))) return rc;
+    if ((rc = grown(c->ad.reserve(m, ad_bytes), "adapter buffer", ad_bytes))) return rc;
     for (Slot &s : c->slots) {
         if (stage_bytes <= s.cap) continue;
         const size_t cap = ((size_t)stage_bytes + 4095) & ~(size_t)4095;
@@ -1189,12 +1200,12 @@ int32_t rlx_cache_memory(void *h, uint64_t *out) {
     const Cache *c = as_cache(h);
     size_t smin = c->slots[0].cap;
     for (const Slot &s : c->slots) smin = std::min(smin, s.cap);
-    out[0] = c->ws_cap;
-    out[1] = c->ws_peak;
+    out[0] = c->ws.cap;
+    out[1] = c->ws.peak;
     out[2] = smin;
     out[3] = c->stage_peak;
-    out[4] = c->ad_cap;
-    out[5] = c->ad_peak;
+    out[4] = c->ad.cap;
+    out[5] = c->ad.peak;
     return RLX_OK;
 }
 
@@ -1795,8 +1806,8 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
         a.ranges = (const int2 *)((char *)dev + o_g);
         a.merge = (const int4 *)((char *)dev + o_m);
         a.n_merge = (int)sp.merge.size();
-        a.part_o = (float *)c->ws;
-        a.part_ml = (float *)((char *)c->ws + sp.ranges.size() * kPrefillPartO);
+        a.part_o = (float *)c->ws.ptr;
+        a.part_ml = (float *)((char *)c->ws.ptr + sp.ranges.size() * kPrefillPartO);
         a.q = q;
         a.out = out;
         a.q_bf16 = q_dtype == RLX_BF16;
@@ -1870,7 +1881,7 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
     HIP_TRY(launch_gqa_decode(c->stream, plan, ls.pool0, ls.pool1, c->d_table, d_rows, n_rows,
                               d_ranges, n_ranges, q, q_dtype == RLX_BF16, qo_layout, num_heads,
                               c->kvh, c->hd, c->hdi, c->P, total64, kGqaSnap64, ranges_off, qscale,
-                              mask_mode, nqt, (float *)c->ws, (float *)((char *)c->ws + po_bytes),
+                              mask_mode, nqt, (float *)c->ws.ptr, (float *)((char *)c->ws.ptr + po_bytes),
                               out, out_dtype == RLX_BF16, std::min(max_qr, cap),
                               gqa_single(rows.data(), n_rows, q, q_dtype, out, out_dtype, num_heads * c->hdi),
                               e0, e1));
@@ -2020,7 +2031,7 @@ static int32_t gqa_ref_image_impl(Cache *c, int32_t layer, int32_t n_seqs, const
     const size_t po_bytes = (size_t)parts * c->kvh * QRP * c->hd * sizeof(float);
     const size_t pm_bytes = (size_t)parts * c->kvh * QRP * 2 * sizeof(float);
     if ((rc = ensure_ws(c, 2 * img_bytes + tab_bytes + po_bytes + pm_bytes))) return rc;
-    char *ws = (char *)c->ws;
+    char *ws = (char *)c->ws.ptr;
     uint16_t *dk = (uint16_t *)ws, *dv = (uint16_t *)(ws + img_bytes);
     int32_t *dtable = (int32_t *)(ws + 2 * img_bytes);
     float *po = (float *)(ws + 2 * img_bytes + tab_bytes);
@@ -2279,6 +2290,7 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
         const size_t e_bytes = (size_t)tok_off * hg * dp * 2;
         const size_t r_bytes = (size_t)tok_off * kMlaDr * 2;  // rope keys of the call
         const size_t x_bytes = (2 * w_bytes + 2 * e_bytes + r_bytes + 255) & ~(size_t)255;
+        if ((rc = ensure_ws(c, x_bytes))) return rc;
         // (parts chosen over all heads: a head's attention is the same
         // computation however the heads are grouped)
         PrefillSplit sp = prefill_parts(c, pgroups, pcost, rows, mask_mode, kPrefillRows, x_bytes);
@@ -2300,13 +2312,12 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
         };
         sp.merge = heads_below(sp.merge, hg);
         if ((rc = flush_patches(c))) return rc;
-        if ((rc = ensure_ws(c, x_bytes))) return rc;
         Blob b;
         size_t o_r = b.add(rows), o_d = b.add(dwork), o_p = b.add(pwork), o_g = b.add(sp.ranges),
                o_m = b.add(sp.merge);
         void *dev;
         if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
-        char *ws = (char *)c->ws;
+        char *ws = (char *)c->ws.ptr;
         uint16_t *wt_k = (uint16_t *)ws, *wt_v = (uint16_t *)(ws + w_bytes);
         uint16_t *kc = (uint16_t *)(ws + 2 * w_bytes), *vt = (uint16_t *)(ws + 2 * w_bytes + e_bytes);
         uint16_t *kr = (uint16_t *)(ws + 2 * w_bytes + 2 * e_bytes);
@@ -2473,7 +2484,7 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
     }
     if (scale <= 0.f) scale = (float)(1.0 / std::sqrt((double)(head_dim + c->dr)));
     const float qscale = scale * 1.4426950408889634f;
-    char *ws = (char *)c->ws;
+    char *ws = (char *)c->ws.ptr;
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1))) return bail(rc);
     HIP_TRY(launch_mla_decode(c->stream, plan, ls.pool0, c->d_table, d_rows, (int)rows.size(), d_work,
@@ -2983,18 +2994,18 @@ int32_t rlx_free_list(void *h, int32_t layer, int32_t *out, int32_t cap, int32_t
 // ---- token selection ------------------------------------------------------
 
 // Workspace of a Sample call, its split planned at byte `head` (behind what
-// the call keeps there itself).  The mass split is an optional one: a
-// workspace that cannot grow (a cap, or a stream under capture) leaves the
-// call on the whole-row path, which needs none.
+// the call keeps there itself).  The mass split is an optional one: without
+// its scratch (optional_ws) the call takes the whole-row path, which needs
+// none.
 static int32_t sample_scratch(Cache *c, SampleArgs &a, int n_rows, size_t head) {
     const size_t need = head + (size_t)plan_sample_split(a, n_rows, nullptr);
-    int32_t rc = RLX_OK;
     if (a.uch > 0 && !optional_ws(c, need)) {
         a.uch = 0;
         return ensure_ws(c, head);
     }
-    if ((rc = ensure_ws(c, need))) return rc;
-    plan_sample_split(a, n_rows, (char *)c->ws + head);
+    const int32_t rc = ensure_ws(c, need);
+    if (rc) return rc;
+    plan_sample_split(a, n_rows, (char *)c->ws.ptr + head);
     return RLX_OK;
 }
 
@@ -3011,8 +3022,8 @@ int32_t rlx_greedy(void *h, const float *logits, int32_t n_rows, int32_t vocab, 
     if (rc) return rc;
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1, RLX_TIME_SELECT))) return rc;
-    HIP_TRY(launch_greedy(c->stream, logits, row_stride, vocab, n_rows, (int32_t *)c->ws, e0, e1));
-    HIP_TRY(hipMemcpyAsync(out_tokens, c->ws, (size_t)n_rows * 4, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(launch_greedy(c->stream, logits, row_stride, vocab, n_rows, (int32_t *)c->ws.ptr, e0, e1));
+    HIP_TRY(hipMemcpyAsync(out_tokens, c->ws.ptr, (size_t)n_rows * 4, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return RLX_OK;
 }
@@ -3092,11 +3103,11 @@ int32_t rlx_sample(void *h, const float *logits, int32_t n_rows, int32_t vocab, 
     a.seen_freq = pen ? (const int32_t *)(d + o_f) : nullptr;
     a.seen_off = pen ? (const int32_t *)(d + o_o) : nullptr;
     a.u = (const float *)(d + o_u);
-    a.out = (int32_t *)c->ws;
+    a.out = (int32_t *)c->ws.ptr;
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1, RLX_TIME_SELECT))) return rc;
     HIP_TRY(launch_sample(c->stream, a, n_rows, e0, e1));
-    HIP_TRY(hipMemcpyAsync(out_tokens, c->ws, (size_t)n_rows * 4, hipMemcpyDeviceToHost, c->stream));
+    HIP_TRY(hipMemcpyAsync(out_tokens, c->ws.ptr, (size_t)n_rows * 4, hipMemcpyDeviceToHost, c->stream));
     HIP_TRY(hipStreamSynchronize(c->stream));
     return RLX_OK;
 }
@@ -3187,7 +3198,7 @@ int32_t rlx_spec_accept_async(void *h, const float *draft_logits, const float *t
                     vocab);
     int32_t rc = ensure_ws(c, (size_t)ws_bytes);
     if (rc) return rc;
-    plan_spec_split(a, n_rows, (char *)c->ws);
+    plan_spec_split(a, n_rows, (char *)c->ws.ptr);
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1, RLX_TIME_SELECT))) return rc;
     HIP_TRY(launch_spec_accept(c->stream, a, n_rows, e0, e1));
@@ -3232,7 +3243,7 @@ int32_t rlx_spec_accept(void *h, const float *draft_logits, const float *target_
         return fail(RLX_ERR_UNSUPPORTED, "rlx_spec_accept: max_k=%d at vocab %d exceeds the grid", max_k, vocab);
     int32_t rc = ensure_ws(c, o_split + (size_t)split_bytes);
     if (rc) return rc;
-    plan_spec_split(a, n_rows, (char *)c->ws + o_split);
+    plan_spec_split(a, n_rows, (char *)c->ws.ptr + o_split);
     if ((rc = stage(c, bl.bytes.data(), bl.bytes.size(), &dev))) return rc;
     char *d = (char *)dev;
     a.d_logits = draft_logits;
@@ -3246,8 +3257,8 @@ int32_t rlx_spec_accept(void *h, const float *draft_logits, const float *target_
     a.top_k = p->top_k;
     a.top_p = p->top_p;
     a.min_p = p->min_p;
-    a.n_acc = (int32_t *)c->ws;
-    a.next = (int32_t *)c->ws + n_rows;
+    a.n_acc = (int32_t *)c->ws.ptr;
+    a.next = (int32_t *)c->ws.ptr + n_rows;
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1, RLX_TIME_SELECT))) return rc;
     HIP_TRY(launch_spec_accept(c->stream, a, n_rows, e0, e1));

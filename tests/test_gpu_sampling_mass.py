@@ -98,8 +98,9 @@ def test_split_rows_past_the_scratch(gpu, handles, monkeypatch):
 
 @pytest.mark.parametrize("grown", [False, True])
 def test_split_under_capture(gpu, grown):
-    """A captured call allocates nothing: the whole-row path until the
-    workspace is there, the split after; replays follow their draws."""
+    """A captured call allocates nothing and holds no scratch: the whole-row
+    path, whether the split's workspace is there or not; replays follow their
+    draws."""
     from relux_amd import KVCache, Sampler
     g = torch.Generator(device=gpu).manual_seed(9)
     B, V = 4, 40000
