@@ -159,8 +159,14 @@ int32_t rlx_cache_set_stream(void *cache, void *stream);
  * at least staging_bytes and the adapter buffer (rows of a head_dim, d_model
  * or k_in that the kernels take padded) to at least adapter_bytes now, so
  * that a serving loop pays for it once at set-up; a size the current
- * capacity covers leaves it unchanged.  No reference counterpart: the
- * reference's scratch is Go heap memory. */
+ * capacity covers leaves it unchanged.  After it the workspace no longer
+ * grows for scratch that a call can do without, which runs without it
+ * instead: chunked prefill of few query tiles cuts them along the keys with
+ * up to 64 MiB of partial sums (behind the expanded latents, for MLA), and
+ * sampling without top-k on more than 12288 entries splits rows with up to
+ * 64 MiB -- reserve that much more where such calls are to run at full
+ * speed.  No reference counterpart: the reference's scratch is Go heap
+ * memory. */
 int32_t rlx_cache_reserve(void *cache, uint64_t workspace_bytes, uint64_t staging_bytes,
                           uint64_t adapter_bytes);
 /* out[0] workspace capacity, out[1] the largest workspace any call on the
@@ -168,7 +174,8 @@ int32_t rlx_cache_reserve(void *cache, uint64_t workspace_bytes, uint64_t stagin
  * capacity, out[3] the largest plan any call has staged, out[4] adapter
  * capacity, out[5] the largest adapter request (bytes).  A trial run of the
  * largest calls followed by rlx_cache_reserve(out[1], out[3], out[5]) on a
- * fresh handle keeps every later call of those sizes from allocating. */
+ * fresh handle keeps every later call of those sizes, and smaller ones, from
+ * allocating. */
 int32_t rlx_cache_memory(void *cache, uint64_t *out);
 
 /* ---- append (scatter into pages) -------------------------------------- */
@@ -481,9 +488,10 @@ int32_t rlx_sample(void *cache, const float *logits, int32_t n_rows, int32_t voc
  * needs a larger cache workspace (the split paths' chunk lists, top-k in
  * (0, 256] past 8192 entries, or no top-k past 12288: at most 64 MiB),
  * which synchronises the stream and allocates it once.  Without top-k a
- * call runs its rows unsplit where there is no memory for it, and always on
- * a stream under capture, so that its graph holds no scratch.  Same tokens
- * as rlx_sample given the same windows and draws. */
+ * call runs its rows unsplit where there is no such workspace (a
+ * reservation without room for it, no memory) and always on a stream under
+ * capture, so that its graph holds no scratch.  Same tokens as rlx_sample
+ * given the same windows and draws. */
 int32_t rlx_sample_async(void *cache, const float *logits, int32_t n_rows, int32_t vocab,
                          int64_t row_stride, const rlx_sampler_t *params, const int32_t *history,
                          int64_t hist_stride, const int32_t *hist_len, const float *uniforms,

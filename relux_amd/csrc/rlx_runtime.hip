@@ -325,7 +325,7 @@ int32_t ensure_ws(Cache *c, size_t bytes) {
 }
 
 // A workspace of `bytes` that a call can do without: false where it cannot
-// grow (a cap, no memory), and on a stream under capture, where
+// grow (a cap, a reservation, no memory), and on a stream under capture, where
 // a graph would keep the scratch of a call that needs none.
 bool optional_ws(Cache *c, size_t bytes) {
     long long kb;

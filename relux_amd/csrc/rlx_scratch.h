@@ -25,6 +25,7 @@ struct Scratch {
     size_t peak = 0;               // largest request so far
     size_t refused = 0;            // smallest optional request the allocator refused (0: none)
     bool held = false;             // a captured graph may hold ptr
+    bool reserved = false;         // sized ahead of time: optional requests do not grow it
     std::vector<void *> retired;   // superseded buffers a captured graph may hold
 
     // Growth to `bytes` for a call that needs them.
@@ -42,7 +43,7 @@ struct Scratch {
     bool want(Mem &m, size_t bytes) {
         peak = std::max(peak, bytes);
         if (bytes <= cap) return true;
-        if (refused && bytes >= refused) return false;
+        if (reserved || (refused && bytes >= refused)) return false;
         const size_t n = round(std::max(bytes, std::min(2 * cap, kOptionalDouble)));
         if (!m.sync()) return false;
         void *p = m.get(n);
@@ -54,10 +55,15 @@ struct Scratch {
         return true;
     }
 
-    // At least `bytes` from now on.
+    // At least `bytes` from now on, and no optional growth after it.
     template <class Mem>
     Grow reserve(Mem &m, size_t bytes) {
-        return bytes > cap ? grow(m, bytes, bytes) : Grow::kOk;
+        if (bytes > cap) {
+            const Grow g = grow(m, bytes, bytes);
+            if (g != Grow::kOk) return g;
+        }
+        reserved = true;
+        return Grow::kOk;
     }
 
     template <class Mem>

@@ -136,12 +136,32 @@ static int last_resort() {
     return 0;
 }
 
+// A reserved buffer does not grow for an optional request; it still counts it.
+static int reserved() {
+    Mem m;
+    Scratch s;
+    CHECK(s.want(m, MB));
+    CHECK(s.reserve(m, 8 * MB) == Grow::kOk && s.cap == 8 * MB && s.peak == MB);
+    const int gets = m.gets;
+    CHECK(s.want(m, 8 * MB) && !s.want(m, 9 * MB) && m.gets == gets);
+    CHECK(s.peak == 9 * MB);
+    CHECK(s.need(m, 10 * MB) == Grow::kOk);  // (a call that needs it)
+    CHECK(s.reserve(m, 2 * MB) == Grow::kOk && s.cap >= 10 * MB);
+    m.limit = 0;
+    const size_t cap = s.cap;
+    s.held = true;
+    CHECK(s.reserve(m, 100 * MB) == Grow::kMemory && s.cap == cap && s.ptr);
+    Scratch none;  // calls that need no workspace reserve none
+    CHECK(none.reserve(m, 0) == Grow::kOk && !none.want(m, MB) && none.cap == 0);
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         int (*run)();
     } all[] = {{"held", held},         {"refused", refused},   {"no_doubling", no_doubling},
-               {"last_resort", last_resort}};
+               {"last_resort", last_resort}, {"reserved", reserved}};
     for (auto &t : all)
         if (argc > 1 && !std::strcmp(argv[1], t.name)) return t.run();
     return 2;

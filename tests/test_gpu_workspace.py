@@ -1,6 +1,7 @@
-"""The workspace of a handle under graphs: scratch that a captured call holds
-outlives every later growth, and a captured call that can do without scratch
-holds none."""
+"""The workspace of a handle under graphs and reservations: scratch that a
+captured call holds outlives every later growth, a captured call that can do
+without scratch holds none, and a reserved handle does not grow for a call
+that can do without."""
 import pytest
 import torch
 
@@ -83,3 +84,33 @@ def test_scratch_of_a_captured_call(gpu, kw, holds):
     before = _used()
     c.close()
     assert before - _used() >= new - SLACK
+
+
+def test_reserved_handle_does_not_grow_for_optional_scratch(gpu):
+    """A trial run of the largest call gives the sizes to reserve, and no call
+    of those sizes allocates after: a prefill that fills the chip takes no
+    scratch, and a smaller one then takes none either."""
+    g = torch.Generator(device=gpu).manual_seed(5)
+    H, KVH, D, T = 32, 8, 128, 4096
+    k, v = (torch.randn(T, KVH, D, device=gpu, generator=g).bfloat16() for _ in range(2))
+    q = torch.randn(T, H, D, device=gpu, generator=g).bfloat16()
+
+    def prefill(c, n):
+        c.Append(0, k[:n], v[:n], seq_ids=[0], n_tok=[n], layout="SHD")
+        o = c.Attend(0, q[:n].contiguous(), H, seq_ids=[0], n_q=[n])
+        c.Rollback([0], [n])
+        return o
+
+    trial, served, free = (_handle(gpu, max_len=T, num_kv_heads=KVH, head_dim=D) for _ in range(3))
+    prefill(trial, T)
+    st = trial.MemoryStats()
+    served.Reserve(st["workspace_peak"], st["staging_peak"], st["adapter_peak"])
+    before = served.MemoryStats()
+    got, want = prefill(served, 1100), prefill(free, 1100)
+    prefill(served, T)
+    assert free.MemoryStats()["workspace"] > 0, "the smaller call has no optional scratch: choose another"
+    after = served.MemoryStats()
+    assert after["workspace"] == before["workspace"] and after["staging"] == before["staging"]
+    assert after["workspace_peak"] == free.MemoryStats()["workspace_peak"]  # what to reserve for it
+    e = (got.double() - want.double()).abs()
+    assert float(e.max()) <= 1e-2 and float(e.mean()) <= 1e-3

@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["held", "refused", "no_doubling", "last_resort"])
+@pytest.mark.parametrize("scenario", ["held", "refused", "no_doubling", "last_resort", "reserved"])
 def test_scratch(program, scenario):
     r = subprocess.run([program, scenario], stdout=subprocess.PIPE, text=True)
     assert r.returncode == 0, r.stdout
