@@ -89,9 +89,7 @@ struct LayerState {
 };
 
 struct Slot {
-    void *host = nullptr;
-    void *dev = nullptr;
-    size_t cap = 0;
+    StagePair buf;
     hipEvent_t ev = nullptr;
     bool pending = false;
 };
@@ -160,6 +158,11 @@ struct HipMem {
         return checked(hipMalloc(&p, n)) ? p : nullptr;
     }
     void put(void *p) { (void)hipFree(p); }
+    void *get_host(size_t n) {
+        void *p = nullptr;
+        return checked(hipHostMalloc(&p, n, hipHostMallocDefault)) ? p : nullptr;
+    }
+    void put_host(void *p) { (void)hipHostFree(p); }
     bool sync() { return checked(hipStreamSynchronize(stream)); }
 
 private:
@@ -185,26 +188,19 @@ int32_t stage(Cache *c, const void *data, size_t bytes, void **dev_out) {
         HIP_TRY(hipEventSynchronize(s.ev));
         s.pending = false;
     }
-    if (bytes > s.cap) {
-        size_t cap = std::max<size_t>(bytes, 64 * 1024);
-        cap = (cap + 4095) & ~(size_t)4095;
-        // The device copy of this slot may still be read by queued kernels.
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        if (s.host) HIP_TRY(hipHostFree(s.host));
-        if (s.dev) HIP_TRY(hipFree(s.dev));
-        s.host = nullptr;
-        s.dev = nullptr;
-        HIP_TRY(hipHostMalloc(&s.host, cap, hipHostMallocDefault));
-        HIP_TRY(hipMalloc(&s.dev, cap));
-        s.cap = cap;
+    if (bytes > s.buf.cap) {
+        HipMem m{c->stream};
+        const size_t cap = std::max<size_t>(bytes, 64 * 1024);
+        const int32_t rc = grown(s.buf.grow(m, cap), "staging slot", cap);
+        if (rc) return rc;
     }
     if (bytes) {
-        memcpy(s.host, data, bytes);
-        HIP_TRY(hipMemcpyAsync(s.dev, s.host, bytes, hipMemcpyHostToDevice, c->stream));
+        memcpy(s.buf.host, data, bytes);
+        HIP_TRY(hipMemcpyAsync(s.buf.dev, s.buf.host, bytes, hipMemcpyHostToDevice, c->stream));
         HIP_TRY(hipEventRecord(s.ev, c->stream));
         s.pending = true;
     }
-    *dev_out = s.dev;
+    *dev_out = s.buf.dev;
     return RLX_OK;
 }
 
@@ -447,8 +443,7 @@ void destroy_cache(Cache *c) {
         (void)hipEventDestroy(p.second);
     }
     for (auto &s : c->slots) {
-        if (s.host) (void)hipHostFree(s.host);
-        if (s.dev) (void)hipFree(s.dev);
+        s.buf.release(mem);
         if (s.ev) (void)hipEventDestroy(s.ev);
     }
     if (c->spill.base) {
@@ -1178,19 +1173,7 @@ int32_t rlx_cache_reserve(void *h, uint64_t ws_bytes, uint64_t stage_bytes, uint
     if ((rc = grown(c->ws.reserve(m, ws_bytes), "workspace", ws_bytes))) return rc;
     if ((rc = grown(c->ad.reserve(m, ad_bytes), "adapter buffer", ad_bytes))) return rc;
     for (Slot &s : c->slots) {
-        if (stage_bytes <= s.cap) continue;
-        const size_t cap = ((size_t)stage_bytes + 4095) & ~(size_t)4095;
-        // The slot's device copy may still be read by queued kernels.
-        HIP_TRY(hipStreamSynchronize(c->stream));
-        s.pending = false;
-        if (s.host) HIP_TRY(hipHostFree(s.host));
-        if (s.dev) HIP_TRY(hipFree(s.dev));
-        s.host = nullptr;
-        s.dev = nullptr;
-        s.cap = 0;
-        HIP_TRY(hipHostMalloc(&s.host, cap, hipHostMallocDefault));
-        HIP_TRY(hipMalloc(&s.dev, cap));
-        s.cap = cap;
+        if ((rc = grown(s.buf.grow(m, stage_bytes), "staging slot", stage_bytes))) return rc;
     }
     return RLX_OK;
 }
@@ -1198,8 +1181,8 @@ int32_t rlx_cache_reserve(void *h, uint64_t ws_bytes, uint64_t stage_bytes, uint
 int32_t rlx_cache_memory(void *h, uint64_t *out) {
     if (!h || !out) return fail(RLX_ERR_INVALID, "null argument");
     const Cache *c = as_cache(h);
-    size_t smin = c->slots[0].cap;
-    for (const Slot &s : c->slots) smin = std::min(smin, s.cap);
+    size_t smin = c->slots[0].buf.cap;
+    for (const Slot &s : c->slots) smin = std::min(smin, s.buf.cap);
     out[0] = c->ws.cap;
     out[1] = c->ws.peak;
     out[2] = smin;

@@ -1,7 +1,8 @@
-// Growable buffers of a handle: the device scratch its calls share and the
-// adapter rows.  Host code over an allocator the runtime supplies (Mem: get /
-// put device memory -- null when refused -- and sync, which waits for the
-// handle's queued work), so that the rules can be tested without a device.
+// Growable buffers of a handle: the device scratch its calls share, the
+// adapter rows, and the staging slots.  Host code over an allocator the
+// runtime supplies (Mem: get / put device memory, get_host / put_host pinned
+// memory -- null when refused -- and sync, which waits for the handle's
+// queued work), so that the rules can be tested without a device.
 //
 // The rules: a buffer that fits is replaced only once its successor is there,
 // and a buffer whose address a captured graph may hold is never given back
@@ -110,6 +111,40 @@ private:
         cap = n;
         refused = 0;
         held = false;
+    }
+};
+
+// A staging slot's pair of buffers (pinned host, device) of one capacity.
+struct StagePair {
+    void *host = nullptr;
+    void *dev = nullptr;
+    size_t cap = 0;
+
+    // Growth to `bytes`; on failure the pair there was stays.
+    template <class Mem>
+    Grow grow(Mem &m, size_t bytes) {
+        if (bytes <= cap) return Grow::kOk;
+        // The device copy may still be read by queued kernels.
+        if (!m.sync()) return Grow::kSync;
+        const size_t n = (bytes + 4095) & ~(size_t)4095;
+        void *h = m.get_host(n), *d = h ? m.get(n) : nullptr;
+        if (!d) {
+            if (h) m.put_host(h);
+            return Grow::kMemory;
+        }
+        release(m);
+        host = h;
+        dev = d;
+        cap = n;
+        return Grow::kOk;
+    }
+
+    template <class Mem>
+    void release(Mem &m) {
+        if (host) m.put_host(host);
+        if (dev) m.put(dev);
+        host = dev = nullptr;
+        cap = 0;
     }
 };
 

@@ -11,11 +11,12 @@
 
 using rlx::Grow;
 using rlx::Scratch;
+using rlx::StagePair;
 
 struct Mem {
-    std::map<void *, size_t> live;
+    std::map<void *, size_t> live, host;
     size_t limit = (size_t)1 << 40;  // device bytes that may be alive at once
-    bool sync_ok = true;
+    bool host_ok = true, sync_ok = true;
     int gets = 0, puts = 0, syncs = 0;
     uintptr_t next = 0x1000;
     size_t used() const {
@@ -33,6 +34,15 @@ struct Mem {
     void put(void *p) {
         puts++;
         if (!live.erase(p)) std::abort();  // not alive: freed twice
+    }
+    void *get_host(size_t n) {
+        if (!host_ok) return nullptr;
+        void *p = (void *)(next += 0x1000);
+        host[p] = n;
+        return p;
+    }
+    void put_host(void *p) {
+        if (!host.erase(p)) std::abort();
     }
     bool sync() {
         syncs++;
@@ -156,12 +166,37 @@ static int reserved() {
     return 0;
 }
 
+// A staging slot whose growth fails keeps its pair and the capacity that goes
+// with it; the next plans that fit are copied into live buffers.
+static int stage() {
+    Mem m;
+    StagePair s;
+    CHECK(s.grow(m, 65536) == Grow::kOk && s.cap == 65536);
+    void *h = s.host, *d = s.dev;
+    m.limit = 65536;  // the device half
+    CHECK(s.grow(m, 200000) == Grow::kMemory);
+    CHECK(s.host == h && s.dev == d && s.cap == 65536 && m.host.count(h) && m.live.count(d));
+    CHECK(m.host.size() == 1);
+    m.limit = 10 * MB;
+    m.host_ok = false;  // the pinned half
+    CHECK(s.grow(m, 200000) == Grow::kMemory && s.host == h && s.dev == d && s.cap == 65536);
+    m.host_ok = true;
+    CHECK(s.grow(m, 200000) == Grow::kOk && s.cap >= 200000 && !m.host.count(h) && !m.live.count(d));
+    s.release(m);
+    CHECK(m.host.empty() && m.live.empty() && s.cap == 0);
+    // a first growth that fails leaves nothing to copy into, and says so
+    StagePair e;
+    m.limit = 0;
+    CHECK(e.grow(m, 100) == Grow::kMemory && e.cap == 0 && !e.host && m.host.empty());
+    return 0;
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         int (*run)();
     } all[] = {{"held", held},         {"refused", refused},   {"no_doubling", no_doubling},
-               {"last_resort", last_resort}, {"reserved", reserved}};
+               {"last_resort", last_resort}, {"reserved", reserved}, {"stage", stage}};
     for (auto &t : all)
         if (argc > 1 && !std::strcmp(argv[1], t.name)) return t.run();
     return 2;

@@ -1,4 +1,4 @@
-"""The growth rules of a handle's workspace and adapter buffer
+"""The growth rules of a handle's workspace, adapter buffer and staging slots
 (relux_amd/csrc/rlx_scratch.h) on the CPU, over an allocator that refuses on
 demand: tests/scratch_host.cpp holds the scenarios."""
 import os
@@ -18,7 +18,7 @@ def program(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("scenario", ["held", "refused", "no_doubling", "last_resort", "reserved"])
+@pytest.mark.parametrize("scenario", ["held", "refused", "no_doubling", "last_resort", "reserved", "stage"])
 def test_scratch(program, scenario):
     r = subprocess.run([program, scenario], stdout=subprocess.PIPE, text=True)
     assert r.returncode == 0, r.stdout
