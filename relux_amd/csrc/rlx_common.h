@@ -742,13 +742,15 @@ hipError_t launch_proj_gemm(hipStream_t s, int model, const Patch *patches, int 
 // Work-groups of the decode kernels one CU holds at once (occupancy).
 int mla_decode_wgs_per_cu(int nqt);
 
+// p32: the split partials (part_o) as f32 instead of bf16; head dim 128 and
+// head groups of 32 rows only.
 hipError_t launch_mla_decode(hipStream_t s, const PlanArg *plan, const uint16_t *pool,
                              const int32_t *table, const AttRow *rows, int n_rows,
                              const int2 *work, int n_work,
                              const void *q_nope, const void *q_rope, int q_bf16,
                              const uint16_t *w_uk, const uint16_t *w_uv, int H, int hd, int dc,
                              int dr, int total_q, int max_nq, int P, float qscale,
-                             int mask_mode, int nqt, uint16_t *qlat, uint16_t *part_o,
+                             int mask_mode, int nqt, uint16_t *qlat, bool p32, void *part_o,
                              float *part_ml, void *out, int out_bf16, int cus,
                              hipEvent_t ev0, hipEvent_t ev1, const MlaAppendJob *app = nullptr);
 

@@ -21,6 +21,7 @@
 #include "rlx_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace rlx {
 
@@ -195,16 +196,19 @@ template <int NQT> struct MlaShape {
     static constexpr int CH = kMlaDc / NW;            // latent channels per wave
 };
 
+template <bool P32> using MlaPart = std::conditional_t<P32, float, uint16_t>;  // a split partial's element
+
 // KEEP: ring loads without the non-temporal hint, for calls whose head
 // groups re-read the same latent rows (they then meet them in L2: 128 heads
 // at 8k, 66.4 -> 61.3 us); single-group calls keep the hint (config 3:
 // 53.0 against 58.0 us without it).
-template <int NQT, bool ARG, bool KEEP>
+// P32: the split partials leave as f32 (launch_mla_decode).
+template <int NQT, bool ARG, bool KEEP, bool P32>
 __global__ __launch_bounds__(64 * MlaShape<NQT>::NW, MlaShape<NQT>::WGS) void mla_decode_kernel(
     typename PlanSel<ARG>::T plan, const uint16_t *__restrict__ pool,
     const int32_t *__restrict__ table, const AttRow *__restrict__ rows,
     const int2 *__restrict__ work, int n_rows, const uint16_t *__restrict__ qlat, int H, int P,
-    int mask_mode, uint16_t *__restrict__ part_o, float *__restrict__ part_ml) {
+    int mask_mode, MlaPart<P32> *__restrict__ part_o, float *__restrict__ part_ml) {
     using SH = MlaShape<NQT>;
     constexpr int NW = SH::NW, S = SH::S, CH = SH::CH, MT = CH / 16;
     constexpr int QRP = 16 * NQT;
@@ -482,33 +486,42 @@ __global__ __launch_bounds__(64 * MlaShape<NQT>::NW, MlaShape<NQT>::WGS) void ml
 
     const int pidx = R.part + wk.y;
     // The unnormalised latent partial is stored as bf16 (the merge weighs
-    // and sums it in f32).  A lane's accumulators hold 4 channels of one
-    // query row, so stored as they are, each store instruction would write
-    // 16 pieces of 32 bytes, 1 KB apart; the wave's 128 channels x 16 rows
-    // go through LDS instead (the ring, free once every wave is past its
+    // and sums it in f32), or as it is (P32: 16 pieces of 64 bytes a store).
+    // A lane's accumulators hold 4 channels of one query row, so the bf16
+    // pieces would be of 32 bytes, 1 KB apart; the wave's 128 channels x 16
+    // rows go through LDS instead (the ring, free once every wave is past its
     // last tile; rows padded by 16 bytes against bank conflicts) and leave
     // as 256 contiguous bytes per query row.
     constexpr int SP = CH + 8;  // staging row pitch, bf16
     static_assert(NW * NQT * 16 * SP <= S * TILE, "the staging rows fit the ring");
-    __syncthreads();
     uint16_t *stg = ring + wave * NQT * 16 * SP;
+    if constexpr (!P32) {
+        __syncthreads();
 #pragma unroll
-    for (int nt = 0; nt < NQT; nt++)
+        for (int nt = 0; nt < NQT; nt++)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            const u32x2 pk = {pack_bf16x2(acc[nt][mt][0], acc[nt][mt][1]),
-                              pack_bf16x2(acc[nt][mt][2], acc[nt][mt][3])};
-            *(u32x2 *)(stg + (nt * 16 + col) * SP + mt * 16 + grp * 4) = pk;
-        }
-    __syncthreads();
+            for (int mt = 0; mt < MT; mt++) {
+                const u32x2 pk = {pack_bf16x2(acc[nt][mt][0], acc[nt][mt][1]),
+                                  pack_bf16x2(acc[nt][mt][2], acc[nt][mt][3])};
+                *(u32x2 *)(stg + (nt * 16 + col) * SP + mt * 16 + grp * 4) = pk;
+            }
+        __syncthreads();
+    }
 #pragma unroll
     for (int nt = 0; nt < NQT; nt++) {
+        if constexpr (P32) {
 #pragma unroll
-        for (int it = 0; it < 4; it++) {
-            const int r = it * 4 + (lane >> 4), ch = (lane & 15) * 8;
-            const u32x4 v = *(const u32x4 *)(stg + (nt * 16 + r) * SP + ch);
-            __builtin_nontemporal_store(
-                v, (u32x4 *)(part_o + ((int64_t)pidx * QRP + nt * 16 + r) * kMlaDc + wave * CH + ch));
+            for (int mt = 0; mt < MT; mt++)
+                *(fl4 *)(part_o + ((int64_t)pidx * QRP + nt * 16 + col) * kMlaDc + wave * CH + mt * 16 + grp * 4) =
+                    acc[nt][mt];
+        } else {
+#pragma unroll
+            for (int it = 0; it < 4; it++) {
+                const int r = it * 4 + (lane >> 4), ch = (lane & 15) * 8;
+                const u32x4 v = *(const u32x4 *)(stg + (nt * 16 + r) * SP + ch);
+                __builtin_nontemporal_store(
+                    v, (u32x4 *)(part_o + ((int64_t)pidx * QRP + nt * 16 + r) * kMlaDc + wave * CH + ch));
+            }
         }
         const int qr = nt * 16 + col;
         const float lt = rows4_sum(l_part[nt]);
@@ -769,10 +782,10 @@ __global__ __launch_bounds__(256) void mla_out_kernel(
 // (m, l) pairs, the split partials, then the W_UV slice (into registers);
 // the slice goes to LDS after the merge, so the merge waits only for the
 // partials.
-template <int RPB, bool ARG>
+template <int RPB, bool ARG, bool P32>
 __global__ __launch_bounds__(256) void mla_out_mfma_kernel(
     typename PlanSel<ARG>::T plan, const AttRow *__restrict__ rows, int n_rows, int total_q, int one_q,
-    const uint16_t *__restrict__ part_o, const float *__restrict__ part_ml,
+    const MlaPart<P32> *__restrict__ part_o, const float *__restrict__ part_ml,
     const uint16_t *__restrict__ w_uv, int H, int dc, int QRP, void *__restrict__ out, int out_bf16) {
     constexpr int D = 128;                     // head dim
     constexpr int WD = D / 4;                  // output dims per wave
@@ -815,12 +828,13 @@ __global__ __launch_bounds__(256) void mla_out_mfma_kernel(
     float2 ml0 = make_float2(-INFINITY, 0.f);
     if (wave < RPB) ml0 = ml[min(lane, nw - 1) * st];
     const int64_t sstride = (int64_t)QRP * kMlaDc;
-    uint32_t v[RPB][SB];
+    using Pair = std::conditional_t<P32, float2, uint32_t>;  // a lane's two channels of a split
+    Pair v[RPB][SB];
 #pragma unroll
     for (int j = 0; j < RPB; j++) {
-        const uint16_t *src = part_o + b0[j] * kMlaDc + 2 * t;
+        const MlaPart<P32> *src = part_o + b0[j] * kMlaDc + 2 * t;
 #pragma unroll
-        for (int i = 0; i < SB; i++) v[j][i] = *(const uint32_t *)(src + (int64_t)min(i, ns[j] - 1) * sstride);
+        for (int i = 0; i < SB; i++) v[j][i] = *(const Pair *)(src + (int64_t)min(i, ns[j] - 1) * sstride);
     }
     // Slice load k of this lane: channel 128 wave + 4k + lane / 16,
     // 16-byte chunk lane % 16 of the head's 128 dims.  Channels past d_c
@@ -871,18 +885,23 @@ __global__ __launch_bounds__(256) void mla_out_mfma_kernel(
 #pragma unroll
         for (int i = 0; i < SB; i++) {
             const float f = f4[i / 4][i % 4];
-            o0 += f * bf16_lo(v[j][i]);
-            o1 += f * bf16_hi(v[j][i]);
+            if constexpr (P32) {
+                o0 += f * v[j][i].x;
+                o1 += f * v[j][i].y;
+            } else {
+                o0 += f * bf16_lo(v[j][i]);
+                o1 += f * bf16_hi(v[j][i]);
+            }
         }
     };
 #pragma unroll
     for (int j = 0; j < RPB; j++) {
-        const uint16_t *src = part_o + b0[j] * kMlaDc + 2 * t;
+        const MlaPart<P32> *src = part_o + b0[j] * kMlaDc + 2 * t;
         float o0 = 0.f, o1 = 0.f;
         merge_batch(j, 0, o0, o1);
         for (int s0 = SB; s0 < ns[j]; s0 += SB) {
 #pragma unroll
-            for (int i = 0; i < SB; i++) v[j][i] = *(const uint32_t *)(src + (int64_t)min(s0 + i, ns[j] - 1) * sstride);
+            for (int i = 0; i < SB; i++) v[j][i] = *(const Pair *)(src + (int64_t)min(s0 + i, ns[j] - 1) * sstride);
             merge_batch(j, s0, o0, o1);
         }
         uint16_t h0, l0, h1, l1;
@@ -954,14 +973,21 @@ __global__ __launch_bounds__(256) void mla_out_mfma_kernel(
 }
 
 template <int NQT, bool ARG>
-static void launch_mla_t(hipStream_t s, bool keep, typename PlanSel<ARG>::T plan, const uint16_t *pool,
+static void launch_mla_t(hipStream_t s, bool keep, bool p32, typename PlanSel<ARG>::T plan, const uint16_t *pool,
                          const int32_t *table, const AttRow *rows, int n_rows, const int2 *work,
                          int n_work, const uint16_t *qlat, int H, int P, int mask_mode,
-                         uint16_t *part_o, float *part_ml, hipEvent_t ev0, hipEvent_t ev1) {
-    (void)launch_timed(keep ? mla_decode_kernel<NQT, ARG, true> : mla_decode_kernel<NQT, ARG, false>,
-                       dim3(n_work), dim3(64 * MlaShape<NQT>::NW), s,
-                       ev0, ev1, plan, pool, table, rows, work, n_rows, qlat, H, P, mask_mode,
-                       part_o, part_ml);
+                         void *part_o, float *part_ml, hipEvent_t ev0, hipEvent_t ev1) {
+    const dim3 g(n_work), b(64 * MlaShape<NQT>::NW);
+    if constexpr (NQT == 2) {
+        if (p32) {
+            (void)launch_timed(mla_decode_kernel<2, ARG, true, true>, g, b, s, ev0, ev1, plan, pool, table, rows,
+                               work, n_rows, qlat, H, P, mask_mode, (float *)part_o, part_ml);
+            return;
+        }
+    }
+    (void)launch_timed(keep ? mla_decode_kernel<NQT, ARG, true, false> : mla_decode_kernel<NQT, ARG, false, false>,
+                       g, b, s, ev0, ev1, plan, pool, table, rows, work, n_rows, qlat, H, P, mask_mode,
+                       (uint16_t *)part_o, part_ml);
 }
 
 template <int DMAX, bool ARG>
@@ -982,8 +1008,8 @@ static void launch_mla_out_d(hipStream_t s, typename PlanSel<ARG>::T plan, const
 }
 
 template <bool ARG>
-static void launch_mla_out(hipStream_t s, typename PlanSel<ARG>::T plan, const AttRow *rows,
-                           int n_rows, int total_q, int one_q, const uint16_t *part_o, const float *part_ml,
+static void launch_mla_out(hipStream_t s, bool p32, typename PlanSel<ARG>::T plan, const AttRow *rows,
+                           int n_rows, int total_q, int one_q, const void *parts, const float *part_ml,
                            const uint16_t *w_uv, int H, int hd, int dc, int QRP, void *out,
                            int out_bf16, int cus) {
     // Rows per block: the most (4, 2, 1) that still give every CU a block;
@@ -996,22 +1022,26 @@ static void launch_mla_out(hipStream_t s, typename PlanSel<ARG>::T plan, const A
         const int x = e ? atoi(e) : 0;
         return (x == 1 || x == 2 || x == 4) ? x : 0;
     }();
-    if (hd == 128) {
+    const uint16_t *part_o = (const uint16_t *)parts;
+    if (p32) {  // (past 1024 query rows: 4 a block fill the CUs)
+        mla_out_mfma_kernel<4, ARG, true><<<dim3(H, (total_q + 3) / 4), 256, 0, s>>>(
+            plan, rows, n_rows, total_q, one_q, (const float *)parts, part_ml, w_uv, H, dc, QRP, out, out_bf16);
+    } else if (hd == 128) {
         int rpb = rpb_override;
         if (!rpb)
             rpb = (int64_t)H * ((total_q + 3) / 4) >= cus   ? 4
                   : (int64_t)H * ((total_q + 1) / 2) >= cus ? 2
                                                             : 1;
         if (rpb == 4)
-            mla_out_mfma_kernel<4, ARG><<<dim3(H, (total_q + 3) / 4), 256, 0, s>>>(
+            mla_out_mfma_kernel<4, ARG, false><<<dim3(H, (total_q + 3) / 4), 256, 0, s>>>(
                 plan, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, dc, QRP,
                 out, out_bf16);
         else if (rpb == 2)
-            mla_out_mfma_kernel<2, ARG><<<dim3(H, (total_q + 1) / 2), 256, 0, s>>>(
+            mla_out_mfma_kernel<2, ARG, false><<<dim3(H, (total_q + 1) / 2), 256, 0, s>>>(
                 plan, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, dc, QRP,
                 out, out_bf16);
         else
-            mla_out_mfma_kernel<1, ARG><<<dim3(H, total_q), 256, 0, s>>>(
+            mla_out_mfma_kernel<1, ARG, false><<<dim3(H, total_q), 256, 0, s>>>(
                 plan, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, dc, QRP,
                 out, out_bf16);
     } else if (hd <= 32)
@@ -1030,11 +1060,12 @@ hipError_t launch_mla_decode(hipStream_t s, const PlanArg *plan, const uint16_t 
                              const void *q_nope, const void *q_rope, int q_bf16,
                              const uint16_t *w_uk, const uint16_t *w_uv, int H, int hd, int dc,
                              int dr, int total_q, int max_nq, int P, float qscale,
-                             int mask_mode, int nqt, uint16_t *qlat, uint16_t *part_o,
+                             int mask_mode, int nqt, uint16_t *qlat, bool p32, void *part_o,
                              float *part_ml, void *out, int out_bf16, int cus,
                              hipEvent_t ev0, hipEvent_t ev1, const MlaAppendJob *app) {
     if (n_work <= 0) return hipSuccess;
     if (hd > 256 || hd % 8 != 0 || dc > kMlaDc || dr > kMlaDr) return hipErrorInvalidValue;
+    if (p32 && (hd != 128 || nqt != 2 || H * max_nq <= 32)) return hipErrorInvalidValue;
     const int nz = (total_q + 15) / 16;
     const dim3 ag(H, kMlaDc / 64, nz);
     if (app && (app->n_tok > 0 || app->n_patch > 0)) {
@@ -1077,16 +1108,16 @@ hipError_t launch_mla_decode(hipStream_t s, const PlanArg *plan, const uint16_t 
     // latent rows: keep them in L2
     const bool keep = H * max_nq > 16 * nqt;
     if (plan && nqt == 1)
-        launch_mla_t<1, true>(s, keep, *plan, pool, table, rows, n_rows, work, n_work, qlat, H, P,
+        launch_mla_t<1, true>(s, keep, p32, *plan, pool, table, rows, n_rows, work, n_work, qlat, H, P,
                               mask_mode, part_o, part_ml, ev0, ev1);
     else if (plan)
-        launch_mla_t<2, true>(s, keep, *plan, pool, table, rows, n_rows, work, n_work, qlat, H, P,
+        launch_mla_t<2, true>(s, keep, p32, *plan, pool, table, rows, n_rows, work, n_work, qlat, H, P,
                               mask_mode, part_o, part_ml, ev0, ev1);
     else if (nqt == 1)
-        launch_mla_t<1, false>(s, keep, NoPlan{0}, pool, table, rows, n_rows, work, n_work, qlat, H, P,
+        launch_mla_t<1, false>(s, keep, p32, NoPlan{0}, pool, table, rows, n_rows, work, n_work, qlat, H, P,
                                mask_mode, part_o, part_ml, ev0, ev1);
     else
-        launch_mla_t<2, false>(s, keep, NoPlan{0}, pool, table, rows, n_rows, work, n_work, qlat, H, P,
+        launch_mla_t<2, false>(s, keep, p32, NoPlan{0}, pool, table, rows, n_rows, work, n_work, qlat, H, P,
                                mask_mode, part_o, part_ml, ev0, ev1);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
@@ -1094,10 +1125,10 @@ hipError_t launch_mla_decode(hipStream_t s, const PlanArg *plan, const uint16_t 
     // one plan row (no head groups).
     const int one_q = total_q == n_rows && max_nq == 1;
     if (plan)
-        launch_mla_out<true>(s, *plan, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, hd, dc,
+        launch_mla_out<true>(s, p32, *plan, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, hd, dc,
                              16 * nqt, out, out_bf16, cus);
     else
-        launch_mla_out<false>(s, NoPlan{0}, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, hd, dc,
+        launch_mla_out<false>(s, p32, NoPlan{0}, rows, n_rows, total_q, one_q, part_o, part_ml, w_uv, H, hd, dc,
                               16 * nqt, out, out_bf16, cus);
     return hipGetLastError();
 }
@@ -1105,8 +1136,8 @@ hipError_t launch_mla_decode(hipStream_t s, const PlanArg *plan, const uint16_t 
 int mla_decode_wgs_per_cu(int nqt) {
     int n = 0;
     hipError_t e = hipErrorInvalidValue;
-    if (nqt == 1) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, mla_decode_kernel<1, true, false>, 64 * MlaShape<1>::NW, 0);
-    if (nqt == 2) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, mla_decode_kernel<2, true, false>, 64 * MlaShape<2>::NW, 0);
+    if (nqt == 1) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, mla_decode_kernel<1, true, false, false>, 64 * MlaShape<1>::NW, 0);
+    if (nqt == 2) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, mla_decode_kernel<2, true, false, false>, 64 * MlaShape<2>::NW, 0);
     return (e == hipSuccess && n > 0) ? n : 1;
 }
 

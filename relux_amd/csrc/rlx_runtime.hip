@@ -2139,10 +2139,13 @@ int32_t rlx_gqa_attend_noalloc(void *h, int32_t layer, int32_t n_seqs, const int
 // an expansion (4 bytes x 128 dims x heads per token written and read back)
 // costs far more, and past them by an estimate of both, of n = the call's
 // rows, their pairs with keys, and heads x keys expanded (us, fitted at 16,
-// 32 and 128 heads, head_dim 128, 1 and 4 sequences; absorbed / FA2: 16 heads
-// on 8192 keys, 65 new tokens 87 / 116, 128 138 / 124, 256 277 / 136; 128
-// heads on 8192, 9 92 / 442, 32 268 / 436, 64 642 / 447; 4 x 1024 keys, 16
-// heads, 96 137 / 86).  Other head dims, whose merge is slower, keep the
+// 32 and 128 heads, head_dim 128, 1 and 4 sequences; a pass, absorbed / FA2: 16
+// heads on 8192 keys, 65 new tokens 94 / 132, 128 148 / 141, 256 302 / 151; 128
+// heads on 8192, 9 100 / 487, 32 295 / 487, 64 654 / 475; 4 x 1024 keys, 16
+// heads, 96 149 / 106; 16 x 512 keys, 128 heads, 9 337 / 643).  Past the
+// bound the split partials are f32 (p32 below; bf16 as in decode: 93 and 291
+// for the 9 and 32 of 128 heads, but up to 1.07 times FA2's error against 64
+// bits, where f32 reads 0.66 to 0.94 times).  Other head dims, whose merge is slower, keep the
 // bound alone.  RLX_MLA_FA2_ROWS overrides it (tests run both paths on one
 // shape; read per call).
 // len(i): the live tokens of sequence i the call attends.
@@ -2447,7 +2450,10 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
     }
     if ((rc = flush_patches(c))) return bail(rc);
     const size_t ql_bytes = ((size_t)total_q * num_heads * kMlaRow * 2 + 255) & ~(size_t)255;
-    const size_t po_bytes = ((size_t)parts * QRP * kMlaDc * sizeof(uint16_t) + 255) & ~(size_t)255;
+    // Past kMlaGroupRowsMax rows the other form keeps its sums in f32
+    // throughout, so here the split partials stay f32 too.
+    const bool p32 = max_qr > kMlaGroupRowsMax && head_dim == 128;
+    const size_t po_bytes = ((size_t)parts * QRP * kMlaDc * (p32 ? 4 : 2) + 255) & ~(size_t)255;
     const size_t pm_bytes = ((size_t)parts * QRP * 2 * sizeof(float) + 255) & ~(size_t)255;
     if ((rc = ensure_ws(c, ql_bytes + po_bytes + pm_bytes))) return bail(rc);
     PlanArg plan_arg;
@@ -2474,8 +2480,8 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
                               parts, q_nope,
                               q_rope, q_dtype == RLX_BF16, (const uint16_t *)w_uk,
                               (const uint16_t *)w_uv, num_heads, head_dim, c->dc, c->dr, total_q,
-                              row_nq, c->P, qscale, kmask, nqt, (uint16_t *)ws,
-                              (uint16_t *)(ws + ql_bytes), (float *)(ws + ql_bytes + po_bytes), out,
+                              row_nq, c->P, qscale, kmask, nqt, (uint16_t *)ws, p32,
+                              ws + ql_bytes, (float *)(ws + ql_bytes + po_bytes), out,
                               out_dtype == RLX_BF16, c->cus, e0, e1, app));
     return RLX_OK;
 }
