@@ -94,6 +94,15 @@ struct PfShape {
     // plain schedule).
     static constexpr bool STAG = SRC == kSrcDense && ST * 16 * (S + 1) <= 163840;
     static constexpr int SR = S + (STAG ? 1 : 0);                    // ring stages
+    // Weights as hi + lo bf16 pairs.  Stored head dim 96 also runs as query
+    // tiles of the decode kernel, whose running max is exact at every block
+    // (so the largest weights are exact ones): weights scaled by this kernel's
+    // lazy max and rounded once read up to 1.13 times its error against 64
+    // bits, the pair 0.28 to 1.0 times (N(0, 0.3) to N(0, 3) queries).  A
+    // block costs a third more (937 and 1875 new tokens, 64 heads over 8:
+    // 112 -> 153 us, as query tiles 815).
+    static constexpr bool SPLIT = SRC == kSrcPaged && DQK == 96;
+    static_assert(!SPLIT || !STAG, "pv_plain multiplies the rounded weights alone");
     static constexpr int MD = DV / 32;                               // output dim tiles
     static_assert(DQK % 32 == 0 && DV % 32 == 0 && (SRC == kSrcPaged || DQK % 64 == 0), "whole 32-dim tiles");
     static_assert(SRC == kSrcPaged || DV == 128, "dense: 128 value dims per launch");
@@ -390,8 +399,8 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
 #pragma unroll
     for (int i = 0; i < 16; i++) negm[i] = 0.f;
     // P^T operands of the current block (the lagging waves keep them into
-    // the next iteration).
-    u32x4 pw[4];
+    // the next iteration), and what their rounding to bf16 leaves (SPLIT).
+    u32x4 pw[4], pl[4];
     // P.V of the weights in pw over the V^T region of stage sv, operand
     // reads kPfD steps ahead (the lagging waves' form: no softmax work to
     // interleave).
@@ -483,6 +492,11 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
             const uint32_t w = pack_bf16x2(p0, p1);
             pw[2 * kt + (k >> 2)][k & 3] = w;
             lt[kt] = add_bf16x2(w, lt[kt]);
+            if constexpr (SH::SPLIT) {
+                const uint32_t r = pack_bf16x2(p0 - bf16_lo(w), p1 - bf16_hi(w));
+                pl[2 * kt + (k >> 2)][k & 3] = r;
+                lt[kt] = add_bf16x2(r, lt[kt]);
+            }
             asm volatile("" ::"v"(w), "v"(lt[kt]));
         };
         // Causal mask of key tile kt (value i is masked when its key offset
@@ -596,6 +610,10 @@ __global__ __launch_bounds__(64 * kWaves) void prefill_kernel(const PrefillArgs 
                 acc[md] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
                     __builtin_bit_cast(bf16x8, va[n % (kPfD + 1)]), __builtin_bit_cast(bf16x8, pw[n / MD]),
                     acc[md], 0, 0, 0);
+                if constexpr (SH::SPLIT)
+                    acc[md] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(
+                        __builtin_bit_cast(bf16x8, va[n % (kPfD + 1)]), __builtin_bit_cast(bf16x8, pl[n / MD]),
+                        acc[md], 0, 0, 0);
                 if (n < HALF) {
 #pragma unroll
                     for (int k = (n * 8) / HALF; k < ((n + 1) * 8) / HALF; k++) pword(1, k);

@@ -117,3 +117,26 @@ def test_mla_parts(gpu, monkeypatch, H, D, before, n, fa2):
         Q = torch.cat([qn, qr], 2)[qt:qt + n[i]].double()
         _check(o[qt:qt + n[i]], _exact(Q, K, V, n[i], "causal", 1.0 / math.sqrt(D + 64)))
         at, qt = at + T[i], qt + n[i]
+
+
+@pytest.mark.parametrize("D", [80, 96])
+@pytest.mark.parametrize("scale", [0.3, 1.0, 3.0])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_hd96_no_less_precise_than_query_tiles(gpu, D, scale, dtype):
+    """Stored head dim 96 in the prefill kernel is no further off the 64-bit
+    result than as query tiles of the decode kernel (the call that allocates
+    nothing takes those)."""
+    from relux_amd import KVCache
+    H, T, n = 2, 9000, 1800
+    g = torch.Generator(device=gpu).manual_seed(D)
+    k, v = (torch.randn(T, H, D, device=gpu, generator=g).to(torch.bfloat16) for _ in range(2))
+    q = (torch.randn(n, H, D, device=gpu, generator=g) * scale).to(dtype)
+    c = KVCache(num_layers=1, max_len=T, num_kv_heads=H, head_dim=D, device=gpu.index)
+    c.Append(0, k, v, seq_ids=[0], n_tok=[T], layout="SHD")
+    tiles = torch.empty_like(q)
+    c.AttendNoAlloc(0, q, H, tiles, seq_ids=[0], n_q=[n], layout="SHD")
+    o = c.Attend(0, q, H, seq_ids=[0], n_q=[n])
+    assert not torch.equal(o, tiles), "the call took query tiles"
+    want = _exact(q.double(), k.double(), v.double(), n, "causal", 1.0 / math.sqrt(D))
+    off = [float((x.double() - want).norm()) for x in (o, tiles)]
+    assert off[0] <= 1.005 * off[1], off
