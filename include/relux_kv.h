@@ -333,8 +333,9 @@ int32_t rlx_gqa_append_attend(void *cache, int32_t layer, int32_t n_seqs, const 
  * split partials go to a fixed 32 MiB scratch array per device (held until
  * the process ends) instead of the cache's workspace, pending page-table
  * writes travel in kernel arguments, and no staging buffer is used (a
- * head_dim of 65 to 96 past 32 query rows runs query tiles where
- * rlx_gqa_attend takes its prefill kernel: same results within tolerance).
+ * head_dim of 65 to 96 past 32 query rows runs query tiles at any size,
+ * where rlx_gqa_attend takes its prefill kernel for the larger calls: same
+ * results within tolerance).
  * Limits
  * (RLX_ERR_UNSUPPORTED beyond them, nothing launched): at most 32 query rows
  * per kv head, at most 64 rows (sequences, or query tiles of head_dim 16/32

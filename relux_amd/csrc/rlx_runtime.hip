@@ -1688,8 +1688,7 @@ int32_t check_gqa_attend(Cache *c, int32_t layer, int32_t n_seqs, const int32_t 
 // holds run as FA2 chunked prefill: stored head dims 64, 128 and 256 (any
 // caller head_dim they hold), any G = heads per kv head up to 256 (a tile
 // holds floor(256 / G) tokens); head dim 96 with groups the decode kernel
-// takes too (1000 new tokens of 2 sequences on 2000, 32 heads over 8 of 80
-// dims: 468 us as query tiles, 116 in FA2).  Other shapes tile their queries
+// takes too, where gqa_hd96_fa2 says so.  Other shapes tile their queries
 // through the decode kernel.
 bool gqa_use_fa2(const Cache *c, int G) {
     if (c->hd == 96) return G <= gqa_rows_cap(c);
@@ -1727,6 +1726,107 @@ int32_t gqa_call_padded(Cache *c, int64_t rows, const void *q, int32_t q_dtype, 
     return RLX_OK;
 }
 
+// Stored head dim 96 past the decode kernel's rows: whether a call is faster in
+// FA2 than as query tiles, by estimates of both in us.  A query tile (cap / G
+// tokens) walks all keys of its sequence, spread over the CUs; past 64 tiles
+// the plan is staged.  FA2 waits for its longest tile (cut past 12 blocks).
+// Measured at 8/2, 32/8, 64/8 and 16/16 heads, 1 and 4 sequences, 0 to 8000
+// cached tokens (us, tiles / FA2): 32/8, 128 new tokens alone 15.9 / 19.4, on
+// 500 17.8 / 32.6, on 3000 31.7 / 45.1, on 8000 85.8 / 59.1; 600 alone 50.7 /
+// 35.0, on 3000 163 / 81.  The choice costs 0.2 % of the faster one on average
+// there, 2 % against the tiles at most.
+// A stream under capture takes the tiles, whose plan travels in the kernel
+// arguments where it fits.
+bool gqa_hd96_fa2(Cache *c, int layer, int n_seqs, const int32_t *seq_ids, const int32_t *n_q, int G,
+                  int mask_mode) {
+    const int per = gqa_rows_cap(c) / G, toks = kPrefillRows / G;
+    double rows = 0.0, keys = 0.0, blocks = 0.0;
+    int most = 0;
+    for (int i = 0; i < n_seqs; i++) {
+        AttRow r{};
+        r.len = c->L[layer].seqs[seq_ids[i]].len;
+        r.nq = n_q ? n_q[i] : 1;
+        const int tiles = (r.nq + per - 1) / per;
+        rows += tiles;
+        keys += (double)tiles * r.len;
+        for (int qt = 0; qt * toks < r.nq; qt++) {
+            const int b = (tile_keys(r, mask_mode, toks, qt) + 63) / 64;
+            blocks += b;
+            most = std::max(most, b);
+        }
+    }
+    const double tiles_us = 13.0 + 0.01 * rows * c->kvh + 4.5e-5 * keys * c->kvh + (rows > 64 ? 8.0 : 0.0);
+    const double fa2_us = 16.0 + 1.4 * std::min(most, 12) + 0.005 * blocks * c->kvh;
+    return fa2_us < 0.95 * tiles_us;
+}
+// GQA chunked prefill / long verify: FA2 tiles of kPrefillRows query rows.
+int32_t gqa_prefill_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *seq_ids,
+                         const int32_t *n_q, int32_t num_heads, const void *q, int32_t q_dtype,
+                         int32_t qo_layout, float scale, int32_t mask_mode, void *out, int32_t out_dtype) {
+    int32_t rc = RLX_OK;
+    const int G = num_heads / c->kvh;
+    LayerState &ls = c->L[layer];
+    std::vector<AttRow> rows;
+    std::vector<int2> unused;
+    int total_q = 0, mnq = 0, parts = 0;
+    if ((rc = build_rows(c, layer, n_seqs, seq_ids, n_q, nullptr, rows, unused, &total_q, &mnq, &parts)))
+        return rc;
+    const int toks = kPrefillRows / G;
+    std::vector<std::vector<int4>> groups;
+    std::vector<double> cost;
+    for (int i = 0; i < n_seqs; i++) {
+        const int tiles = (rows[i].nq + toks - 1) / toks;
+        for (int kvh = 0; kvh < c->kvh; kvh++) {
+            groups.emplace_back();
+            cost.push_back(0.0);
+            for (int qt = tiles - 1; qt >= 0; qt--) {
+                groups.back().push_back(int4{i, kvh, qt, -1});
+                cost.back() += tile_keys(rows[i], mask_mode, toks, qt);
+            }
+        }
+    }
+    const PrefillSplit sp = prefill_parts(c, groups, cost, rows, mask_mode, toks, 0);
+    const std::vector<int4> work = xcd_order(groups, cost);
+    if ((rc = flush_patches(c))) return rc;
+    Blob b;
+    size_t o_r = b.add(rows), o_w = b.add(work), o_g = b.add(sp.ranges), o_m = b.add(sp.merge);
+    void *dev;
+    if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
+    if (scale <= 0.f) scale = (float)(1.0 / std::sqrt((double)c->hdu));
+    PrefillArgs a{};
+    a.kpool = ls.pool0;
+    a.vpool = ls.pool1;
+    a.table = c->d_table;
+    a.rows = (const AttRow *)((char *)dev + o_r);
+    a.work = (const int4 *)((char *)dev + o_w);
+    a.ranges = (const int2 *)((char *)dev + o_g);
+    a.merge = (const int4 *)((char *)dev + o_m);
+    a.n_merge = (int)sp.merge.size();
+    a.part_o = (float *)c->ws.ptr;
+    a.part_ml = (float *)((char *)c->ws.ptr + sp.ranges.size() * kPrefillPartO);
+    a.q = q;
+    a.out = out;
+    a.q_bf16 = q_dtype == RLX_BF16;
+    a.layout = qo_layout;
+    a.out_bf16 = out_dtype == RLX_BF16;
+    a.mask_mode = mask_mode;
+    a.H = num_heads;
+    a.HQ = num_heads;
+    a.h0 = 0;
+    a.KVH = c->kvh;
+    a.P = c->P;
+    a.pshift = (c->P & (c->P - 1)) == 0 ? __builtin_ctz((unsigned)c->P) : -1;
+    a.qscale = scale * 1.4426950408889634f;
+    a.qd = c->hdi;
+    a.od = c->hdi;
+    a.vd = c->hd;
+    a.dv0 = 0;
+    hipEvent_t e0, e1;
+    if ((rc = timing_events(c, &e0, &e1))) return rc;
+    HIP_TRY(launch_prefill(c->stream, kSrcPaged, c->hd, a, (int)work.size(), e0, e1));
+    return RLX_OK;
+}
+
 // GQA attention after the argument checks.
 int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *seq_ids,
                         const int32_t *n_q, int32_t num_heads, const void *q, int32_t q_dtype,
@@ -1744,75 +1844,19 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
     const int max_qr = G * max_nq;
     // Query rows past cap (the decode kernel's per kv head) take FA2 or query
     // tiles (gqa_use_fa2).
-    // (Head dim 96 under capture: query tiles, whose plan travels in the kernel
-    // arguments where it fits.)
     const int cap = gqa_rows_cap(c);
-    const bool fa2 = gqa_use_fa2(c, G) && !(c->hd == 96 && max_qr > cap && capturing(c));
+    bool fa2 = gqa_use_fa2(c, G);
+    const bool choice = fa2 && c->hd == 96 && max_qr > cap;
+    const bool may = choice && !capturing(c);
+    if (choice) fa2 = may && gqa_hd96_fa2(c, layer, n_seqs, seq_ids, n_q, G, mask_mode);
     if (max_qr > cap && !fa2 && G > cap)
         return fail(RLX_ERR_UNSUPPORTED, "heads per kv head = %d with head_dim %d (at most %d)", G,
                     c->hdi, cap);
-    if (max_qr > cap && fa2) {
-        // Chunked prefill / long verify: FA2 tiles of kPrefillRows query rows.
-        std::vector<AttRow> rows;
-        std::vector<int2> unused;
-        int total_q = 0, mnq = 0, parts = 0;
-        if ((rc = build_rows(c, layer, n_seqs, seq_ids, n_q, nullptr, rows, unused, &total_q, &mnq, &parts)))
-            return rc;
-        const int toks = kPrefillRows / G;
-        std::vector<std::vector<int4>> groups;
-        std::vector<double> cost;
-        for (int i = 0; i < n_seqs; i++) {
-            const int tiles = (rows[i].nq + toks - 1) / toks;
-            for (int kvh = 0; kvh < c->kvh; kvh++) {
-                groups.emplace_back();
-                cost.push_back(0.0);
-                for (int qt = tiles - 1; qt >= 0; qt--) {
-                    groups.back().push_back(int4{i, kvh, qt, -1});
-                    cost.back() += tile_keys(rows[i], mask_mode, toks, qt);
-                }
-            }
-        }
-        const PrefillSplit sp = prefill_parts(c, groups, cost, rows, mask_mode, toks, 0);
-        const std::vector<int4> work = xcd_order(groups, cost);
-        if ((rc = flush_patches(c))) return rc;
-        Blob b;
-        size_t o_r = b.add(rows), o_w = b.add(work), o_g = b.add(sp.ranges), o_m = b.add(sp.merge);
-        void *dev;
-        if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
-        if (scale <= 0.f) scale = (float)(1.0 / std::sqrt((double)c->hdu));
-        PrefillArgs a{};
-        a.kpool = ls.pool0;
-        a.vpool = ls.pool1;
-        a.table = c->d_table;
-        a.rows = (const AttRow *)((char *)dev + o_r);
-        a.work = (const int4 *)((char *)dev + o_w);
-        a.ranges = (const int2 *)((char *)dev + o_g);
-        a.merge = (const int4 *)((char *)dev + o_m);
-        a.n_merge = (int)sp.merge.size();
-        a.part_o = (float *)c->ws.ptr;
-        a.part_ml = (float *)((char *)c->ws.ptr + sp.ranges.size() * kPrefillPartO);
-        a.q = q;
-        a.out = out;
-        a.q_bf16 = q_dtype == RLX_BF16;
-        a.layout = qo_layout;
-        a.out_bf16 = out_dtype == RLX_BF16;
-        a.mask_mode = mask_mode;
-        a.H = num_heads;
-        a.HQ = num_heads;
-        a.h0 = 0;
-        a.KVH = c->kvh;
-        a.P = c->P;
-        a.pshift = (c->P & (c->P - 1)) == 0 ? __builtin_ctz((unsigned)c->P) : -1;
-        a.qscale = scale * 1.4426950408889634f;
-        a.qd = c->hdi;
-        a.od = c->hdi;
-        a.vd = c->hd;
-        a.dv0 = 0;
-        hipEvent_t e0, e1;
-        if ((rc = timing_events(c, &e0, &e1))) return rc;
-        HIP_TRY(launch_prefill(c->stream, kSrcPaged, c->hd, a, (int)work.size(), e0, e1));
-        return RLX_OK;
-    }
+    const auto prefill = [&] {
+        return gqa_prefill_impl(c, layer, n_seqs, seq_ids, n_q, num_heads, q, q_dtype, qo_layout, scale,
+                                mask_mode, out, out_dtype);
+    };
+    if (max_qr > cap && fa2) return prefill();
     const int qtile = max_qr > cap ? cap / G : 0;
     const int nqt = std::min(max_qr, cap) > 16 ? 2 : 1;
     int n_rows = 0;
@@ -1831,7 +1875,7 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
     const int QRP = 16 * nqt;
     const size_t po_bytes = (size_t)parts * c->kvh * QRP * c->hd * sizeof(float);
     const size_t pm_bytes = (size_t)parts * c->kvh * QRP * 2 * sizeof(float);
-    if ((rc = ensure_ws(c, po_bytes + pm_bytes))) return rc;
+    if ((rc = ensure_ws(c, po_bytes + pm_bytes))) return may ? prefill() : rc;  // (FA2 needs no workspace)
     // Rows travel in the kernel arguments when they fit, followed by the
     // ranges when those fit too (else the kernel recomputes its range from
     // the rows: <= 64 rows, one per lane); otherwise rows and ranges are

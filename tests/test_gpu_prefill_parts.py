@@ -135,8 +135,34 @@ def test_hd96_no_less_precise_than_query_tiles(gpu, D, scale, dtype):
     c.Append(0, k, v, seq_ids=[0], n_tok=[T], layout="SHD")
     tiles = torch.empty_like(q)
     c.AttendNoAlloc(0, q, H, tiles, seq_ids=[0], n_q=[n], layout="SHD")
-    o = c.Attend(0, q, H, seq_ids=[0], n_q=[n])
+    o = c.Attend(0, q, H, seq_ids=[0], n_q=[n], out=torch.empty_like(q))
     assert not torch.equal(o, tiles), "the call took query tiles"
     want = _exact(q.double(), k.double(), v.double(), n, "causal", 1.0 / math.sqrt(D))
     off = [float((x.double() - want).norm()) for x in (o, tiles)]
     assert off[0] <= 1.005 * off[1], off
+
+
+def _hd96(gpu, H, KVH, D, before, n, dtype):
+    from relux_amd import KVCache
+    g = torch.Generator(device=gpu).manual_seed(D + H)
+    S, T = len(before), [a + b for a, b in zip(before, n)]
+    k, v = (torch.randn(sum(T), KVH, D, device=gpu, generator=g).to(torch.bfloat16) for _ in range(2))
+    c = KVCache(num_layers=1, max_len=max(T), num_kv_heads=KVH, head_dim=D, max_seqs=S, device=gpu.index)
+    c.Append(0, k, v, seq_ids=list(range(S)), n_tok=T, layout="SHD")
+    q = torch.randn(sum(n), H, D, device=gpu, generator=g).to(dtype)
+    tiles = c.AttendNoAlloc(0, q, H, torch.empty_like(q), seq_ids=list(range(S)), n_q=n)
+    return c, q, tiles, dict(seq_ids=list(range(S)), n_q=n)
+
+
+@pytest.mark.parametrize("H,KVH,D,before,n,fa2", [
+    (32, 8, 80, [2000], [100], False),
+    (16, 16, 80, [300, 50], [200, 400], False),
+    (32, 8, 96, [0], [40], False),
+    (8, 2, 72, [8000], [64], False),
+    (64, 8, 80, [8000], [128], True),
+    (16, 16, 96, [8000], [1000], True),
+])
+def test_hd96_route(gpu, H, KVH, D, before, n, fa2):
+    """Query tiles where they are the faster form, which is most small calls."""
+    c, q, tiles, kw = _hd96(gpu, H, KVH, D, before, n, torch.bfloat16)
+    assert torch.equal(c.Attend(0, q, H, out=torch.empty_like(q), **kw), tiles) != fa2
