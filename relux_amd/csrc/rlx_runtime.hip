@@ -894,6 +894,14 @@ PrefillSplit prefill_parts(Cache *c, std::vector<std::vector<int4>> &groups, std
     return sp;
 }
 
+// Whether q and out of `rows` rows of row_elems elements share memory.
+bool qo_overlap(size_t rows, const void *q, int q_dtype, const void *out, int out_dtype, int row_elems) {
+    const char *qb = (const char *)q, *ob = (const char *)out;
+    const size_t qn = rows * row_elems * (q_dtype == RLX_BF16 ? 2 : 4);
+    const size_t on = rows * row_elems * (out_dtype == RLX_BF16 ? 2 : 4);
+    return ob < qb + qn && qb < ob + on;
+}
+
 // Whether the decode kernel may write a call's outputs itself: every row lies in
 // one range, and out does not overlap q, which other work-groups may still read
 // (the merge runs after all of them).
@@ -904,10 +912,7 @@ bool gqa_single(const AttRow *rows, int n, const void *q, int q_dtype, const voi
         if (rows[i].nsplit != 1) return false;
         tokens = std::max(tokens, (size_t)rows[i].qrow + rows[i].nq);
     }
-    const char *qb = (const char *)q, *ob = (const char *)out;
-    const size_t qn = tokens * row_elems * (q_dtype == RLX_BF16 ? 2 : 4);
-    const size_t on = tokens * row_elems * (out_dtype == RLX_BF16 ? 2 : 4);
-    return ob >= qb + qn || qb >= ob + on;
+    return !qo_overlap(tokens, q, q_dtype, out, out_dtype, row_elems);
 }
 
 // One AttRow per sequence of an attention call, with nsplit[i] context
@@ -1735,8 +1740,11 @@ int32_t gqa_call_padded(Cache *c, int64_t rows, const void *q, int32_t q_dtype, 
 // 500 17.8 / 32.6, on 3000 31.7 / 45.1, on 8000 85.8 / 59.1; 600 alone 50.7 /
 // 35.0, on 3000 163 / 81.  The choice costs 0.2 % of the faster one on average
 // there, 2 % against the tiles at most.
-// A stream under capture takes the tiles, whose plan travels in the kernel
-// arguments where it fits.
+// FA2 reads a tile's queries when it starts and writes its rows when it ends,
+// so memory that q and out share other than row for row takes the tiles, whose
+// merge runs last; so do outputs off their stores' alignment, and a stream
+// under capture (the tiles' plan travels in the kernel arguments where it
+// fits).
 bool gqa_hd96_fa2(Cache *c, int layer, int n_seqs, const int32_t *seq_ids, const int32_t *n_q, int G,
                   int mask_mode) {
     const int per = gqa_rows_cap(c) / G, toks = kPrefillRows / G;
@@ -1759,6 +1767,12 @@ bool gqa_hd96_fa2(Cache *c, int layer, int n_seqs, const int32_t *seq_ids, const
     const double fa2_us = 16.0 + 1.4 * std::min(most, 12) + 0.005 * blocks * c->kvh;
     return fa2_us < 0.95 * tiles_us;
 }
+bool gqa_hd96_may_fa2(Cache *c, int64_t rows, const void *q, int q_dtype, const void *out, int out_dtype) {
+    if ((uintptr_t)out & (out_dtype == RLX_BF16 ? 7 : 15)) return false;
+    if (!(q == out && q_dtype == out_dtype) && qo_overlap(rows, q, q_dtype, out, out_dtype, c->hdi)) return false;
+    return !capturing(c);
+}
+
 // GQA chunked prefill / long verify: FA2 tiles of kPrefillRows query rows.
 int32_t gqa_prefill_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *seq_ids,
                          const int32_t *n_q, int32_t num_heads, const void *q, int32_t q_dtype,
@@ -1847,7 +1861,7 @@ int32_t gqa_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t *
     const int cap = gqa_rows_cap(c);
     bool fa2 = gqa_use_fa2(c, G);
     const bool choice = fa2 && c->hd == 96 && max_qr > cap;
-    const bool may = choice && !capturing(c);
+    const bool may = choice && gqa_hd96_may_fa2(c, gqa_qo_rows(n_seqs, n_q, num_heads), q, q_dtype, out, out_dtype);
     if (choice) fa2 = may && gqa_hd96_fa2(c, layer, n_seqs, seq_ids, n_q, G, mask_mode);
     if (max_qr > cap && !fa2 && G > cap)
         return fail(RLX_ERR_UNSUPPORTED, "heads per kv head = %d with head_dim %d (at most %d)", G,

@@ -166,3 +166,24 @@ def test_hd96_route(gpu, H, KVH, D, before, n, fa2):
     """Query tiles where they are the faster form, which is most small calls."""
     c, q, tiles, kw = _hd96(gpu, H, KVH, D, before, n, torch.bfloat16)
     assert torch.equal(c.Attend(0, q, H, out=torch.empty_like(q), **kw), tiles) != fa2
+
+
+def test_hd96_outputs_in_the_queries_memory(gpu):
+    """The prefill kernel writes a tile's rows while others still read theirs:
+    outputs in the queries' own memory, but not row for row, and outputs off
+    their stores' alignment, run as query tiles at any size."""
+    H, KVH, D, before, n = 64, 8, 80, [8000], [128]
+    c, q, tiles, kw = _hd96(gpu, H, KVH, D, before, n, torch.float32)
+    out = torch.empty(q.shape, dtype=torch.bfloat16, device=gpu)
+    want = c.AttendNoAlloc(0, q, H, out, **kw).clone()
+    m = q.numel()
+    buf = q.reshape(-1).clone().view(torch.bfloat16)  # 2 m elements, the queries as f32
+    for off in (0, m, 8):
+        buf.view(torch.float32).copy_(q.reshape(-1))
+        c.Attend(0, buf.view(torch.float32).view(q.shape), H, out=buf[off:off + m].view(q.shape), **kw)
+        assert torch.equal(buf[off:off + m].view(q.shape), want), off
+    odd = torch.empty(m + 1, dtype=torch.bfloat16, device=gpu)[1:].view(q.shape)
+    assert torch.equal(c.Attend(0, q, H, out=odd, **kw), want)
+    same = q.clone()  # row for row: as with separate outputs
+    assert torch.equal(c.Attend(0, same, H, out=same, **kw), c.Attend(0, q, H, **kw))
+    assert not torch.equal(same, tiles), "the call took query tiles"
