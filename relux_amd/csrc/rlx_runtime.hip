@@ -28,6 +28,7 @@
 
 #include "../../include/relux_kv.h"
 #include "rlx_common.h"
+#include "rlx_prefill_plan.h"
 #include "rlx_scratch.h"
 
 using namespace rlx;
@@ -572,144 +573,12 @@ std::vector<int> mla_splits(const std::vector<int> &lens, int64_t slots) {
     return n;
 }
 
-// Prefill work order for the 8 XCDs.  Work-group b runs on XCD b % 8 and
-// each XCD has its own L2, so all query tiles of one (sequence, head group)
-// -- which stream the same K/V blocks in the same order -- are placed on one
-// XCD at consecutive positions: the XCD then fetches each block from HBM once.
-// Groups go to the least-loaded XCD, largest first; shorter XCD lists are
-// padded with empty items (row -1).
-constexpr int kXcds = 8;
-std::vector<int4> xcd_order(const std::vector<std::vector<int4>> &groups,
-                            const std::vector<double> &cost) {
-    static const bool plain = [] {
-        const char *e = getenv("RLX_PREFILL_ORDER");  // tuning override: "plain"
-        return e && strcmp(e, "plain") == 0;
-    }();
-    if (plain) {
-        std::vector<int4> out;
-        for (auto &g : groups) out.insert(out.end(), g.begin(), g.end());
-        return out;
-    }
-    std::vector<int> idx(groups.size());
-    for (size_t i = 0; i < idx.size(); i++) idx[i] = (int)i;
-    std::stable_sort(idx.begin(), idx.end(), [&](int a, int b) { return cost[a] > cost[b]; });
-    std::vector<std::vector<int4>> lists(kXcds);
-    std::vector<double> load(kXcds, 0.0);
-    for (int g : idx) {
-        const int x = (int)(std::min_element(load.begin(), load.end()) - load.begin());
-        load[x] += cost[g];
-        lists[x].insert(lists[x].end(), groups[g].begin(), groups[g].end());
-    }
-    size_t n = 0;
-    for (auto &l : lists) n = std::max(n, l.size());
-    std::vector<int4> out(n * kXcds, int4{-1, 0, 0, 0});
-    for (int x = 0; x < kXcds; x++)
-        for (size_t i = 0; i < lists[x].size(); i++) out[i * kXcds + x] = lists[x][i];
-    return out;
-}
-
 // Keys a prefill query tile attends (its work is proportional).
 int tile_keys(const AttRow &r, int mask_mode, int toks, int qt) {
     const int jmax = std::min(r.nq - 1, qt * toks + toks - 1);
     if (mask_mode == RLX_MASK_CAUSAL) return std::min(r.len, r.len - r.nq + jmax + 1);
     if (mask_mode == RLX_MASK_REF && r.nq == r.len) return jmax + 1;
     return r.len;
-}
-
-// Cuts of a prefill call's tiles along the keys.  A work-group (one per CU)
-// walks its tile's keys in blocks of 64, so a call with fewer tiles than CUs,
-// or a few long ones, leaves most of the chip waiting: B 1, 8 kv heads, 16 new
-// tokens on 8192 ran 8 work-groups of 128 blocks.  Tiles of more than `target`
-// blocks are cut into equal parts, merged by their (max, sum) afterwards;
-// the target is the one of a few whose estimate is least: the longest
-// work-group or the CUs' share of the work, kPfStart blocks of start-up per
-// work-group, the merge's launch and its traffic counted in (a block takes
-// about 2 us), if it saves a tenth.  Calls that fill the chip stay whole.
-// Measured (32 heads over 8, D 128, T 8192, us whole / cut): 16 new tokens 231 /
-// 39, 128 235 / 56, 512 251 / 112; T 0: 1024 60 / 55.
-constexpr double kPfStart = 2.5, kPfMerge = 1.5, kPfMergePart = 0.035;
-constexpr int kPfMaxParts = 480;  // 64 MB of partial sums
-struct PrefillSplit {
-    std::vector<int2> ranges;  // part slot -> key blocks
-    std::vector<int4> merge;   // PrefillArgs::merge
-};
-// groups: the tiles by (sequence, head group), `w` -1; blocks(tile): its key
-// blocks.  Cut groups are regrouped by part, so that parts of the same keys
-// stay together and single groups spread over the XCDs.
-// fill: the share of a tile's 256 rows that hold queries (what the merge moves).
-template <class F>
-PrefillSplit split_prefill(std::vector<std::vector<int4>> &groups, std::vector<double> &cost, int cus,
-                           double fill, F blocks) {
-    PrefillSplit sp;
-    int64_t total = 0, tiles = 0;
-    int most = 0;
-    for (auto &g : groups)
-        for (auto &t : g) {
-            const int b = blocks(t);
-            total += b;
-            tiles++;
-            most = std::max(most, b);
-        }
-    if (tiles == 0 || tiles >= 2 * (int64_t)cus) return sp;
-    auto estimate = [&](int64_t n, double longest) {
-        const double share = ((double)total + (double)n * kPfStart) / cus;
-        const double last = n > cus ? 0.5 * ((double)total / n + kPfStart) : 0.0;
-        return std::max(longest + kPfStart, share + last);
-    };
-    int target = 0;
-    double best = 0.9 * estimate(tiles, most);
-    const int base = (int)std::max<int64_t>(4, (total + cus - 1) / cus);
-    for (int k = 4; k <= 10; k += 1) {
-        const int t = base * k / 4;
-        if (t >= most) break;
-        int64_t n = 0, cut = 0;
-        double longest = 0.0;
-        for (auto &g : groups)
-            for (auto &w : g) {
-                const int b = blocks(w), m = (b + t - 1) / t;
-                n += std::max(m, 1);
-                if (m > 1) cut += m;
-                longest = std::max(longest, m > 1 ? std::ceil((double)b / m) : (double)b);
-            }
-        if (cut > kPfMaxParts) continue;
-        const double e = estimate(n, longest) + kPfMerge + kPfMergePart * fill * (double)cut;
-        if (e < best) {
-            best = e;
-            target = t;
-        }
-    }
-    if (target == 0) return sp;
-    std::vector<std::vector<int4>> out;
-    std::vector<double> oc;
-    for (auto &g : groups) {
-        std::vector<std::vector<int4>> part;  // by part number
-        std::vector<double> pc;
-        for (auto &w : g) {
-            const int b = blocks(w), m = std::max(1, (b + target - 1) / target);
-            if ((int)part.size() < m) {
-                part.resize(m);
-                pc.resize(m, 0.0);
-            }
-            if (m > 1) sp.merge.push_back(int4{w.x, w.y, w.z | m << 20, (int)sp.ranges.size()});
-            for (int k = 0; k < m; k++) {
-                const int lo = (int)((int64_t)b * k / m), hi = (int)((int64_t)b * (k + 1) / m);
-                int4 item = w;
-                if (m > 1) {
-                    item.w = (int)sp.ranges.size();
-                    sp.ranges.push_back(int2{lo, hi});
-                }
-                part[k].push_back(item);
-                pc[k] += hi - lo;
-            }
-        }
-        for (size_t k = 0; k < part.size(); k++) {
-            out.push_back(std::move(part[k]));
-            oc.push_back(pc[k]);
-        }
-    }
-    groups = std::move(out);
-    cost = std::move(oc);
-    return sp;
 }
 
 // One AttRow per sequence, or -- with qtile > 0 (GQA decode kernel only) --
@@ -874,24 +743,30 @@ int gqa_decode_split(const Cache *c, int nqt, AttRow *rows, int n_rows, int *pre
     return n_ranges;
 }
 
-// split_prefill for a call whose own scratch is `head` bytes of the workspace
-// (there already), the partial sums behind it.  Without room for them
-// (optional_ws) the tiles stay whole.
-PrefillSplit prefill_parts(Cache *c, std::vector<std::vector<int4>> &groups, std::vector<double> &cost,
-                           const std::vector<AttRow> &rows, int mask_mode, int toks, size_t head) {
-    auto g = groups;
-    auto k = cost;
+// The work lists of a prefill call over `rows`, heads [0, launched) of `heads`
+// (a call's head groups share the choice), whose own scratch is `head` bytes of
+// the workspace (there already), the partial sums behind it.  Without room for
+// them (optional_ws) the tiles stay whole.
+typedef PrefillPlan<int2, int4> PfPlan;
+PfPlan plan_prefill(Cache *c, const std::vector<AttRow> &rows, int mask_mode, int toks, int heads, int launched,
+                    size_t head) {
+    static const bool plain = [] {
+        const char *e = getenv("RLX_PREFILL_ORDER");  // tuning override: "plain"
+        return e && strcmp(e, "plain") == 0;
+    }();
+    PfTiles t;
     int nq = 0;
-    for (const AttRow &r : rows) nq = std::max(nq, r.nq);
-    const double fill = std::min(1.0, (double)nq / toks);
-    PrefillSplit sp = split_prefill(g, k, c->cus, fill, [&](const int4 &w) {
-        return (tile_keys(rows[w.x], mask_mode, toks, w.z) + 63) / 64;
-    });
-    const size_t need = head + sp.ranges.size() * (kPrefillPartO + kPrefillPartMl);
-    if (sp.ranges.empty() || !optional_ws(c, need)) return {};
-    groups = std::move(g);
-    cost = std::move(k);
-    return sp;
+    for (const AttRow &r : rows) {
+        for (int qt = 0; qt * toks < r.nq; qt++) t.add(tile_keys(r, mask_mode, toks, qt));
+        t.end_seq();
+        nq = std::max(nq, r.nq);
+    }
+    const int target = prefill_target(t, heads, c->cus, std::min(1.0, (double)nq / toks));
+    if (target > 0) {
+        PfPlan plan = prefill_plan<int2, int4>(t, launched, target, plain);
+        if (optional_ws(c, head + plan.ranges.size() * (kPrefillPartO + kPrefillPartMl))) return plan;
+    }
+    return prefill_plan<int2, int4>(t, launched, 0, plain);
 }
 
 // Whether q and out of `rows` rows of row_elems elements share memory.
@@ -1786,24 +1661,10 @@ int32_t gqa_prefill_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t 
     if ((rc = build_rows(c, layer, n_seqs, seq_ids, n_q, nullptr, rows, unused, &total_q, &mnq, &parts)))
         return rc;
     const int toks = kPrefillRows / G;
-    std::vector<std::vector<int4>> groups;
-    std::vector<double> cost;
-    for (int i = 0; i < n_seqs; i++) {
-        const int tiles = (rows[i].nq + toks - 1) / toks;
-        for (int kvh = 0; kvh < c->kvh; kvh++) {
-            groups.emplace_back();
-            cost.push_back(0.0);
-            for (int qt = tiles - 1; qt >= 0; qt--) {
-                groups.back().push_back(int4{i, kvh, qt, -1});
-                cost.back() += tile_keys(rows[i], mask_mode, toks, qt);
-            }
-        }
-    }
-    const PrefillSplit sp = prefill_parts(c, groups, cost, rows, mask_mode, toks, 0);
-    const std::vector<int4> work = xcd_order(groups, cost);
+    const PfPlan plan = plan_prefill(c, rows, mask_mode, toks, c->kvh, c->kvh, 0);
     if ((rc = flush_patches(c))) return rc;
     Blob b;
-    size_t o_r = b.add(rows), o_w = b.add(work), o_g = b.add(sp.ranges), o_m = b.add(sp.merge);
+    size_t o_r = b.add(rows), o_w = b.add(plan.work), o_g = b.add(plan.ranges), o_m = b.add(plan.merge);
     void *dev;
     if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
     if (scale <= 0.f) scale = (float)(1.0 / std::sqrt((double)c->hdu));
@@ -1815,9 +1676,9 @@ int32_t gqa_prefill_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t 
     a.work = (const int4 *)((char *)dev + o_w);
     a.ranges = (const int2 *)((char *)dev + o_g);
     a.merge = (const int4 *)((char *)dev + o_m);
-    a.n_merge = (int)sp.merge.size();
+    a.n_merge = (int)plan.merge.size();
     a.part_o = (float *)c->ws.ptr;
-    a.part_ml = (float *)((char *)c->ws.ptr + sp.ranges.size() * kPrefillPartO);
+    a.part_ml = (float *)((char *)c->ws.ptr + plan.ranges.size() * kPrefillPartO);
     a.q = q;
     a.out = out;
     a.q_bf16 = q_dtype == RLX_BF16;
@@ -1837,7 +1698,7 @@ int32_t gqa_prefill_impl(Cache *c, int32_t layer, int32_t n_seqs, const int32_t 
     a.dv0 = 0;
     hipEvent_t e0, e1;
     if ((rc = timing_events(c, &e0, &e1))) return rc;
-    HIP_TRY(launch_prefill(c->stream, kSrcPaged, c->hd, a, (int)work.size(), e0, e1));
+    HIP_TRY(launch_prefill(c->stream, kSrcPaged, c->hd, a, (int)plan.work.size(), e0, e1));
     return RLX_OK;
 }
 
@@ -2304,23 +2165,12 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
         if ((rc = build_rows(c, layer, n_seqs, seq_ids, n_q, nullptr, rows, unused, &total_q, &mnq, &parts)))
             return rc;
         std::vector<int2> dwork;
-        std::vector<std::vector<int4>> pgroups;
-        std::vector<double> pcost;
         int64_t tok_off = 0;
         for (int i = 0; i < n_seqs; i++) {
             const int Tp = (rows[i].len + 127) / 128 * 128;
             rows[i].part = (int32_t)tok_off;  // token offset in the expanded buffers
             rows[i].nsplit = Tp;              // padded length (row pitch of V^T)
             for (int t0 = 0; t0 < Tp; t0 += 128) dwork.push_back(int2{i, t0});
-            const int tiles = (rows[i].nq + kPrefillRows - 1) / kPrefillRows;
-            for (int h = 0; h < num_heads; h++) {
-                pgroups.emplace_back();
-                pcost.push_back(0.0);
-                for (int qt = tiles - 1; qt >= 0; qt--) {
-                    pgroups.back().push_back(int4{i, h, qt, -1});
-                    pcost.back() += tile_keys(rows[i], mask_mode, kPrefillRows, qt);
-                }
-            }
             tok_off += Tp;
         }
         // Heads per expansion (mla_prefill_heads); larger calls run head
@@ -2335,29 +2185,20 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
         const size_t r_bytes = (size_t)tok_off * kMlaDr * 2;  // rope keys of the call
         const size_t x_bytes = (2 * w_bytes + 2 * e_bytes + r_bytes + 255) & ~(size_t)255;
         if ((rc = ensure_ws(c, x_bytes))) return rc;
-        // (parts chosen over all heads: a head's attention is the same
-        // computation however the heads are grouped)
-        PrefillSplit sp = prefill_parts(c, pgroups, pcost, rows, mask_mode, kPrefillRows, x_bytes);
-        // work items of the group of heads [0, hg) (the xcd order), reused by
-        // every group with its heads counted from the group's first
-        std::vector<std::vector<int4>> pg_grp;
-        std::vector<double> pc_grp;
-        for (size_t k = 0; k < pgroups.size(); k++)
-            if (pgroups[k][0].y < hg) {
-                pg_grp.push_back(pgroups[k]);
-                pc_grp.push_back(pcost[k]);
-            }
-        const std::vector<int4> pwork = xcd_order(pg_grp, pc_grp);
+        // The lists of the group of heads [0, hg), reused by every group with
+        // its heads counted from the group's first (parts chosen over all
+        // heads: a head's attention is the same computation however the heads
+        // are grouped).
+        const PfPlan sp = plan_prefill(c, rows, mask_mode, kPrefillRows, num_heads, hg, x_bytes);
         auto heads_below = [](const std::vector<int4> &v, int n) {
             std::vector<int4> o;
             for (const int4 &w : v)
                 if (w.y < n) o.push_back(w);
             return o;
         };
-        sp.merge = heads_below(sp.merge, hg);
         if ((rc = flush_patches(c))) return rc;
         Blob b;
-        size_t o_r = b.add(rows), o_d = b.add(dwork), o_p = b.add(pwork), o_g = b.add(sp.ranges),
+        size_t o_r = b.add(rows), o_d = b.add(dwork), o_p = b.add(sp.work), o_g = b.add(sp.ranges),
                o_m = b.add(sp.merge);
         void *dev;
         if ((rc = stage(c, b.bytes.data(), b.bytes.size(), &dev))) return rc;
@@ -2411,9 +2252,9 @@ static int32_t mla_attend_impl(Cache *c, int32_t layer, int32_t n_seqs, const in
             a.vd = dp;
             a.dv0 = 0;
             // work items of heads >= nh (a last, smaller group) are dropped
-            int n_work = (int)pwork.size();
+            int n_work = (int)sp.work.size();
             if (nh < hg) {
-                const std::vector<int4> w = heads_below(pwork, nh), m = heads_below(sp.merge, nh);
+                const std::vector<int4> w = heads_below(sp.work, nh), m = heads_below(sp.merge, nh);
                 Blob lb;
                 const size_t l_w = lb.add(w), l_m = lb.add(m);
                 void *dw;
