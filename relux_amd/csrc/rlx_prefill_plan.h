@@ -36,7 +36,7 @@ inline int pf_blocks(int keys) { return (keys + 63) / 64; }  // key blocks of th
 // 39, 128 235 / 56, 512 251 / 112; T 0: 1024 60 / 55.
 // fill: the share of a tile's 256 rows that hold queries (what the merge moves).
 // Returns the target, 0: every tile stays whole.
-constexpr double kPfStart = 2.5, kPfMerge = 1.5, kPfMergePart = 0.035;
+constexpr double kPfStart = 2.5, kPfMerge = 2.2, kPfMergePart = 0.035;
 constexpr int kPfMaxParts = 480;  // 64 MB of partial sums
 inline int prefill_target(const PfTiles &t, int heads, int cus, double fill) {
     int64_t total = 0;
@@ -92,7 +92,9 @@ struct PrefillPlan {
 // positions: the XCD then fetches each block from HBM once.  Cut tiles are
 // grouped by part, so that parts of the same keys stay together.  Groups go to
 // the least-loaded XCD, largest first; shorter XCD lists are padded with empty
-// items.
+// items.  A cut call has about a work-group per CU, so there no XCD may get
+// more than its eighth of them (a second round on a few CUs costs as much as
+// the first): the ends of the longer lists move to the shorter ones.
 // plain: the tiles in order, nothing placed (tuning).
 template <class I2, class I4>
 PrefillPlan<I2, I4> prefill_plan(const PfTiles &t, int heads, int target, bool plain = false) {
@@ -158,6 +160,18 @@ PrefillPlan<I2, I4> prefill_plan(const PfTiles &t, int heads, int target, bool p
             load[x] += g.cost;
             put(lists[x], g, h);
         }
+    size_t total = 0;
+    for (auto &l : lists) total += l.size();
+    if (base > 0) {
+        const size_t most = (total + kXcds - 1) / kXcds;
+        int to = 0;
+        for (auto &l : lists)
+            while (l.size() > most) {
+                while (lists[to].size() >= most) to++;
+                lists[to].push_back(l.back());
+                l.pop_back();
+            }
+    }
     size_t n = 0;
     for (auto &l : lists) n = std::max(n, l.size());
     plan.work.assign(n * kXcds, I4{-1, 0, 0, 0});

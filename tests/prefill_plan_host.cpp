@@ -23,7 +23,7 @@ struct I4 {
         }                                                                                    \
     } while (0)
 
-static int check(const rlx::PfTiles &t, int heads, int target) {
+static int check(const rlx::PfTiles &t, int heads, int target, int cus) {
     const auto plan = rlx::prefill_plan<I2, I4>(t, heads, target);
     CHECK(plan.work.size() % rlx::kXcds == 0);
     // every item once; where it runs
@@ -76,6 +76,9 @@ static int check(const rlx::PfTiles &t, int heads, int target) {
     CHECK(n == (size_t)std::accumulate(per_xcd.begin(), per_xcd.end(), 0));
     for (int u : used) CHECK(u == 1);
     CHECK(plan.merge.size() == merged.size());
+    // a cut call's work-groups fit one round of every XCD's CUs if they fit the chip's
+    if (!plan.ranges.empty() && (int)n <= cus)
+        for (int x : per_xcd) CHECK(x <= cus / rlx::kXcds);
     return 0;
 }
 
@@ -93,14 +96,14 @@ int main() {
         }
         const int target = rlx::prefill_target(t, heads, 256, 1.0);
         cut += target > 0;
-        if (check(t, heads, 0) || (target > 0 && check(t, heads, target)) ||
-            check(t, heads, upto(40)))
+        if (check(t, heads, 0, 256) || (target > 0 && check(t, heads, target, 256)) ||
+            check(t, heads, upto(40), 256))
             return 1;
         // the heads of a smaller launch, and a sequence whose queries see no key
-        if (target > 0 && check(t, upto(heads), target)) return 1;
+        if (target > 0 && check(t, upto(heads), target, 256)) return 1;
         t.add(0);
         t.end_seq();
-        if (check(t, heads, target)) return 1;
+        if (check(t, heads, target, 256)) return 1;
     }
     if (cut < 300) {
         std::printf("only %d calls were cut\n", cut);
