@@ -664,34 +664,49 @@ int gqa_wg_per_cu() {
 }
 // Cuts at row boundaries only, for calls whose work-groups stay short that way:
 // with no row divided the decode kernel writes the outputs itself and the merge
-// launch falls away.  The ranges hold consecutive rows, at most as much as the
-// longest row or an even share.  The line is the tokens a work-group may hold:
-// 768 at head_dim 128, and by the row bytes elsewhere.  At batch 1, 32/8 heads of
-// 128, one range against cuts and a merge: 600 tokens 13.6 against 16.6 us, 800
-// 14.7 against 16.6, 1000 18.2 against 16.8; heads of 64: 1000 tokens 13.7 against
-// 16.8, 1600 17.1 against 17.9, 2000 20.4 against 20.4.  With two query tiles (17 to
-// 32 query rows a kv head) two thirds of it: 8 x 760 tokens, 32 query rows,
-// took 23.9 whole against 23.0, 8 x 510 22.0 against 24.7.  The ranges have to fit the
-// kernel arguments (the kernel's own search knows even cuts only).  Returns their
-// number, or 0.
+// launch falls away.  A row has a range of its own, or, with more rows than
+// ranges, consecutive rows share one by their tokens and kGqaRowStart units a
+// row for its start.  The line: a work-group's tokens past an even share cost
+// less than the merge launch saves (kernel us per 64 tokens: 0.22, 0.30, 0.34,
+// 0.42 and 1.1 at stored head dims 32, 64, 96, 128 and 256, with two query tiles
+// twice that; the merge 3.2 to 5.6), and rows of up to 8 units, which even cuts
+// would leave whole too (kGqaSnap64), always.  Measured, GPU time back to back, even
+// cuts / whole: 32/8 heads of 128, 1 x 500 tokens 10.7 / 9.3, 1 x 750 9.8 / 11.0
+// (cut), 31 x 750 21.6 / 18.4; heads of 64, 1 x 750 8.4 / 8.4, 4 x 1500 9.6 / 12.7
+// (cut), 31 x 1000 17.1 / 12.8.  The ranges have to fit the kernel arguments (the
+// kernel's own search knows even cuts only).  Returns their number, or 0.
+constexpr int kGqaRowStart = 3;
 int gqa_whole_rows(const Cache *c, int nqt, const int *pre, int n_rows, int full, int *cuts) {
     const int line = (nqt == 1 ? 1536 : 1024) / std::max(c->hd, 64);  // 64-token units
+    const int slack = (c->hd <= 32 ? 13 : c->hd == 64 ? 10 : c->hd == 96 ? 9 : c->hd == 128 ? 8 : 5) / nqt;
+    const int share = (pre[n_rows] + full - 1) / full;
     if ((size_t)n_rows * sizeof(AttRow) + (size_t)full * sizeof(int4) > kPlanArgBytes) return 0;
-    int most = (pre[n_rows] + full - 1) / full;
-    for (int i = 0; i < n_rows; i++) most = std::max(most, pre[i + 1] - pre[i]);
-    for (; most <= line; most++) {
-        int n = 0;
+    auto too_long = [&](int units) { return units > line || (units > 2 * kGqaSnap64 && units - share > slack); };
+    int longest = 0;
+    for (int i = 0; i < n_rows; i++) longest = std::max(longest, pre[i + 1] - pre[i]);
+    if (too_long(longest)) return 0;
+    if (n_rows <= full) {
+        for (int i = 0; i <= n_rows; i++) cuts[i] = pre[i];
+        return n_rows;
+    }
+    const int all = pre[n_rows] + kGqaRowStart * n_rows;
+    for (int most = std::max(longest + kGqaRowStart, (all + full - 1) / full);; most++) {
+        int n = 0, w = 0, units = 0;
         cuts[0] = 0;
-        for (int i = 0; i < n_rows && n < full; i++)
-            if (pre[i + 1] - cuts[n] > most) {
-                n++;
-                if (n < full) cuts[n] = pre[i];
+        for (int i = 0; i < n_rows && n < full; i++) {
+            const int r = pre[i + 1] - pre[i] + kGqaRowStart;
+            if (w + r > most) {
+                w = 0;
+                if (++n < full) cuts[n] = pre[i];
             }
+            w += r;
+            if (n < full) units = std::max(units, pre[i + 1] - cuts[n]);
+        }
         if (n >= full) continue;
+        if (too_long(units)) return 0;
         cuts[n + 1] = pre[n_rows];
         return n + 1;
     }
-    return 0;
 }
 
 int gqa_decode_split(const Cache *c, int nqt, AttRow *rows, int n_rows, int *pre, int *cuts,

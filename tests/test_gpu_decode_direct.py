@@ -64,3 +64,26 @@ def test_direct_outputs(gpu, H, KVH, D, lens, nq, dtype, layout):
         # a probability and the output rounded to bf16; scores in float32 to 2^-12 of the sum
         assert ((r - want).abs() <= (2 * U + 2.0 ** -10) * bound + 1e-6).all()
         kr, qr, off = kr + t, qr + n, off + n * H * D
+
+
+@pytest.mark.parametrize("lens,ranges", [
+    ([200, 40, 130, 90, 65, 10, 190, 25] * 3, 24),  # a range each: 32 are there
+    ([500], 1),
+    ([750], 12),                                    # cut: 11 units past an even share
+    ([750] * 31, 31),                               # an even share is a row
+    ([60] * 40, 20),                                # more rows than ranges: even in rows
+])
+def test_ranges_of_short_rows(gpu, lens, ranges):
+    """Rows share a work-group only where there are more rows than ranges (32
+    at 8 kv heads on 256 CUs), and a row is cut where that is the faster form.
+    The call's scratch request tells its ranges: a partial a row and a range."""
+    from relux_amd import KVCache
+    H, KVH, D, S = 32, 8, 128, len(lens)
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the counts are of 256 CUs")
+    c = KVCache(num_layers=1, max_len=max(lens), num_kv_heads=KVH, head_dim=D, max_seqs=S, device=gpu.index)
+    k = torch.randn(sum(lens), KVH, D, device=gpu)
+    c.Append(0, k, k, seq_ids=range(S), n_tok=lens, layout="SHD")
+    c.Attend(0, torch.randn(S, H, D, device=gpu), H, seq_ids=range(S))
+    parts = c.MemoryStats()["workspace_peak"] / (KVH * 16 * (D * 4 + 8))
+    assert parts == S + ranges, parts
