@@ -487,7 +487,8 @@ int32_t rlx_sample(void *cache, const float *logits, int32_t n_rows, int32_t voc
  * int32 [n_rows].  Enqueued on the cache's stream: nothing is copied to or
  * from the host and the call does not wait -- except the first call that
  * needs a larger cache workspace (the split paths' chunk lists, top-k in
- * (0, 256] past 8192 entries, or no top-k past 12288: at most 64 MiB),
+ * (0, 256] past 8192 entries, or no top-k past 12288 -- past 18432 without
+ * top-p, and some sizes between: at most 64 MiB),
  * which synchronises the stream and allocates it once.  Without top-k a
  * call runs its rows unsplit where there is no such workspace (a
  * reservation without room for it, no memory) and always on a stream under

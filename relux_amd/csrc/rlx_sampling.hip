@@ -3,10 +3,10 @@
 // work-groups.
 //
 // Launch shapes:
-//   * Greedy, and Sample without top-k on a vocabulary of at most
-//     kMassMinVocab entries, with top-k above kPartMaxK, or with top-k on one
-//     of at most kPartChunk: one work-group per row (the whole-row path
-//     below).
+//   * Greedy, and Sample without top-k where mass_split_pays says no (up to
+//     12288 entries with top-p, about 18432 without), with top-k above
+//     kPartMaxK, or with top-k on at most kPartChunk entries: one work-group
+//     per row (the whole-row path below).
 //   * Sample without top-k on a larger vocabulary: the mass split (its own
 //     comment below).
 //   * Sample with top-k on a larger vocabulary (the split path):
@@ -2380,11 +2380,18 @@ void topk_split(int V, int top_k, int &nch, int &pch, int &pcap) {
 }
 
 // Mass split (top-k off): chunks of up to kPartChunk entries, as many rows
-// at a time as 64 MiB of scratch hold.  Taken past 12288 entries, where the
-// whole row in one work-group's LDS starts to cost more than three or four
-// launches (16 rows, us, whole row / split: top-p at V 8200 18 / 27, 16000
-// 33 / 27, 32000 43 / 27; temperature alone 10 / 16, 22 / 16, 25 / 16).
-constexpr int kMassMinVocab = 12288;
+// at a time as 64 MiB of scratch hold.  Taken where the whole row in one
+// work-group's LDS costs more than the split's launches: with top-p past 12288
+// entries (16 rows, us, whole row / split: V 8200 18 / 27, 16000 33 / 27, 32000
+// 43 / 27), without it past 18432 (temperature alone / with min-p: V 12289 12
+// and 14 / 18, 14000 13 and 15 / 17, 18000 16 and 18 / 17, 20000 19 and 22 / 17),
+// and from 12289 on where a thread's entries, read 8 at a time, end with 6 or 7
+// that are read one by one (16000: 22 and 24 / 17).
+constexpr int kMassMinVocab = 12288, kMassMinPlain = 18432;
+bool mass_split_pays(const SampleArgs &a) {
+    const bool topp = a.top_p > 0.f && a.top_p < 1.f;
+    return a.V > (topp || a.V / kST % 8 >= 6 ? kMassMinVocab : kMassMinPlain);
+}
 constexpr int64_t kMassScratch = 64 << 20;
 void mass_split(SampleArgs &a, int n_rows) {
     a.uch = a.upch = a.useg = a.urows = 0;
@@ -2393,7 +2400,7 @@ void mass_split(SampleArgs &a, int n_rows) {
     a.mass_l = nullptr;
     a.mass_r = nullptr;
     const bool topk = a.top_k > 0 && a.top_k < a.V;
-    if (topk || a.V <= kMassMinVocab || a.V > kSampMaxVocab) return;
+    if (topk || !mass_split_pays(a) || a.V > kSampMaxVocab) return;
     const int n = (a.V + kPartChunk - 1) / kPartChunk;
     a.upch = ((a.V + n - 1) / n + 3) & ~3;
     a.uch = (a.V + a.upch - 1) / a.upch;
