@@ -725,12 +725,20 @@ hipError_t launch_proj(hipStream_t s, int model, const PlanArg *plan, const Patc
                        void *q_out2, int q_bf16, uint16_t *kpool, uint16_t *vpool, int32_t *table,
                        int P, int cus, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 // The same over any number of rows in one launch (the MFMA GEMM of prefill
-// sizes); plans on the device only.  Taken past kProjRows rows, and past 32
-// when launch_proj's 16-feature work-groups are more than one round of the
-// CUs (us at K 4096, chunked kernel against GEMM: N 6144, 33 rows 23.8 / 22,
-// 64 rows 36.6 / 22; N 4096, 64 rows 21.0 / 20.8, 33 rows 14.3 / 21).
-inline bool proj_use_gemm(int rows, int model, const ProjDims &pd, int cus) {
-    return rows > kProjRows || (rows > 32 && proj_features(model, pd) > 16 * cus);
+// sizes); plans on the device only.  Taken from the rows on at which a whole
+// pass is shorter than launch_proj's, by the rounds of the CUs its 16-feature
+// work-groups take: the GEMM's time hardly depends on the rows, twice as long
+// for f32 activations, and a call that appends stages its plan (4 us).  us a
+// pass at d_model 4096, launch_proj / GEMM: N 6144 (2 rounds) bf16 33 rows 26.6 /
+// 28.1, 40 29.7 / 27.7, 64 40.8 / 28.1; f32 33 48 / 57, 48 55.5 / 57.4, 56 67 / 58.
+// N 10240 (3 rounds) 33 rows bf16 37 / 28, f32 69 / 58.  N 1536 (1 round) 65 rows
+// bf16 31.1 / 28.1, f32 48.7 / 57.9, 72 51.1 / 57.3, 96 62.4 / 57.4.  Without a
+// plan, K 1024, N 4096, f32: 65 rows 18.1 / 16.6.
+inline bool proj_use_gemm(int rows, int model, const ProjDims &pd, int K, bool x_bf16, int cus) {
+    const int rounds = (proj_features(model, pd) / 16 + cus - 1) / cus;
+    if (rounds > 2) return rows > 32;
+    if (rounds == 2) return rows > (x_bf16 ? 36 : 48);
+    return rows > (x_bf16 || (model == kProjModelOut && K <= 1024) ? kProjRows : kProjRows + 16);
 }
 hipError_t launch_proj_gemm(hipStream_t s, int model, const Patch *patches, int n_patch,
                             const AppendTok *toks, const int32_t *pos, int rows, const void *x,

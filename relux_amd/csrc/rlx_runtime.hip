@@ -1237,7 +1237,7 @@ int32_t rlx_out_project(void *h, int32_t rows, const void *x, int32_t x_dtype, i
     ProjDims pd{};
     pd.D = n_out;
     pd.DW = (n_out + 15) / 16 * 16;
-    if (proj_use_gemm(rows, kProjModelOut, pd, c->cus)) {  // prefill sizes: one GEMM over all rows
+    if (proj_use_gemm(rows, kProjModelOut, pd, k_in, x_dtype == RLX_BF16, c->cus)) {  // prefill sizes: one GEMM over all rows
         hipEvent_t e0, e1;
         if ((rc = timing_events(c, &e0, &e1, RLX_TIME_PROJECT))) return rc;
         HIP_TRY(launch_proj_gemm(c->stream, kProjModelOut, nullptr, 0, nullptr, nullptr, rows, x,
@@ -1332,7 +1332,7 @@ int32_t project_append(Cache *c, int model, int32_t layer, int32_t n_seqs, const
     if ((rc = plan_append(c, layer, n_seqs, seq_ids, n_tok, toks))) return rc;
     std::vector<Patch> patches = take_pending(c);
     const int xb = x_dtype == RLX_BF16 ? 2 : 4, qb = q_dtype == RLX_BF16 ? 2 : 4;
-    if (proj_use_gemm(total, model, pd, c->cus) && !capturing(c)) {
+    if (proj_use_gemm(total, model, pd, d_model, x_dtype == RLX_BF16, c->cus) && !capturing(c)) {
         // Prefill sizes: one GEMM over all rows, its plan staged.  A stream
         // under capture keeps the launches below, whose plans travel in the
         // kernel arguments; so does a call whose plan cannot be staged.

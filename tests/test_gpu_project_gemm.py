@@ -1,6 +1,7 @@
-"""The prefill-size projection GEMM (calls of more than 64 rows, or of 33 and
-more whose features are more than one round of the CUs) against the
-decode-size kernels: the same rows through calls of at most 32 rows.
+"""The prefill-size projection GEMM (calls of more than 64 rows, of more than
+80 with f32 activations, and from fewer whose features are more than one round
+of the CUs: proj_use_gemm) against the decode-size kernels: the same rows
+through calls of at most 32 rows.
 
 Both take the same bf16 products (f32 activations as hi + lo pairs) and
 differ in the order of the f32 sums: |difference| <= 2^-17 S per output, S =
@@ -47,8 +48,9 @@ GQA = [
     (160, 8, 8, 6, [2], [90], torch.bfloat16, torch.bfloat16),
     (64, 2, 2, 50, [11], [129], torch.float32, torch.bfloat16),
     (64, 6, 2, 24, [0, 0], [64, 64], torch.bfloat16, torch.bfloat16),
-    # more 16-feature tiles than CUs: the GEMM from 33 rows
+    # more 16-feature tiles than CUs: the GEMM from 37 rows
     (128, 259, 1, 16, [4], [33], torch.bfloat16, torch.bfloat16),
+    (128, 259, 1, 16, [4], [37], torch.bfloat16, torch.bfloat16),
 ]
 
 
@@ -118,7 +120,8 @@ def test_mla_gemm_equals_small_calls(gpu, d_model, H, D, dC, dR, lens, ntok, x_d
     (129, 96, 100, torch.float32, torch.float32, True, 0),
     (200, 64, 37, torch.bfloat16, torch.float32, False, 0),  # rows not a multiple of 4 elements
     (70, 32, 64, torch.bfloat16, torch.bfloat16, True, 1),   # out and residual 2 bytes off alignment
-    (33, 64, 4112, torch.float32, torch.bfloat16, False, 0),  # 257 tiles: the GEMM from 33 rows
+    (33, 64, 4112, torch.float32, torch.bfloat16, False, 0),
+    (49, 64, 4112, torch.float32, torch.bfloat16, False, 0),  # 257 tiles: the GEMM from 49 rows
 ])
 def test_out_gemm_equals_small_calls(gpu, rows, k_in, n_out, x_dtype, out_dtype, resid, off):
     from relux_amd import KVCache, pack_out
@@ -141,3 +144,56 @@ def test_out_gemm_equals_small_calls(gpu, rows, k_in, n_out, x_dtype, out_dtype,
         part = c.OutProject(x[r:r + n].contiguous(), wp, n_out,
                             residual=res[r:r + n].contiguous() if resid else None, out_dtype=out_dtype)
         _close(out[r:r + n], part, k_in, out_dtype == torch.bfloat16)
+
+
+@pytest.mark.parametrize("H,KVH,rows,x_dtype,gemm", [
+    (32, 8, 36, torch.bfloat16, False), (32, 8, 37, torch.bfloat16, True),  # two rounds of the CUs
+    (32, 8, 48, torch.float32, False), (32, 8, 49, torch.float32, True),
+    (64, 8, 32, torch.bfloat16, False), (64, 8, 33, torch.float32, True),   # three
+    (8, 2, 64, torch.bfloat16, False), (8, 2, 65, torch.bfloat16, True),    # one
+    (8, 2, 80, torch.float32, False), (8, 2, 81, torch.float32, True),
+])
+def test_rows_from_which_the_gemm_is_taken(gpu, H, KVH, rows, x_dtype, gemm):
+    """The GEMM only where it shortens the pass (sums in another order tell it
+    from the decode-size kernels, which a stream under capture takes)."""
+    from relux_amd import KVCache, pack_qkv, rope_tables
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the bounds are of 256 CUs")
+    D, dm = 128, 4096
+    g = torch.Generator().manual_seed(H + rows)
+    wp = pack_qkv(*_weights(g, gpu, (dm, H * D), (dm, KVH * D), (dm, KVH * D)), H, KVH, D)
+    rope = rope_tables(D, 10000.0, 128, gpu)
+    x = torch.randn(rows, dm, generator=g).to(gpu).to(x_dtype)
+
+    def step(c):
+        return c.ProjectAppend(0, x, wp, H, rope=rope, seq_ids=[0], n_tok=[rows], q_dtype=torch.float32)
+    caches = [KVCache(num_layers=1, max_len=128, num_kv_heads=KVH, head_dim=D, device=gpu.index) for _ in range(2)]
+    q = step(caches[0])
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    caches[1].use_stream(stream)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        small = step(caches[1])
+    graph.replay()
+    torch.cuda.synchronize()
+    _close(q, small, dm, False)
+    assert torch.equal(q, small) != gemm
+
+
+@pytest.mark.parametrize("rows,k_in,n_out,x_dtype,gemm", [
+    (72, 4096, 4096, torch.float32, False), (81, 4096, 4096, torch.float32, True),
+    (72, 640, 4096, torch.float32, True), (65, 4096, 4096, torch.bfloat16, True),
+])
+def test_out_rows_from_which_the_gemm_is_taken(gpu, rows, k_in, n_out, x_dtype, gemm):
+    from relux_amd import KVCache, pack_out
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the bounds are of 256 CUs")
+    g = torch.Generator().manual_seed(rows + n_out)
+    w, = _weights(g, gpu, (k_in, n_out))
+    wp = pack_out(w)
+    c = KVCache(num_layers=1, max_len=16, num_kv_heads=1, head_dim=64, device=gpu.index)
+    x = torch.randn(rows, k_in, generator=g).to(gpu).to(x_dtype)
+    y = c.OutProject(x, wp, n_out, out_dtype=torch.float32)
+    first = c.OutProject(x[:64].contiguous(), wp, n_out, out_dtype=torch.float32)
+    assert torch.equal(y[:64], first) != gemm
