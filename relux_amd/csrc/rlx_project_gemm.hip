@@ -384,11 +384,8 @@ hipError_t launch_proj_gemm(hipStream_t s, int model, const Patch *patches, int 
     static const Shape shapes[] = {{128, 32, {{43.5f, 70.f, 37.f}, {107.f, 162.f, 83.f}}},
                                    {64, 32, {{25.5f, 46.f, 23.8f}, {59.f, 98.f, 46.f}}},
                                    {64, 16, {{21.f, 29.5f, 15.1f}, {53.f, 72.f, 33.5f}}}};
-    static const int forced = [] {
-        const char *e = getenv("RLX_PROJ_GEMM");  // tuning override: tile shape 0 to 2
-        return e ? atoi(e) : -1;
-    }();
-    int best = forced;
+    const char *forced = getenv("RLX_PROJ_GEMM");  // override: tile shape 0 to 2 (tests; read per call)
+    int best = forced ? atoi(forced) : -1;
     if (best < 0 || best > 2) {
         float cost = 0.f;
         for (int i = 0; i < 3; i++) {

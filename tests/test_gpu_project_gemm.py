@@ -197,3 +197,83 @@ def test_out_rows_from_which_the_gemm_is_taken(gpu, rows, k_in, n_out, x_dtype, 
     y = c.OutProject(x, wp, n_out, out_dtype=torch.float32)
     first = c.OutProject(x[:64].contiguous(), wp, n_out, out_dtype=torch.float32)
     assert torch.equal(y[:64], first) != gemm
+
+
+# every tile shape the cost table may pick, at sizes past a turn of the unrolled
+# loop (12 k-steps of 64) and of the register rings, with a last half k-step
+# (800, 1568), chains of 4, 8 and 12 steps, and more than 16 row tiles whose
+# last group is partial (2100 rows: 33 tiles of 64, 17 of 128)
+@pytest.mark.parametrize("shape", [0, 1, 2])
+@pytest.mark.parametrize("rows,k_in,n_out,x_dtype,out_dtype", [
+    (200, 800, 300, torch.bfloat16, torch.float32),
+    (131, 1568, 256, torch.float32, torch.float32),
+    (2100, 4096, 520, torch.bfloat16, torch.bfloat16),
+    (2100, 2048, 256, torch.float32, torch.float32),
+])
+def test_out_gemm_shapes(gpu, monkeypatch, shape, rows, k_in, n_out, x_dtype, out_dtype):
+    """Against the 64-bit product: the f32 sums of exact products are within
+    K 2^-24 S, S = sum |x||w| of the output itself, f32 activations lose
+    2^-17 S to their bf16 pair, and a bf16 result one step."""
+    from relux_amd import KVCache, pack_out
+    monkeypatch.setenv("RLX_PROJ_GEMM", str(shape))
+    g = torch.Generator().manual_seed(rows + k_in)
+    w, = _weights(g, gpu, (k_in, n_out))
+    x = torch.randn(rows, k_in, generator=g).to(gpu).to(x_dtype)
+    res = torch.randn(rows, n_out, generator=g).to(gpu).to(out_dtype)
+    c = KVCache(num_layers=1, max_len=16, num_kv_heads=1, head_dim=64, device=gpu.index)
+    y = c.OutProject(x, pack_out(w), n_out, residual=res, out_dtype=out_dtype).double()
+    want = torch.matmul(x.double(), w.double()) + res.double()
+    S = torch.matmul(x.double().abs(), w.double().abs()) + res.double().abs()
+    tol = S * (k_in * 2.0 ** -24 + (2.0 ** -17 if x_dtype == torch.float32 else 0.0))
+    if out_dtype == torch.bfloat16:
+        tol = tol + want.abs() * 2.0 ** -8
+    assert bool(((y - want).abs() <= tol).all()), float(((y - want).abs() / tol).max())
+    # (the bound would hide little: the sums' own error is a hundredth of it)
+    if out_dtype == torch.float32:
+        assert float((y - want).norm() / want.norm()) <= 1e-5
+
+
+@pytest.mark.parametrize("shape", [0, 1, 2])
+@pytest.mark.parametrize("H,KVH,D,dm,lens,ntok,x_dtype", [
+    (8, 2, 128, 1568, [0, 7], [150, 61], torch.bfloat16),
+    (4, 4, 80, 800, [3], [2100], torch.float32),
+])
+def test_gqa_gemm_shapes(gpu, monkeypatch, shape, H, KVH, D, dm, lens, ntok, x_dtype):
+    """Q/K/V with RoPE and the append at every tile shape, against the 64-bit
+    projection and rotation: bounds as above, twice for the rotation's two
+    terms, and a bf16 step for the cached rows."""
+    from relux_amd import KVCache, pack_qkv, rope_tables
+    monkeypatch.setenv("RLX_PROJ_GEMM", str(shape))
+    g = torch.Generator().manual_seed(dm)
+    ws = _weights(g, gpu, (dm, H * D), (dm, KVH * D), (dm, KVH * D))
+    S, rope = len(lens), rope_tables(D, 10000.0, 2200, gpu)
+    x = torch.randn(sum(ntok), dm, generator=g).to(gpu).to(x_dtype)
+    c = KVCache(num_layers=1, max_len=2200, num_kv_heads=KVH, head_dim=D, max_seqs=S, device=gpu.index)
+    for i, n in enumerate(lens):
+        if n:
+            c.Append(0, torch.ones(n, KVH, D, device=gpu), torch.ones(n, KVH, D, device=gpu), seq_ids=[i], n_tok=[n],
+                     layout="SHD")
+    q = c.ProjectAppend(0, x, pack_qkv(*ws, H, KVH, D), H, rope=rope, seq_ids=list(range(S)), n_tok=ntok,
+                        q_dtype=torch.float32)
+    pos = torch.cat([torch.arange(a, a + b, device=gpu) for a, b in zip(lens, ntok)])
+    co, si = (t.double()[pos][:, None, :] for t in rope)
+    rel = dm * 2.0 ** -24 + 2.0 ** -20 + (2.0 ** -17 if x_dtype == torch.float32 else 0.0)
+
+    def want(w, heads, turn):
+        y = torch.matmul(x.double(), w.double()).view(-1, heads, D)
+        s = torch.matmul(x.double().abs(), w.double().abs()).view(-1, heads, D)
+        if turn:
+            a, b, sa, sb = y[..., 0::2], y[..., 1::2], s[..., 0::2], s[..., 1::2]
+            y = torch.stack([a * co - b * si, a * si + b * co], -1).flatten(-2)
+            s = torch.stack([sa + sb, sa + sb], -1).flatten(-2)
+        return y, s * rel
+    y, tol = want(ws[0], H, True)
+    assert bool(((q.double() - y).abs() <= tol).all())
+    at = 0
+    for i, n in enumerate(ntok):
+        for (w, turn), got in zip(((ws[1], True), (ws[2], False)), c.View(0, i)):
+            y, tol = want(w, KVH, turn)
+            y, tol = (t[at:at + n].transpose(0, 1) for t in (y, tol))
+            got = got[0].double()[:, lens[i]:]
+            assert bool(((got - y).abs() <= tol + y.abs() * 2.0 ** -8 + 1e-9).all())
+        at += n
