@@ -88,11 +88,12 @@ static_assert(kSeenOff + 2 * kSampMaxSeen <= kTileOff, "seen list must fit befor
 static_assert(kTileOff + kSampMaxVocab / 64 <= kRowCap, "tile counts must fit in the region");
 static_assert(kRowCap / 64 <= kST, "LDS-row tile counts use one slot per thread");
 
+constexpr int kFastexpBias = 1064948224;  // f32(127 * 2^23 - 405000); fastexp32(0) has these bits
 __device__ __forceinline__ float fastexp32_dev(float x) {
     if (x < -87.f) return 0.f;
     if (x > 87.f) return __uint_as_float(0x7F800000u);
     const float factor = 12102203.0f;  // f32(2^23 / ln 2)
-    const float bias = 1064948224.0f;  // f32(127 * 2^23 - 405000)
+    const float bias = (float)kFastexpBias;
     return __int_as_float((int)__fadd_rn(__fmul_rn(factor, x), bias));
 }
 
@@ -623,7 +624,9 @@ __device__ __forceinline__ void topk_select(Src &c, int top_k, SampLds &s) {
 // the 4096 weights of the bucket it falls in, where a bisection over the
 // float keys takes 31 passes over the set (one work-group, 16 rows, T 0.8,
 // top-p 0.95: V 1000 18.7 -> 10.9 us, 4000 37.9 -> 16.7, 8192 33.4 -> 18.8).
-constexpr int kMassTop = 0x3F79D1C0 >> 18;  // bucket of the largest weight: fastexp32(0)
+constexpr int kMassTop = kFastexpBias >> 18;  // bucket of the largest weight: fastexp32(0)
+static_assert(kFastexpBias % 64 == 0 && (kMassTop - (kMassBuckets - 2)) << 18 >= 1 << 29 && kFastexpBias < 1 << 30,
+              "the bits of every weight in a bucket are an f32 of 64-unit spacing");
 __device__ __forceinline__ int mass_bucket(uint32_t bits) { return kMassTop - (int)(bits >> 18); }
 __device__ __forceinline__ uint32_t mass_sig(uint32_t bits) { return ((bits & 0x7FFFFFu) | 0x800000u) >> 6; }
 // Weight of one unit of mass_sig in a bucket: 2^(exponent - 150 + 6).
