@@ -24,8 +24,10 @@ namespace rlx {
 // dims d >= D of every head and channels c >= dc (the expansion then writes
 // exact zeros for the padded dims, and the zero-padded channels of the latent
 // rows meet zero weights).  Thread = 8 channels x 8 features (D a multiple of
-// 8), turned in registers: 16-byte loads and stores.  Bound: memory; 16384
-// features 12 us (17 by 2-byte accesses through LDS).
+// 8), turned in registers: 16-byte loads (by elements where w is not aligned
+// for them: the caller's weights may start at any element) and stores.  Bound:
+// memory; 16384 features 12 us (17 by 2-byte accesses through LDS).
+template <bool VEC>
 __global__ __launch_bounds__(256) void mla_wt_kernel(const uint16_t *__restrict__ w,
                                                      uint16_t *__restrict__ wt, int dc, int H, int D,
                                                      int DP) {
@@ -34,8 +36,17 @@ __global__ __launch_bounds__(256) void mla_wt_kernel(const uint16_t *__restrict_
     const int h = f / DP, d = f - h * DP;
     u32x4 r[8];
 #pragma unroll
-    for (int k = 0; k < 8; k++)
-        r[k] = (c + k < dc && d < D) ? *(const u32x4 *)(w + (int64_t)(c + k) * H * D + h * D + d) : u32x4{0, 0, 0, 0};
+    for (int k = 0; k < 8; k++) {
+        r[k] = u32x4{0, 0, 0, 0};
+        if (c + k >= dc || d >= D) continue;
+        const uint16_t *p = w + (int64_t)(c + k) * H * D + h * D + d;
+        if constexpr (VEC) {
+            r[k] = *(const u32x4 *)p;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) r[k][j] = (uint32_t)p[2 * j] | ((uint32_t)p[2 * j + 1] << 16);
+        }
+    }
     uint16_t *o = wt + (((int64_t)(f >> 4) * (kMlaDc / 32) + (c >> 5)) * 16 + (f & 15)) * 32 + (c & 31);
 #pragma unroll
     for (int e = 0; e < 8; e++) {
@@ -234,8 +245,14 @@ hipError_t launch_mla_wt(hipStream_t s, const uint16_t *w_uk, const uint16_t *w_
                          int dc, int DP, uint16_t *wt_k, uint16_t *wt_v) {
     if (D > DP || D % 8 != 0 || DP % 64 != 0 || dc > kMlaDc) return hipErrorInvalidValue;
     const dim3 g((H * DP / 8 + 255) / 256, kMlaDc / 8);
-    mla_wt_kernel<<<g, 256, 0, s>>>(w_uk, wt_k, dc, H, D, DP);
-    mla_wt_kernel<<<g, 256, 0, s>>>(w_uv, wt_v, dc, H, D, DP);
+    auto pack = [&](const uint16_t *w, uint16_t *wt) {
+        if (((uintptr_t)w & 15) == 0)
+            mla_wt_kernel<true><<<g, 256, 0, s>>>(w, wt, dc, H, D, DP);
+        else
+            mla_wt_kernel<false><<<g, 256, 0, s>>>(w, wt, dc, H, D, DP);
+    };
+    pack(w_uk, wt_k);
+    pack(w_uv, wt_v);
     return hipGetLastError();
 }
 

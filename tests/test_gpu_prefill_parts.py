@@ -187,3 +187,22 @@ def test_hd96_outputs_in_the_queries_memory(gpu):
     same = q.clone()  # row for row: as with separate outputs
     assert torch.equal(c.Attend(0, same, H, out=same, **kw), c.Attend(0, q, H, **kw))
     assert not torch.equal(same, tiles), "the call took query tiles"
+
+
+def test_mla_prefill_weights_off_alignment(gpu):
+    """W_UK and W_UV that start at any element: the expansion packs them by
+    elements, with the same result."""
+    from relux_amd import MLACache
+    H, D, T, n = 3, 64, 500, 400
+    g = torch.Generator(device=gpu).manual_seed(2)
+    w = [(torch.randn(512, H * D, device=gpu, generator=g) * 0.02).to(torch.bfloat16) for _ in range(2)]
+    odd = []
+    for off, x in zip((1, 3), w):
+        buf = torch.empty(x.numel() + 8, dtype=torch.bfloat16, device=gpu)
+        odd.append(buf[off:off + x.numel()].view(x.shape).copy_(x))
+    c = MLACache(num_layers=1, max_len=T, page_tokens=64, device=gpu.index)
+    c.Append(0, torch.randn(T, 512, device=gpu, generator=g), torch.randn(T, 64, device=gpu, generator=g),
+             seq_ids=[0], n_tok=[T])
+    qn, qr = (torch.randn(n, H, d, device=gpu, generator=g) for d in (D, 64))
+    want = c.Attend(0, qn, qr, *w, H, D, seq_ids=[0], n_q=[n])
+    assert torch.equal(c.Attend(0, qn, qr, *odd, H, D, seq_ids=[0], n_q=[n]), want)
