@@ -2150,8 +2150,8 @@ static int32_t mla_attend_check(Cache *c, int32_t n_seqs, const int32_t *n_q, in
     if (mask_mode < RLX_MASK_CAUSAL || mask_mode > RLX_MASK_NONE) return fail(RLX_ERR_INVALID, "mask_mode");
     if (n_seqs == 0) return RLX_OK;
     if (!q_nope || !q_rope || !w_uk || !w_uv || !out) return fail(RLX_ERR_INVALID, "null operand");
-    // (Calls of more than 32 query rows per sequence take the FA2 path, which
-    // covers every head_dim accepted above.)
+    // (Both forms, the absorbed kernel and FA2, cover every head_dim accepted
+    // above.)
     return RLX_OK;
 }
 
