@@ -666,19 +666,21 @@ int gqa_wg_per_cu() {
 // with no row divided the decode kernel writes the outputs itself and the merge
 // launch falls away.  A row has a range of its own, or, with more rows than
 // ranges, consecutive rows share one by their tokens and kGqaRowStart units a
-// row for its start.  The line: a work-group's tokens past an even share cost
-// less than the merge launch saves (kernel us per 64 tokens: 0.22, 0.30, 0.34,
-// 0.42 and 1.1 at stored head dims 32, 64, 96, 128 and 256, with two query tiles
-// twice that; the merge 3.2 to 5.6), and rows of up to 8 units, which even cuts
-// would leave whole too (kGqaSnap64), always.  Measured, GPU time back to back, even
-// cuts / whole: 32/8 heads of 128, 1 x 500 tokens 10.7 / 9.3, 1 x 750 9.8 / 11.0
-// (cut), 31 x 750 21.6 / 18.4; heads of 64, 1 x 750 8.4 / 8.4, 4 x 1500 9.6 / 12.7
-// (cut), 31 x 1000 17.1 / 12.8.  The ranges have to fit the kernel arguments (the
-// kernel's own search knows even cuts only).  Returns their number, or 0.
+// row for its start.  The lines: 1536 tokens of head dim 64 in one query tile and
+// as many bytes elsewhere; with two tiles (a work-group's 64 tokens take twice as
+// long) 1024, and no more past an even share than the merge launch and its kernel
+// cost.  Rows of up to 8 units stay whole under even cuts too (kGqaSnap64).
+// Measured, us a pass of append and attention, cut / whole: 32/8 heads of 128, 1
+// x 600 tokens 15.6 / 12.7, 1 x 750 15.3 / 13.2 (GPU time alone 9.8 / 11.0); heads
+// of 64, 1 x 1000 15.0 / 12.3 (GPU time 8.5 / 9.6), 1 x 1500 16.2 / 14.4 and 8 x 1500
+// 17.0 / 14.9 (GPU time of 4 x 1500 9.6 / 12.7); 64/8 of 64 with 24 query rows, 1 x
+// 600 15.0 / 15.0, 1 x 900 15.5 / 18.3 (cut), 8 x 680 17.6 / 16.4, 16 x 750 20.8 / 17.6.
+// The ranges have to fit the kernel arguments (the kernel's own search knows even
+// cuts only).  Returns their number, or 0.
 constexpr int kGqaRowStart = 3;
 int gqa_whole_rows(const Cache *c, int nqt, const int *pre, int n_rows, int full, int *cuts) {
     const int line = (nqt == 1 ? 1536 : 1024) / std::max(c->hd, 64);  // 64-token units
-    const int slack = (c->hd <= 32 ? 13 : c->hd == 64 ? 10 : c->hd == 96 ? 9 : c->hd == 128 ? 8 : 5) / nqt;
+    const int slack = nqt == 1 ? line : c->hd <= 32 ? 12 : c->hd == 64 ? 9 : 8;
     const int share = (pre[n_rows] + full - 1) / full;
     if ((size_t)n_rows * sizeof(AttRow) + (size_t)full * sizeof(int4) > kPlanArgBytes) return 0;
     auto too_long = [&](int units) { return units > line || (units > 2 * kGqaSnap64 && units - share > slack); };

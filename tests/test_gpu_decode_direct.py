@@ -69,7 +69,8 @@ def test_direct_outputs(gpu, H, KVH, D, lens, nq, dtype, layout):
 @pytest.mark.parametrize("lens,ranges", [
     ([200, 40, 130, 90, 65, 10, 190, 25] * 3, 24),  # a range each: 32 are there
     ([500], 1),
-    ([750], 12),                                    # cut: 11 units past an even share
+    ([750], 1),
+    ([800], 13),                                    # cut: longer than 12 units
     ([750] * 31, 31),                               # an even share is a row
     ([60] * 40, 20),                                # more rows than ranges: even in rows
 ])
