@@ -732,13 +732,17 @@ hipError_t launch_proj(hipStream_t s, int model, const PlanArg *plan, const Patc
 // pass at d_model 4096, launch_proj / GEMM: N 6144 (2 rounds) bf16 33 rows 26.6 /
 // 28.1, 40 29.7 / 27.7, 64 40.8 / 28.1; f32 33 48 / 57, 48 55.5 / 57.4, 56 67 / 58.
 // N 10240 (3 rounds) 33 rows bf16 37 / 28, f32 69 / 58.  N 1536 (1 round) 65 rows
-// bf16 31.1 / 28.1, f32 48.7 / 57.9, 72 51.1 / 57.3, 96 62.4 / 57.4.  Without a
-// plan, K 1024, N 4096, f32: 65 rows 18.1 / 16.6.
+// bf16 31.1 / 28.1, f32 48.7 / 57.9, 72 51.1 / 57.3, 96 62.4 / 57.4.  d_model
+// 1024, N 3072, where the plan is the larger part: bf16 65 rows 18.3 / 19.8, 96
+// 19.4 / 20.2, 128 25.9 / 20.6.  Without a plan, K 1024, N 4096: 65 rows bf16
+// 13.4 / 9.0, f32 18.1 / 16.6.
 inline bool proj_use_gemm(int rows, int model, const ProjDims &pd, int K, bool x_bf16, int cus) {
     const int rounds = (proj_features(model, pd) / 16 + cus - 1) / cus;
     if (rounds > 2) return rows > 32;
     if (rounds == 2) return rows > (x_bf16 ? 36 : 48);
-    return rows > (x_bf16 || (model == kProjModelOut && K <= 1024) ? kProjRows : kProjRows + 16);
+    const bool small = K <= 1024, out = model == kProjModelOut;
+    if (x_bf16) return rows > (small && !out ? kProjRows + 32 : kProjRows);
+    return rows > (small && out ? kProjRows : kProjRows + 16);
 }
 hipError_t launch_proj_gemm(hipStream_t s, int model, const Patch *patches, int n_patch,
                             const AppendTok *toks, const int32_t *pos, int rows, const void *x,

@@ -51,6 +51,10 @@ GQA = [
     # more 16-feature tiles than CUs: the GEMM from 37 rows
     (128, 259, 1, 16, [4], [33], torch.bfloat16, torch.bfloat16),
     (128, 259, 1, 16, [4], [37], torch.bfloat16, torch.bfloat16),
+    # one round of tiles of a d_model of at most 1024 in bf16: the GEMM from 97 rows
+    (512, 8, 2, 64, [0, 40], [97, 0], torch.bfloat16, torch.bfloat16),
+    (96, 3, 1, 20, [0], [98], torch.bfloat16, torch.bfloat16),
+    (160, 8, 8, 6, [2], [122], torch.bfloat16, torch.bfloat16),
 ]
 
 
@@ -89,6 +93,8 @@ def test_gqa_gemm_equals_small_calls(gpu, d_model, H, KVH, D, lens, ntok, x_dtyp
     (96, 2, 32, 130, 10, [7], [129], torch.float32),   # latent and rope widths not multiples of 4
     (64, 2, 4, 16, 2, [0], [70], torch.bfloat16),      # heads narrower than a fragment
     (64, 5, 6, 16, 8, [0], [70], torch.bfloat16),      # q_c heads packed padded, 6 dims stored
+    (64, 2, 4, 16, 2, [0], [102], torch.bfloat16),     # the same in the GEMM
+    (64, 5, 6, 16, 8, [0], [102], torch.bfloat16),
 ])
 def test_mla_gemm_equals_small_calls(gpu, d_model, H, D, dC, dR, lens, ntok, x_dtype):
     from relux_amd import MLACache, pack_mla_proj, rope_tables
@@ -277,3 +283,21 @@ def test_gqa_gemm_shapes(gpu, monkeypatch, shape, H, KVH, D, dm, lens, ntok, x_d
             got = got[0].double()[:, lens[i]:]
             assert bool(((got - y).abs() <= tol + y.abs() * 2.0 ** -8 + 1e-9).all())
         at += n
+
+
+@pytest.mark.parametrize("rows,dm,x_dtype,gemm", [
+    (96, 640, torch.bfloat16, False), (97, 640, torch.bfloat16, True),
+    (80, 640, torch.float32, False), (81, 640, torch.float32, True),
+])
+def test_rows_from_which_a_narrow_model_takes_the_gemm(gpu, rows, dm, x_dtype, gemm):
+    from relux_amd import KVCache, pack_qkv
+    if torch.cuda.get_device_properties(gpu).multi_processor_count != 256:
+        pytest.skip("the bounds are of 256 CUs")
+    H, KVH, D = 8, 2, 64
+    g = torch.Generator().manual_seed(rows)
+    wp = pack_qkv(*_weights(g, gpu, (dm, H * D), (dm, KVH * D), (dm, KVH * D)), H, KVH, D)
+    x = torch.randn(rows, dm, generator=g).to(gpu).to(x_dtype)
+    c = KVCache(num_layers=1, max_len=128, num_kv_heads=KVH, head_dim=D, max_seqs=2, device=gpu.index)
+    q = c.ProjectAppend(0, x, wp, H, seq_ids=[0], n_tok=[rows], q_dtype=torch.float32)
+    first = c.ProjectAppend(0, x[:64].contiguous(), wp, H, seq_ids=[1], n_tok=[64], q_dtype=torch.float32)
+    assert torch.equal(q[:64], first) != gemm
